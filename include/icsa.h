@@ -96,6 +96,8 @@ enum icsa_ws_slot {
                       /* before them, the compressed stage's split value means,      */
                       /* bf16 [B*H, 2, D, ceil(NB/64)*64]; sized for the larger)     */
   ICSA_WS_RSTAT,      /* f32 [B*H, NB, 2]   row max and 1 / row sum of the compressed softmax */
+  ICSA_WS_FLASHP,     /* f32 partials of the peaked blocks whose keys are split (O, max, sum; */
+                      /* a workspace that ends before this slot is accepted: nothing is split) */
   ICSA_WS_COUNT
 };
 
@@ -263,7 +265,9 @@ int icsa_sparse_piecewise_attn_bwd(
     void* dv, int dv_dtype, int64_t dv_sb, int64_t dv_sh, int64_t dv_st,
     void* workspace, int64_t workspace_bytes, void* stream);
 
-/* Workspace bytes of icsa_flash_attn. */
+/* Workspace bytes of icsa_flash_attn for any Sq: V^T, then room for the partials of query
+ * blocks whose keys are split over several workgroups.  A workspace that holds the V^T alone
+ * (B * H * D * 64 ceil(Sk / 64) bf16, rounded up to 256 bytes) is accepted as well. */
 int64_t icsa_flash_attn_workspace_size(int B, int Sk, int H, int D);
 
 /* Dense non-causal attention softmax(q k^T / sqrt(D)) v: q [B, Sq, H, D], k/v [B, Sk, H, D]

@@ -113,6 +113,7 @@ Layout editing_layout(int B, int S, int H, const Sizes& z, int t, int q_dtype, i
   // the level-3 scores, and before them the compressed stage's split value means
   sz[ICSA_WS_L3S] = std::max(BH * std::max(z.n_diffuse, 1) * z.NKV * 4, compressed_vmt_bytes((int)BH, z.NB));
   sz[ICSA_WS_RSTAT] = BH * z.NB * 2 * 4;
+  sz[ICSA_WS_FLASHP] = flash_plan(flash_items((int)BH, z.n_peaked), ceil_div(t, ICSA_BLOCK) + z.topK, true).part_bytes;
   Layout L;
   int64_t o = 0;
   for (int i = 0; i < ICSA_WS_COUNT; ++i) {
@@ -238,7 +239,8 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
   if (z.NKV > 2048 || z.top_k > 512)
     return fail(ICSA_EUNSUPPORTED, "NKV=%d / top_k=%d exceed limits (2048 / 512)", z.NKV, z.top_k);
   const Layout L = editing_layout(B, S, H, z, t_seq_len, q_dtype, k_dtype, v_dtype);
-  if (workspace_bytes < L.total)
+  // the last slot may be missing: the peaked blocks then run without being split
+  if (workspace_bytes < L.off[ICSA_WS_FLASHP])
     return fail(ICSA_EWORKSPACE, "workspace %lld bytes < required %lld", (long long)workspace_bytes,
                 (long long)L.total);
   char* ws = reinterpret_cast<char*>(workspace);
@@ -408,6 +410,8 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
     f.sel = sel; f.sel_stride = std::max(z.topK, 1); f.n_sel = z.topK; f.sel_base = z.n_t;
     f.out_c = cp.out_c; f.nb_q = z.NB;
     f.alpha = av; f.out = ov; f.scale_log2 = scale_log2;
+    f.part = reinterpret_cast<float*>(WS(ICSA_WS_FLASHP));
+    f.part_bytes = workspace_bytes - L.off[ICSA_WS_FLASHP];
     ICSA_HIP_TRY(launch_flash(f, stream), "flash attention");
   }
   ICSA_HIP_TRY(mark(ICSA_STAGE_FLASH), "event");
@@ -498,7 +502,7 @@ int icsa_editing_sparse_attention_noalloc(
     return rc;
   if (t_seq_len < 0 || t_seq_len > S) return fail(ICSA_EINVAL, "t_seq_len %d outside [0, S=%d]", t_seq_len, S);
   const Sizes z = derive(S, t_seq_len, sparsity, srr, flat_ratio);
-  const int64_t need = editing_layout(B, S, H, z, t_seq_len, q_dtype, k_dtype, v_dtype).total;
+  const int64_t need = editing_layout(B, S, H, z, t_seq_len, q_dtype, k_dtype, v_dtype).off[ICSA_WS_FLASHP];
   if (need > (int64_t)ICSA_NOALLOC_SCRATCH_BYTES)
     return fail(ICSA_EUNSUPPORTED,
                 "this call needs %lld bytes of scratch, more than the %lld-byte static scratch of "
@@ -920,9 +924,13 @@ int icsa_sparse_piecewise_attn_bwd(
   return ICSA_OK;
 }
 
+static int64_t flash_vt_bytes(int B, int Sk, int H) {
+  return align256((int64_t)B * H * ICSA_D * ceil_div(Sk, ICSA_BLOCK) * ICSA_BLOCK * 2);
+}
+
 int64_t icsa_flash_attn_workspace_size(int B, int Sk, int H, int D) {
   if (B <= 0 || Sk <= 0 || H <= 0 || D != ICSA_D) return -1;
-  return align256((int64_t)B * H * ICSA_D * ceil_div(Sk, ICSA_BLOCK) * ICSA_BLOCK * 2);
+  return flash_vt_bytes(B, Sk, H) + flash_part_bytes_max(ceil_div(Sk, ICSA_BLOCK));
 }
 
 int icsa_flash_attn(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
@@ -939,7 +947,7 @@ int icsa_flash_attn(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
   if (!row_ok(q, ICSA_BF16, q_sb, q_ss, q_sh) || !row_ok(k, ICSA_BF16, k_sb, k_ss, k_sh) ||
       !row_ok(v, ICSA_BF16, v_sb, v_ss, v_sh) || !row_ok(out, out_dtype, o_sb, o_ss, o_sh))
     return fail(ICSA_EINVAL, "q/k/v/out rows must be 16-byte aligned (pointer and strides)");
-  const int64_t need = icsa_flash_attn_workspace_size(B, Sk, H, D);
+  const int64_t need = flash_vt_bytes(B, Sk, H);    // what is left over splits the last items
   if (workspace_bytes < need)
     return fail(ICSA_EWORKSPACE, "workspace %lld bytes < required %lld", (long long)workspace_bytes,
                 (long long)need);
@@ -966,6 +974,8 @@ int icsa_flash_attn(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
   f.alpha = make_alpha(nullptr, ICSA_F32, 0, 0, 0, 0, 0.f);
   f.out = OutView{out, o_sb, o_ss, o_sh, out_dtype};
   f.scale_log2 = kLog2e / std::sqrt((float)ICSA_D);
+  f.part = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + need);
+  f.part_bytes = workspace_bytes - need;
   ICSA_HIP_TRY(launch_flash(f, stream), "flash attention");
   return ICSA_OK;
 }

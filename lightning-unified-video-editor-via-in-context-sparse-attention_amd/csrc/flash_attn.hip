@@ -10,7 +10,21 @@
 // logit 0, exactly like the reference's zero padding of k_padded).  K is read in place;
 // V^T holds tile j at columns 64 j .. 64 j + 63 (the pipeline writes it in that order).
 //
-// Workgroup = 8 waves = four 64-row query blocks (wave w: block w/2, rows 32*(w%2)..+31),
+// Work is dealt in items: four 64-row query blocks of one head against all key tiles.  A
+// workgroup runs a sequence of segments (runs of tiles of one item): several whole items, or
+// one of the equal ranges ("chunks") that the tiles of the last, incomplete round's items
+// are cut into, whose partial O, max and sum icsa_flash_combine_kernel adds up.  The tile
+// stream runs across segment boundaries, so the next item's tiles arrive while an item
+// ends.  Measured against one workgroup per item, with an epilogue of its own: 32 items of
+// 72 tiles (2 heads, 8,192 tokens) 101 -> 27 us plus 9 us for the sums; 640 items of 576
+// tiles (5 heads, 65,536 tokens; 2.5 rounds) 2,825 -> 2,511 + 10 us; 10,240 items of 8
+// tiles (512 keys, 40 heads, 65,520 queries) 853 -> 775 us; 5,120 items of 576 tiles (40
+// heads) unchanged at 20.0 ms.  The rate is then about 1.23 PFLOP/s at every size that
+// fills the chip, the engine clock under this load being 1.7-1.9 GHz; with 8 tiles an item,
+// timing copies without the output stores and without the Q loads take 693 and 755 us (both:
+// 641 us), so what is left there is mostly the first tiles' second pass and the stores.
+//
+// Workgroup = 8 waves = an item's query blocks (wave w: block w/2, rows 32*(w%2)..+31),
 // all sharing each K / V^T tile.  The waves form two groups, G0 = waves 0-3 and G1 = waves
 // 4-7, so every SIMD holds one wave of each.  The groups run the same sequence of phases
 //     GEMM(k) = { S(k) = K(k) Q^T ;  O += V(k-1)^T P(k-1) }      (32 MFMAs)
@@ -32,136 +46,185 @@
 // as against the initial m_ref = -inf) is the row max of the tile taken, the reference
 // raised, O / l rescaled and the tile recomputed.  In the common case no per-tile max
 // reduction precedes the exponentials.  Exact in real arithmetic.
+#include <algorithm>
+
+
 #include "attn_tile.h"
 #include "icsa_kernels.h"
 
 #define FA_WAVES 8
 #define FA_THREADS (FA_WAVES * 64)
 #define FA_QBLK_PER_WG (FA_WAVES / 2)
-#define FA_STAGE_BYTES (FA_WAVES * 32 * O_LDS_STRIDE * 4)    // epilogue staging, all waves
 #define FA_NBUF 4                                            // K and V^T tile buffers
 #define FA_TILE_BYTES (FA_NBUF * (K_TILE_BYTES + V_TILE_BYTES))
-#define FA_MAX_SEL 4096                                      // extra tiles (LDS list)
-#define FA_JUNK_OFF (FA_TILE_BYTES + 4 * FA_MAX_SEL)         // landing area of disabled DMA
-#define FA_LOOP_BYTES (FA_JUNK_OFF + 4096)
-#define FA_LDS_BYTES (FA_LOOP_BYTES > FA_STAGE_BYTES ? FA_LOOP_BYTES : FA_STAGE_BYTES)
+#define FA_JUNK_OFF FA_TILE_BYTES                            // landing area of disabled DMA
+#define FA_STAGE_OFF (FA_JUNK_OFF + 4096)                    // 2 KB of output staging per wave
+#define FA_STAGE_WAVE 2048
+#define FA_LDS_BYTES (FA_STAGE_OFF + FA_WAVES * FA_STAGE_WAVE)
 // A lane's 32 probabilities of a tile sum to at most 2^64 relative to the row's reference
 // max before the reference is raised: O and l then stay below 2^64 * keys * |v|, far inside
 // the fp32 range, and bf16(p) keeps its relative precision at any magnitude.
 #define FA_PSUM_MAX 18446744073709551616.0f
+// The reference max before the first tile: finite, so that a tile whose scores are all -inf
+// leaves O = l = 0 instead of inf - inf.
+#define FA_M_NONE (-3.4028234663852886e38f)
 #ifndef FA_PF
 #define FA_PF 5             // operand prefetch depth (MFMA steps); 3, 4, 6 and 8 measured slower
 #endif
+#define FA_PART_WAVE (64 * 64 + 2 * 64)                      // floats of one wave's partial: O, m, l
+#define FA_PART_FLOATS (FA_WAVES * FA_PART_WAVE)
 
+namespace {
+
+typedef const __attribute__((address_space(4))) int* const_int_ptr;
+// A wave-uniform int of global memory through the scalar cache: a vector load would have to
+// be waited for behind the tile DMA in flight.  Only for data written by earlier kernels.
+__device__ __forceinline__ int uniform_load(const int* p) {
+  return *(const_int_ptr)(unsigned long long)p;
+}
+
+// The parameter block re-read from the kernel-argument segment: what only a segment boundary
+// needs does not stay in scalar registers (which spill into vector lanes) through the tiles.
+__device__ __forceinline__ const FlashParams& cold_params() {
+  auto kp = (const __attribute__((address_space(4))) FlashParams*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(kp));
+  return *(const FlashParams*)kp;
+}
+
+// Iterations [lo, hi) of chunk c: the split items' tiles as one sequence, cut in n_chunk ranges
+__host__ __device__ __forceinline__ int64_t chunk_start(int c, int n_split, int n_tiles, int n_chunk) {
+  return (int64_t)c * ((int64_t)n_split * n_tiles) / n_chunk;
+}
+
+// d-subtile ds of one wave's 32 output rows straight from the accumulators (lane (li, hl)
+// holds dims 32 ds + 8 g + 4 hl + x of query li; g, x = 0..3): 1 / l, residual, output type.
+// The rows pass through 2 KB of the wave's own LDS, 64 bytes of each at a time, so that a
+// store instruction writes 16 segments of 64 bytes; stores straight from the accumulators
+// are 64 segments of 16 bytes, four times the requests.  16-byte chunk c of row r sits at
+// chunk c ^ (r / 4 % 4): writes (one chunk of 16 rows) and reads (4 chunks of 4 rows) both
+// touch every bank once.
+template <bool kBf16, bool kAlphaD>
+__device__ __forceinline__ void store_subtile(unsigned char* stage, const floatx16& o, int ds, float inv_l,
+                                              const OutView& out, int b, int h, int tok0, int n_rows,
+                                              const float* oc_row, const AlphaView& alpha) {
+  const int lane = threadIdx.x & 63, li = lane & 31, hl = lane >> 5;
+  float v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = o[i] * inv_l;
+  if (oc_row != nullptr && li < n_rows) {
+    const float a0 = kAlphaD ? 0.f : alpha_at(alpha, b, tok0 + li, h, 0);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d = 32 * ds + 8 * g + 4 * hl;
+      const floatx4 c = *reinterpret_cast<const floatx4*>(oc_row + d);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[4 * g + e] = fmaf(kAlphaD ? alpha_at(alpha, b, tok0 + li, h, d + e) : a0, c[e], v[4 * g + e]);
+    }
+  }
+  unsigned char* wr = stage + li * 64;
+  const int wx = (li >> 2) & 3;
+  const int64_t off = (int64_t)b * out.sb + (int64_t)tok0 * out.ss + (int64_t)h * out.sh + 32 * ds;
+  auto store_rows64 = [&](unsigned char* dst, int64_t row_bytes) {    // 32 staged rows of 64 bytes
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = 16 * i + (lane >> 2);
+      const u32x4 x = *reinterpret_cast<const u32x4*>(stage + r * 64 + (((lane & 3) ^ ((r >> 2) & 3)) << 4));
+      if (r < n_rows) *reinterpret_cast<u32x4*>(dst + r * row_bytes + 16 * (lane & 3)) = x;
+    }
+  };
+  if constexpr (kBf16) {
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr) {               // lane halves swap: dims 8 (2 pr + hl) .. + 7
+      bf16x4 lo, hi;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { lo[e] = (bf16)v[8 * pr + e]; hi[e] = (bf16)v[8 * pr + 4 + e]; }
+      const u32x2 x = __builtin_bit_cast(u32x2, lo), y = __builtin_bit_cast(u32x2, hi);
+      const auto w0 = __builtin_amdgcn_permlane32_swap(x[0], y[0], false, false);
+      const auto w1 = __builtin_amdgcn_permlane32_swap(x[1], y[1], false, false);
+      *reinterpret_cast<u32x4*>(wr + (((2 * pr + hl) ^ wx) << 4)) = u32x4{w0[0], w1[0], w0[1], w1[1]};
+    }
+    store_rows64(reinterpret_cast<unsigned char*>(reinterpret_cast<bf16*>(out.p) + off), out.ss * 2);
+  } else {
+#pragma unroll
+    for (int pr = 0; pr < 2; ++pr) {               // dims 16 pr .. + 15
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+        *reinterpret_cast<floatx4*>(wr + (((2 * g + hl) ^ wx) << 4)) =
+            floatx4{v[8 * pr + 4 * g], v[8 * pr + 4 * g + 1], v[8 * pr + 4 * g + 2], v[8 * pr + 4 * g + 3]};
+      store_rows64(reinterpret_cast<unsigned char*>(reinterpret_cast<float*>(out.p) + off + 16 * pr), out.ss * 4);
+    }
+  }
+}
+
+}  // namespace
+
+template <bool kBf16, bool kAlphaD>
 __global__ void __launch_bounds__(FA_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 icsa_flash_kernel(FlashParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int ngrp = (p.n_qblk + FA_QBLK_PER_WG - 1) / FA_QBLK_PER_WG;
-  const int work = xcd_remap(blockIdx.x, p.B * p.H * ngrp);
-  if (work < 0) return;
-  const int bh = work / ngrp, grp = work % ngrp;
-  const int b = bh / p.H, h = bh % p.H;
+  const int n_tiles = p.n_tgt_tiles + p.n_sel;
   const int tid = threadIdx.x;
   // wave index made provably wave-uniform (a scalar), so per-group branches stay uniform
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int li = lane & 31, hl = lane >> 5;
   const int group = wave >> 2;                        // 0: leads, 1: one slot behind
-  const int slot = grp * FA_QBLK_PER_WG + (wave >> 1);
-  const bool active = slot < p.n_qblk;
-  int qblk = 0;
-  if (active) qblk = p.qblocks ? p.qblocks[(int64_t)bh * p.qb_stride + p.qb_offset + slot] : slot;
-  const int qtok0 = qblk * ICSA_BLOCK + 32 * (wave & 1);
-  const int q_valid = active ? max(0, min(32, p.Sq - qtok0)) : 0;
+  const bool lag = group == 1;
 
-  // token start of every extra (selected source) tile, kept in LDS past the tile buffers
-  int* sel_l = reinterpret_cast<int*>(smem + FA_TILE_BYTES);
-  for (int r = tid; r < p.n_sel; r += FA_THREADS)
-    sel_l[r] = (p.sel_base + p.sel[(int64_t)bh * p.sel_stride + r]) * ATT_BN;
-
-  bf16x8 qf[8];
-  load_q_frags(qf, p.q + (int64_t)b * p.q_sb + (int64_t)qtok0 * p.q_ss + (int64_t)h * p.q_sh, p.q_ss,
-               q_valid);
-  __syncthreads();                                    // sel_l ready
+  // ---- this workgroup's segments (runs of tiles of one item) ----
+  // The first: len0 tiles from tile0 of item0; each further one: len1 tiles from tile1 of the
+  // item `step` away; n_it tiles in all.  A chunk that ends one item and starts the next
+  // takes the start first: all chunks then begin near tile 0 and walk the keys side by side
+  // (a window of n_tiles - chunk length tiles that L2 holds) instead of being spread over
+  // all of them.
+  int item0, tile0 = 0, len0 = n_tiles, tile1 = 0, len1 = n_tiles, step = 1, n_it, chunk = -1;
+  if ((int)blockIdx.x < xcd_grid(p.n_bundle)) {
+    const int u = xcd_remap(blockIdx.x, p.n_bundle);
+    if (u < 0) return;
+    item0 = u * p.bundle;
+    n_it = min(p.bundle, p.n_whole - item0) * n_tiles;
+  } else {
+    chunk = xcd_remap(blockIdx.x - xcd_grid(p.n_bundle), p.n_chunk);
+    if (chunk < 0) return;
+    const int n_split = p.B * p.H * ngrp - p.n_whole;
+    const int64_t lo = chunk_start(chunk, n_split, n_tiles, p.n_chunk);
+    n_it = (int)(chunk_start(chunk + 1, n_split, n_tiles, p.n_chunk) - lo);    // <= n_tiles
+    if (n_it <= 0) return;
+    item0 = p.n_whole + (int)(lo / n_tiles);
+    tile0 = (int)(lo % n_tiles);
+    len0 = min(n_it, n_tiles - tile0);
+    if (len0 < n_it) {
+      tile1 = tile0;
+      len1 = len0;
+      step = -1;
+      ++item0;
+      tile0 = 0;
+      len0 = n_it - len1;
+    }
+  }
 
   // ---- per-lane offsets, hoisted out of the loop ----
-  const bf16* kb = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh;
-  const bf16* vb = p.vt + (int64_t)b * p.vt_sb + (int64_t)h * p.vt_sh;
   int kro[8], vro[4];                                 // MFMA operand read offsets (bytes)
 #pragma unroll
   for (int kk = 0; kk < 8; ++kk) kro[kk] = k_lds_off(li, 2 * kk + hl) * 2;   // + 32 rows per sub-tile
 #pragma unroll
   for (int m = 0; m < 4; ++m) vro[m] = v_lds_off(li, 2 * m + hl) * 2;        // + 32 d rows per sub-tile
 
-  auto tile_tok0 = [&](int j) -> int {
-    return j < p.n_tgt_tiles ? j * ATT_BN : __builtin_amdgcn_readfirstlane(sel_l[j - p.n_tgt_tiles]);
-  };
-  // buffer of tile j
+  // buffer of iteration j's tile
   auto kbuf = [&](int j) -> unsigned char* { return smem + (j % FA_NBUF) * K_TILE_BYTES; };
   auto vbuf = [&](int j) -> unsigned char* {
     return smem + FA_NBUF * K_TILE_BYTES + (j % FA_NBUF) * V_TILE_BYTES;
   };
 
-  floatx16 o[4] = {};
-  floatx16 s[2];
-  bf16x8 pf[4];
-  float m_ref = -INFINITY, l_run = 0.f;
-  const float c = p.scale_log2;
-  const int n_tiles = p.n_tgt_tiles + p.n_sel;
-
-  // GEMM(k): O += V(k-1)^T P(k-1) (k >= 1) and S(k) = K(k) Q^T (k < n).  Operands are read
-  // from LDS into registers FA_PF MFMA steps ahead of their use (explicit software
-  // pipeline), so the matrix pipe does not wait on LDS latency.
-  auto gemm = [&](int k) {
-    __builtin_amdgcn_s_setprio(1);              // the matrix-feeding wave wins issue ties
-    if (k >= 1) {
-      const unsigned char* vs = vbuf(k - 1);
-      bf16x8 va[16];
-#pragma unroll
-      for (int t = 0; t < FA_PF; ++t)
-        va[t] = *reinterpret_cast<const bf16x8*>(vs + vro[t >> 2] + (t & 3) * 32 * ATT_BN * 2);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        if (t + FA_PF < 16) {
-          const int u = t + FA_PF;
-          va[u] = *reinterpret_cast<const bf16x8*>(vs + vro[u >> 2] + (u & 3) * 32 * ATT_BN * 2);
-        }
-        o[t & 3] = mfma32x32x16(va[t], pf[t >> 2], o[t & 3]);
-        __builtin_amdgcn_sched_barrier(0);    // keep the read-ahead order
-      }
-    }
-    if (k < n_tiles) {
-      const unsigned char* ks = kbuf(k);
-      bf16x8 ka[16];
-      floatx16 acc0 = {}, acc1 = {};
-#pragma unroll
-      for (int t = 0; t < FA_PF; ++t)
-        ka[t] = *reinterpret_cast<const bf16x8*>(ks + kro[t >> 1] + (t & 1) * 32 * ICSA_D * 2);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        if (t + FA_PF < 16) {
-          const int u = t + FA_PF;
-          ka[u] = *reinterpret_cast<const bf16x8*>(ks + kro[u >> 1] + (u & 1) * 32 * ICSA_D * 2);
-        }
-        if (t & 1) acc1 = mfma32x32x16(ka[t], qf[t >> 1], acc1);
-        else acc0 = mfma32x32x16(ka[t], qf[t >> 1], acc0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      s[0] = acc0;
-      s[1] = acc1;
-    }
-    __builtin_amdgcn_s_setprio(0);
-  };
-  // This wave's share (4 one-KB segments) of one tile's DMA, issued one segment at a time
-  // from inside the SOFT phase (see the slot schedule below).
-  const bool lag_w = group == 1;
+  // ---- DMA cursor: the next tile this wave's group fetches (K: group 1, V^T: group 0) ----
+  // It runs 2 to 4 tiles ahead of the computation, across item boundaries.
   const int dw = wave & 3;
   int dofs[4];                            // segment offsets: K rows (group 1) / V^T rows (group 0)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int sg = 4 * dw + i;
-    if (lag_w) {
+    if (lag) {
       const int kr = 4 * sg + (lane >> 4), kc = (lane & 15) ^ (kr & 15);
       dofs[i] = (int)(((int64_t)kr * p.k_ss + 8 * kc) * 2);
     } else {
@@ -169,38 +232,164 @@ icsa_flash_kernel(FlashParams p) {
       dofs[i] = (int)(((int64_t)vd * p.vt_sd + 8 * vc) * 2);
     }
   }
-  __amdgpu_buffer_rsrc_t dma_rs = make_rsrc(kb, 0);
+  int d_j = 0, d_tile = tile0, d_left = len0, d_item = item0, d_bh = 0;
+  int d_tok = 0;                          // group 1: token start of the cursor's tile
+  unsigned kv_ring = 0;                   // group 1: real key rows of the last four tiles, 8 bits each
+  const bf16* d_base = nullptr;           // K / V^T of the cursor's head
+  auto d_head = [&]() {
+    d_bh = d_item / ngrp;
+    const int b = d_bh / p.H, h = d_bh % p.H;
+    d_base = lag ? p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh : p.vt + (int64_t)b * p.vt_sb + (int64_t)h * p.vt_sh;
+  };
+  auto d_token = [&]() {                  // fetched one call ahead: the scalar load's latency is hidden
+    d_tok = d_tile * ATT_BN;
+    if (d_tile >= p.n_tgt_tiles && d_j < n_it)
+      d_tok = (p.sel_base + uniform_load(p.sel + (int64_t)d_bh * p.sel_stride + (d_tile - p.n_tgt_tiles))) * ATT_BN;
+  };
+  d_head();
+  if (lag) d_token();
+  __amdgpu_buffer_rsrc_t dma_rs = make_rsrc(d_base, 0);
   unsigned char* dma_dst = smem;
-  bool dma_on = false;
-  // sets up this wave's part of tile j: K(j) for group 1, V^T(j) for group 0
-  // Byte ranges fit 32 bits (checked at launch), so only the base addresses take 64-bit
-  // arithmetic: the setup runs in the SOFT phase, where its scalar work competes with the
-  // exponentials.  Past the last tile the issue stays branch-free: an empty range into a
-  // junk LDS area.
+  // Sets up this wave's part of the next tile.  Byte ranges fit 32 bits (checked at launch),
+  // so only the base addresses take 64-bit arithmetic: the setup runs in the SOFT phase,
+  // where its scalar work competes with the exponentials.  Past the last tile the issue
+  // stays branch-free: an empty range into a junk LDS area.
   const int k_row_bytes = (int)p.k_ss * 2;
   const int v_rec = (ICSA_D - 1) * (int)p.vt_sd * 2 + ATT_BN * 2;
-  auto dma_setup = [&](int j) {
-    dma_on = j < n_tiles;
-    const int tok0 = dma_on ? tile_tok0(j) : 0;
-    if (lag_w) {
-      const int k_valid = dma_on ? min(ATT_BN, p.Sk - tok0) : 0;
+  auto dma_setup = [&]() __attribute__((always_inline)) {
+    const bool on = d_j < n_it;
+    if (lag) {
+      const int k_valid = on ? min(ATT_BN, p.Sk - d_tok) : 0;
       const int k_rec = k_valid > 0 ? (k_valid - 1) * k_row_bytes + ICSA_D * 2 : 0;
-      dma_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(kb + (int64_t)tok0 * p.k_ss), (short)0, k_rec,
-                                                 0x00020000);
+      dma_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(d_base + (on ? (int64_t)d_tok * p.k_ss : 0)), (short)0,
+                                                 k_rec, 0x00020000);
+      kv_ring = (kv_ring << 8) | (unsigned)max(k_valid, 0);
     } else {
-      dma_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(vb + (int64_t)(dma_on ? j : 0) * ATT_BN),
-                                                 (short)0, dma_on ? v_rec : 0, 0x00020000);
+      dma_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(d_base + (int64_t)(on ? d_tile : 0) * ATT_BN),
+                                                 (short)0, on ? v_rec : 0, 0x00020000);
     }
-    dma_dst = !dma_on ? smem + FA_JUNK_OFF : (lag_w ? kbuf(j) : vbuf(j)) + dw * 4096;
+    dma_dst = !on ? smem + FA_JUNK_OFF : (lag ? kbuf(d_j) : vbuf(d_j)) + dw * 4096;
+    ++d_j;
+    ++d_tile;
+    if (--d_left == 0) {
+      d_tile = tile1;
+      d_left = len1;
+      d_item += step;
+      if (d_j < n_it) d_head();
+    }
+    if (lag) d_token();
   };
   auto dma_seg = [&](int i) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(dma_rs, (lds_ptr)(dma_dst + 1024 * i), 16, dofs[i], 0, 0, 0);
   };
+  auto issue_all = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma_seg(i);
+  };
+
+  struct Seg { int item, qblk, q_valid; };
+  auto seg_of = [&](int item) -> Seg {
+    const FlashParams& cp = cold_params();
+    Seg s;
+    s.item = item;
+    const int bh = item / ngrp, slot = item % ngrp * FA_QBLK_PER_WG + (wave >> 1);
+    const bool on = slot < cp.n_qblk;
+    s.qblk = !on ? 0 : (cp.qblocks ? uniform_load(cp.qblocks + (int64_t)bh * cp.qb_stride + cp.qb_offset + slot) : slot);
+    s.q_valid = on ? max(0, min(32, cp.Sq - s.qblk * ICSA_BLOCK - 32 * (wave & 1))) : 0;
+    return s;
+  };
+  Seg sg = seg_of(item0);                             // the segment whose output is in O
+  Seg nx = sg;                                        // the one after it, looked up a segment ahead
+  if (n_it > len0) nx = seg_of(item0 + step);
+
+  floatx16 o[4] = {};
+  floatx16 s[2];
+  bf16x8 qf[8];
+  bf16x8 pf[4];
+  float m_ref = FA_M_NONE, l_run = 0.f;
+  const float c = p.scale_log2;
+
+  auto load_q = [&](const Seg& g) __attribute__((always_inline)) {
+    const FlashParams& cp = cold_params();
+    const int bh = g.item / ngrp, b = bh / cp.H, h = bh % cp.H;
+    load_q_frags(qf, cp.q + (int64_t)b * cp.q_sb + (int64_t)(g.qblk * ICSA_BLOCK + 32 * (wave & 1)) * cp.q_ss +
+                         (int64_t)h * cp.q_sh, cp.q_ss, g.q_valid);
+  };
+  // The finished segment's O: to its output rows, or (a part of an item) to the partials.
+  auto flush = [&](bool part) __attribute__((always_inline)) {
+    const FlashParams& cp = cold_params();
+    if (part) {
+      const int u = chunk + (sg.item - cp.n_whole);
+      float* dst = cp.part + (int64_t)u * FA_PART_FLOATS + wave * FA_PART_WAVE;
+#pragma unroll
+      for (int ds = 0; ds < 4; ++ds)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<floatx4*>(dst + ((ds * 4 + g) * 64 + lane) * 4) =
+              floatx4{o[ds][4 * g], o[ds][4 * g + 1], o[ds][4 * g + 2], o[ds][4 * g + 3]};
+      dst[4096 + lane] = m_ref;
+      dst[4096 + 64 + lane] = l_run;
+      return;
+    }
+    const int bh = sg.item / ngrp, b = bh / cp.H, h = bh % cp.H;
+    const float inv_l = 1.f / xhalf_sum(l_run);
+    const float* oc = cp.out_c ? cp.out_c + ((int64_t)bh * cp.nb_q + sg.qblk) * ICSA_D : nullptr;
+    const OutView ov = cp.out;
+    const AlphaView av = cp.alpha;
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds) {
+      store_subtile<kBf16, kAlphaD>(smem + FA_STAGE_OFF + wave * FA_STAGE_WAVE, o[ds], ds, inv_l, ov, b, h,
+                    sg.qblk * ICSA_BLOCK + 32 * (wave & 1), sg.q_valid, oc, av);
+      __builtin_amdgcn_sched_barrier(0);              // one sub-tile's temporaries at a time
+    }
+  };
+
+  // GEMM(k): O += V(k-1)^T P(k-1) and S(k) = K(k) Q^T.  Operands are read from LDS into
+  // registers FA_PF MFMA steps ahead of their use (explicit software pipeline), so the
+  // matrix pipe does not wait on LDS latency.
+  auto gemm_pv = [&](int k) __attribute__((always_inline)) {
+    const unsigned char* vs = vbuf(k - 1);
+    bf16x8 va[16];
+#pragma unroll
+    for (int t = 0; t < FA_PF; ++t)
+      va[t] = *reinterpret_cast<const bf16x8*>(vs + vro[t >> 2] + (t & 3) * 32 * ATT_BN * 2);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      if (t + FA_PF < 16) {
+        const int u = t + FA_PF;
+        va[u] = *reinterpret_cast<const bf16x8*>(vs + vro[u >> 2] + (u & 3) * 32 * ATT_BN * 2);
+      }
+      o[t & 3] = mfma32x32x16(va[t], pf[t >> 2], o[t & 3]);
+      __builtin_amdgcn_sched_barrier(0);    // keep the read-ahead order
+    }
+  };
+  auto gemm_qk = [&](int k) __attribute__((always_inline)) {
+    const unsigned char* ks = kbuf(k);
+    bf16x8 ka[16];
+    floatx16 acc0 = {}, acc1 = {};
+#pragma unroll
+    for (int t = 0; t < FA_PF; ++t)
+      ka[t] = *reinterpret_cast<const bf16x8*>(ks + kro[t >> 1] + (t & 1) * 32 * ICSA_D * 2);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      if (t + FA_PF < 16) {
+        const int u = t + FA_PF;
+        ka[u] = *reinterpret_cast<const bf16x8*>(ks + kro[u >> 1] + (u & 1) * 32 * ICSA_D * 2);
+      }
+      if (t & 1) acc1 = mfma32x32x16(ka[t], qf[t >> 1], acc1);
+      else acc0 = mfma32x32x16(ka[t], qf[t >> 1], acc0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    s[0] = acc0;
+    s[1] = acc1;
+  };
   // SOFT(k): mask, P(k) against the reference max, and -- only when some probability of the
   // tile left the allowed range -- a rescale to the tile's row max and a second pass.  The
   // wave's DMA segments go out one at a time between the exponentials of the first pass.
-  auto soft = [&](int k) {
-    const int mask_from = k < p.n_tgt_tiles ? p.t_limit - k * ATT_BN : ATT_BN;
+  auto soft = [&](int tile) __attribute__((always_inline)) {
+    const int mask_from = tile < p.n_tgt_tiles ? p.t_limit - tile * ATT_BN : ATT_BN;
     if (mask_from < ATT_BN) {
       // keys >= mask_from as one 64-bit word; element i of sub-tile sub is key
       // 32 sub + 8 (i / 4) + 4 hl + i % 4, bit 8 (i / 4) + i % 4 of word sub of the word
@@ -235,9 +424,9 @@ icsa_flash_kernel(FlashParams p) {
         pf[2 * sb + (i >> 3)][i & 7] = (bf16)e;
       }
     float rs = (rsv[0] + rsv[1]) + (rsv[2] + rsv[3]);
-    // The partial sum exceeds FA_PSUM_MAX (or is NaN: the first tile, against m_ref = -inf)
-    // only when a score rose far above the reference: then raise the reference of every row
-    // whose tile max exceeds it, rescale O and l, and recompute the tile's probabilities.
+    // The partial sum exceeds FA_PSUM_MAX (or is NaN) only in a segment's first tile and when
+    // a score rose far above the reference: then raise the reference of every row whose tile
+    // max exceeds it, rescale O and l, and recompute the tile's probabilities.
     if (__ballot(!(rs <= FA_PSUM_MAX)) != 0ull) {
       float mx = -INFINITY;
 #pragma unroll
@@ -279,8 +468,13 @@ icsa_flash_kernel(FlashParams p) {
   // overwrites V(j - 4), last read (PV(j - 4)) in slot 2j - 5.  Loads complete in issue
   // order, so vmcnt(8) waits for all but this wave's two newest tiles.  Slots past the last
   // tile issue empty-range loads into a junk LDS area (the issue stays branch-free).
-  const bool compute = q_valid > 0;
-  const bool lag = group == 1;
+  // A segment boundary costs no slot: Q of the next segment is requested in the SOFT phase
+  // of the last tile (its registers are free since that tile's QK) and first used after the
+  // next GEMM's PV and the output, which are written from the accumulators between that
+  // GEMM's PV and QK (the scores and probabilities are not live there).  Those at least 8
+  // loads or stores are newer than the tiles waited for next, so these waits (group 0's in
+  // the same SOFT phase for Q and in the following one for the output, group 1's in the
+  // writing GEMM phase and in the following one) allow 8 more in flight.
   // zero key rows >= k_valid of a group-1 wave's K segments (rows 16 dw .. 16 dw + 15)
   auto fill_tail4 = [&](int j, int k_valid) {
     if (k_valid >= ATT_BN) return;
@@ -291,73 +485,247 @@ icsa_flash_kernel(FlashParams p) {
       for (int e = 0; e < 4; ++e) *reinterpret_cast<u32x4*>(dst + 16 * e) = u32x4{0u, 0u, 0u, 0u};
     }
   };
-  auto issue_all = [&]() {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dma_seg(i);
+  // wait for a tile, leaving the two tiles issued after it (past the last tile: the empty
+  // loads) in flight, and with `extra` the 8 loads or stores of a segment boundary
+  auto wait_tile = [&](bool extra) {
+    if (extra) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   };
-  // wait for a tile, leaving the `newer` (at most two) tiles issued after it in flight
-  auto wait_n = [&](int newer) {
-    if (newer >= 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else if (newer == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // group 1, at the end of GEMM(j - 1): K(j) complete, rows past Sk zero
+  auto wait_k = [&](int j, bool extra) {
+    if (!lag || j >= n_it) return;
+    wait_tile(extra);
+    fill_tail4(j, (int)((kv_ring >> 16) & 0xff));
   };
-  auto kvalid_of = [&](int j) -> int { return min(ATT_BN, p.Sk - tile_tok0(j)); };
   if (lag) {
-    for (int j = 0; j < 3; ++j) { dma_setup(j); issue_all(); }
-    wait_n(min(2, n_tiles - 1));          // K(0): K(1), K(2) are newer when they exist
-    fill_tail4(0, kvalid_of(0));
+    for (int j = 0; j < 3; ++j) { dma_setup(); issue_all(); }
   } else {
-    dma_setup(0); issue_all();
-    dma_setup(1); issue_all();
+    dma_setup(); issue_all();
+    dma_setup(); issue_all();
+  }
+  load_q(sg);
+  if (lag) {                               // K(0); its two newer tiles and Q as well
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    fill_tail4(0, (int)((kv_ring >> 16) & 0xff));
   }
   ATT_BARRIER();
   if (lag) {                               // slot 0 for group 1: K(3)
-    dma_setup(3);
+    dma_setup();
     issue_all();
     ATT_BARRIER();
   }
-  for (int k = 0; k <= n_tiles; ++k) {
-    if (compute) gemm(k);
-    if (lag && k + 1 < n_tiles) {          // K(k + 1); K(k + 2), K(k + 3) are newer
-      wait_n(min(2, n_tiles - (k + 2)));
-      fill_tail4(k + 1, kvalid_of(k + 1));
+  __builtin_amdgcn_s_setprio(1);           // the matrix-feeding wave wins issue ties
+  gemm_qk(0);
+  __builtin_amdgcn_s_setprio(0);
+  wait_k(1, false);
+  ATT_BARRIER();
+  int tile = tile0;                        // tile of iteration k
+  int seg_len = len0;
+  int k = 0;
+  // Every segment goes through the general iteration below for its first and its last tile
+  // and through the plain loop for those between.
+  bool wrote = false;                      // the GEMM phase before this SOFT phase wrote a segment out
+  int last = len0 - 1;                     // the segment's last iteration
+  for (;;) {
+    const bool ends = k == last, more = k + 1 < n_it;
+    bool q_ahead = false, writes = false;
+    if (ends && more) {
+      load_q(nx);
+      q_ahead = nx.q_valid > 0;
+      __builtin_amdgcn_sched_barrier(0);
     }
+    dma_setup();
+    soft(tile);
+    if (!lag) wait_tile(wrote || q_ahead);            // V(k)
     ATT_BARRIER();
-    dma_setup(lag ? k + 4 : k + 2);
-    if (compute && k < n_tiles) soft(k);
-    else issue_all();
-    if (!lag && k < n_tiles) wait_n(min(2, n_tiles - (k + 1)));   // V(k); V(k + 1), V(k + 2) newer
+    __builtin_amdgcn_s_setprio(1);
+    gemm_pv(k + 1);
+    if (!more) break;
+    if (ends) {
+      __builtin_amdgcn_s_setprio(0);
+      writes = sg.q_valid > 0;
+      if (writes) flush(seg_len != n_tiles);
+#pragma unroll
+      for (int ds = 0; ds < 4; ++ds) o[ds] = floatx16{};
+      l_run = 0.f;
+      tile = tile1 - 1;
+      seg_len = len1;
+      last = k + len1;
+      sg = nx;
+      if (n_it - (k + 1) > len1) nx = seg_of(sg.item + step);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+    }
+    gemm_qk(k + 1);
+    __builtin_amdgcn_s_setprio(0);
+    wait_k(k + 2, wrote || writes);
     ATT_BARRIER();
+    ++k;
+    ++tile;
+    if (!ends) {
+      for (; k < last; ++k, ++tile) {
+        dma_setup();
+        soft(tile);
+        if (!lag) wait_tile(false);
+        ATT_BARRIER();
+        __builtin_amdgcn_s_setprio(1);
+        gemm_pv(k + 1);
+        gemm_qk(k + 1);
+        __builtin_amdgcn_s_setprio(0);
+        wait_k(k + 2, false);
+        ATT_BARRIER();
+      }
+    }
+    wrote = writes;
   }
-  if (!lag) ATT_BARRIER();       // group 0's extra slot
-  // empty-range DMA of the last slots may still be in flight towards the junk area, which
-  // the output staging below overlaps
+  __builtin_amdgcn_s_setprio(0);
+  if (!lag) ATT_BARRIER();       // group 1's last SOFT phase ends here
+  // empty-range DMA of the last slots may still be in flight towards the junk area
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-
-  // ---- epilogue: 1/l, residual, scatter (the workgroup owns the CU's LDS: one round) ----
-  float* o_lds = reinterpret_cast<float*>(smem) + wave * 32 * O_LDS_STRIDE;
-  const float l_tot = xhalf_sum(l_run);
-  const float inv_l = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (q_valid > 0) stage_o(o_lds, o, inv_l);
-  __syncthreads();
-  if (q_valid > 0) {
-    const float* oc = p.out_c ? p.out_c + ((int64_t)bh * p.nb_q + qblk) * ICSA_D : nullptr;
-    store_rows(o_lds, p.out, b, h, qtok0, q_valid, oc, p.alpha);
-  }
+  if (sg.q_valid > 0) flush(seg_len != n_tiles);
 }
 
-hipError_t launch_flash(const FlashParams& p, hipStream_t stream) {
+// ------------------------------------------------------------------------------------------
+// Sums the partials of every split item and writes its rows: workgroup (item, wave of the
+// flash workgroup), wave ds: d-subtile ds of its 32 queries.  Segments in tile order, the
+// running reference max as in the flash loop: a fixed order, bitwise reproducible.
+// ------------------------------------------------------------------------------------------
+#define FC_AHEAD 4                                   // partials requested together
+
+template <bool kBf16, bool kAlphaD>
+__global__ void __launch_bounds__(256) icsa_flash_combine_kernel(FlashParams p) {
+  __shared__ __attribute__((aligned(16))) unsigned char stage[4][FA_STAGE_WAVE];
   const int ngrp = (p.n_qblk + FA_QBLK_PER_WG - 1) / FA_QBLK_PER_WG;
-  const int n_work = p.B * p.H * ngrp;
+  const int n_tiles = p.n_tgt_tiles + p.n_sel, n_split = p.B * p.H * ngrp - p.n_whole;
+  const int r = blockIdx.x / FA_WAVES, w = blockIdx.x % FA_WAVES;
+  const int ds = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int bh = (p.n_whole + r) / ngrp, grp = (p.n_whole + r) % ngrp;
+  const int slot = grp * FA_QBLK_PER_WG + (w >> 1);
+  if (slot >= p.n_qblk) return;                      // uniform for the workgroup
+  const int qblk = p.qblocks ? p.qblocks[(int64_t)bh * p.qb_stride + p.qb_offset + slot] : slot;
+  const int q_valid = min(32, p.Sq - qblk * ICSA_BLOCK - 32 * (w & 1));
+  if (q_valid <= 0) return;
+  // chunks c0 .. c1 - 1 hold tiles of the item: the last one that starts at or before its
+  // first tile, up to the last that starts before its end
+  auto start = [&](int c) -> int64_t { return chunk_start(c, n_split, n_tiles, p.n_chunk); };
+  const int64_t t0 = (int64_t)r * n_tiles, t1 = t0 + n_tiles;
+  int c0 = (int)((int64_t)r * p.n_chunk / n_split);
+  while (c0 + 1 < p.n_chunk && start(c0 + 1) <= t0) ++c0;
+  while (c0 > 0 && start(c0) > t0) --c0;
+  int c1 = c0 + 1;
+  while (c1 < p.n_chunk && start(c1) < t1) ++c1;
+  if (c1 - c0 == 1) return;                          // one workgroup had the whole item
+  const float* base = p.part + ((int64_t)(c0 + r) * FA_WAVES + w) * FA_PART_WAVE;
+  floatx16 acc = {};
+  float m = FA_M_NONE, l = 0.f;
+  for (int i = 0; i < c1 - c0; i += FC_AHEAD) {
+    floatx4 v[FC_AHEAD][4];
+    float ms[FC_AHEAD], ls[FC_AHEAD];
+#pragma unroll
+    for (int a = 0; a < FC_AHEAD; ++a) {
+      const float* src = base + (int64_t)min(i + a, c1 - c0 - 1) * FA_PART_FLOATS;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) v[a][g] = *reinterpret_cast<const floatx4*>(src + ((ds * 4 + g) * 64 + lane) * 4);
+      ms[a] = src[4096 + lane];
+      ls[a] = src[4096 + 64 + lane];
+    }
+#pragma unroll
+    for (int a = 0; a < FC_AHEAD; ++a) {
+      if (i + a >= c1 - c0) break;
+      const float mn = ms[a] > m ? ms[a] : m;
+      const float fo = __builtin_amdgcn_exp2f(m - mn), fn = __builtin_amdgcn_exp2f(ms[a] - mn);
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[4 * g + e] = fmaf(v[a][g][e], fn, acc[4 * g + e] * fo);
+      l = fmaf(ls[a], fn, l * fo);
+      m = mn;
+    }
+  }
+  const float* oc = p.out_c ? p.out_c + ((int64_t)bh * p.nb_q + qblk) * ICSA_D : nullptr;
+  store_subtile<kBf16, kAlphaD>(stage[ds], acc, ds, 1.f / xhalf_sum(l), p.out, bh / p.H, bh % p.H,
+                qblk * ICSA_BLOCK + 32 * (w & 1), q_valid, oc, p.alpha);
+}
+
+// ------------------------------------------------------------------------------------------
+// How the items are dealt out.  One workgroup fills a CU's LDS, so the chip runs FA_CUS of
+// them at a time, and a last round of r < FA_CUS items takes as long as a full one.
+//  * Those r items are cut into FA_CUS chunks of r n_tiles / FA_CUS tiles when that saves
+//    more than FA_COMBINE_TILES tiles: the sums' kernel takes 9-13 us and a tile 1.7 us of a
+//    workgroup, and a chunk's workgroup has a start of its own (about 5 us).  Chunks are not
+//    shorter than FA_MIN_CHUNK tiles.
+//  * Whole items go several to a workgroup, up to FA_BUNDLE_TILES tiles, in equal numbers:
+//    beyond that a workgroup's start no longer counts and many workgroups even out the
+//    CUs (220 tiles an item, 8.6 rounds: 4,710 us with bundles of 1 or 2 items, 4,870 us
+//    with 8; 8 tiles an item, 40 rounds: 783, 775 and 773 us with 14, 20 and 40 items).
+// ------------------------------------------------------------------------------------------
+#define FA_CUS 256
+#define FA_MIN_CHUNK 4
+#define FA_COMBINE_TILES 12
+#define FA_BUNDLE_TILES 512
+
+FlashPlan flash_plan(int64_t n_work, int n_tiles, bool may_split) {
+  FlashPlan f;
+  const int64_t rounds = n_work / FA_CUS, rest = n_work % FA_CUS;
+  f.n_whole = (int)n_work;
+  f.n_chunk = 0;
+  if (may_split && rest > 0) {
+    const int64_t g = std::min<int64_t>(FA_CUS, std::max<int64_t>(rest, rest * n_tiles / FA_MIN_CHUNK));
+    if (n_tiles - (rest * n_tiles + g - 1) / g > FA_COMBINE_TILES) {
+      f.n_whole = (int)(rounds * FA_CUS);
+      f.n_chunk = (int)g;
+    }
+  }
+  int64_t m = 1;
+  if (f.n_whole > FA_CUS) {
+    const int64_t per_cu = (f.n_whole + FA_CUS - 1) / FA_CUS;
+    const int64_t want = std::max<int64_t>(1, std::min<int64_t>(per_cu, FA_BUNDLE_TILES / n_tiles));
+    const int64_t k = (per_cu + want - 1) / want;
+    m = (per_cu + k - 1) / k;
+
+  }
+  f.bundle = (int)m;
+  f.n_bundle = (int)((f.n_whole + m - 1) / m);
+  f.part_bytes = f.n_chunk ? (int64_t)(f.n_chunk + rest) * FA_PART_FLOATS * 4 : 0;
+  return f;
+}
+
+int64_t flash_items(int BH, int n_qblk) { return (int64_t)BH * ((n_qblk + FA_QBLK_PER_WG - 1) / FA_QBLK_PER_WG); }
+
+int64_t flash_part_bytes_max(int n_tiles) {
+  return n_tiles > FA_COMBINE_TILES ? (int64_t)(2 * FA_CUS - 1) * FA_PART_FLOATS * 4 : 0;
+}
+
+// kAlphaD: the residual weight varies along the head dim (its own instantiation: its gathers
+// would cost the usual one registers)
+template <bool kBf16, bool kAlphaD>
+static hipError_t run_flash(const FlashParams& p, int64_t n_work, hipStream_t stream) {
+  static std::atomic<unsigned> lds_set{0u};
+  const hipError_t attr = ensure_lds_limit(reinterpret_cast<const void*>(icsa_flash_kernel<kBf16, kAlphaD>),
+                                           FA_LDS_BYTES, &lds_set);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((icsa_flash_kernel<kBf16, kAlphaD>), dim3(xcd_grid(p.n_bundle) + xcd_grid(p.n_chunk)),
+                     dim3(FA_THREADS), FA_LDS_BYTES, stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || p.n_chunk == 0) return e;
+  hipLaunchKernelGGL((icsa_flash_combine_kernel<kBf16, kAlphaD>), dim3((unsigned)(n_work - p.n_whole) * FA_WAVES),
+                     dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_flash(FlashParams p, hipStream_t stream) {
+  const int64_t n_work = flash_items(p.B * p.H, p.n_qblk);
+  const int n_tiles = p.n_tgt_tiles + p.n_sel;
   if (n_work == 0) return hipSuccess;
-  if (p.n_tgt_tiles + p.n_sel <= 0 || p.n_sel > FA_MAX_SEL) return hipErrorInvalidValue;
+  if (n_tiles <= 0 || n_work > 0x7fffffffLL / 2) return hipErrorInvalidValue;
   // per-(b, h) slices must be addressable with 32-bit buffer offsets
   if ((int64_t)p.Sk * p.k_ss * 2 > 0x7fffffffLL || (int64_t)ICSA_D * p.vt_sd * 2 > 0x7fffffffLL)
     return hipErrorInvalidValue;
-  static std::atomic<unsigned> lds_set{0u};
-  const hipError_t attr = ensure_lds_limit(reinterpret_cast<const void*>(icsa_flash_kernel), FA_LDS_BYTES, &lds_set);
-  if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(icsa_flash_kernel, dim3(xcd_grid(n_work)), dim3(FA_THREADS), FA_LDS_BYTES, stream, p);
-  return hipGetLastError();
+  FlashPlan f = flash_plan(n_work, n_tiles, true);
+  if (f.part_bytes > p.part_bytes) f = flash_plan(n_work, n_tiles, false);
+  p.n_whole = f.n_whole; p.n_chunk = f.n_chunk; p.bundle = f.bundle; p.n_bundle = f.n_bundle;
+  const bool alpha_d = p.out_c != nullptr && p.alpha.p != nullptr && p.alpha.sd != 0;
+  if (p.out.dtype == ICSA_DT_BF16)
+    return alpha_d ? run_flash<true, true>(p, n_work, stream) : run_flash<true, false>(p, n_work, stream);
+  return alpha_d ? run_flash<false, true>(p, n_work, stream) : run_flash<false, false>(p, n_work, stream);
 }

@@ -109,7 +109,7 @@ __device__ __forceinline__ int xcd_remap(int wg, int n_work) {
   int w = (wg % nx) * per + wg / nx;
   return w < n_work ? w : -1;
 }
-__host__ __forceinline__ int xcd_grid(int n_work) { return ((n_work + 7) / 8) * 8; }
+__host__ __device__ __forceinline__ int xcd_grid(int n_work) { return ((n_work + 7) / 8) * 8; }
 
 // MFMA wrappers (gfx950).  Operand/result layouts (checked on the device):
 //  32x32x16 bf16: A lane l holds A[l%32][8*(l/32)+i], B lane l holds B[8*(l/32)+i][l%32],

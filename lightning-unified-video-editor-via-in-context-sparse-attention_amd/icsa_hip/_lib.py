@@ -33,7 +33,7 @@ STAGES = ["start", "pool", "compressed", "select", "sparse", "flash"]
 
 # workspace slots of icsa_editing_sparse_attention (enum icsa_ws_slot)
 WS_SLOTS = ["QSUM", "KSUM", "VSUM", "VT", "QB", "KB", "VB", "LOGITS", "OUTC", "SHARP", "SRCSCORE",
-            "SEL", "ORDER", "KVMAP", "KC32", "KC", "VCT", "L3", "VC", "COLP", "L3S", "RSTAT"]
+            "SEL", "ORDER", "KVMAP", "KC32", "KC", "VCT", "L3", "VC", "COLP", "L3S", "RSTAT", "FLASHP"]
 
 # every symbol include/icsa.h declares
 EXPORTS = [
