@@ -812,22 +812,35 @@ int icsa_sparse_piecewise_attn_fwd(
 
 namespace {
 struct BwLayout {
-  int64_t ksum, vsum, dvec, selbits, kcb, vcb, dkc, dvc, total;
+  int64_t ksum, vsum, dvec, selbits, seltr, kcb, vcb, dkc, dvc, total;
   int nsplit, qb_per_split;
 };
-// Interval partials: enough (chunk, query-range) workgroups to fill the GPU, each range at
-// least 8 and at most 1024 query blocks long (the kernel stages a range's selection words
-// in LDS).
+// Interval partials: the query blocks are cut in nsplit ranges, one workgroup per (chunk,
+// range).  512 workgroups run at a time (two per CU); one costs its range plus about 3 steps,
+// and every further range 0.015 steps per (head, chunk) for the f32 partials it writes and
+// the exact part reads (1 KB each way per block sum at the copy rate, a step being 1.8 us).
+// The cheapest count at 40 heads, 122 query blocks, 2 chunks: 6 ranges (one round of 480
+// workgroups, 71 us; 16 ranges: 92 us); at 4 heads, 32 query blocks: 32 (11 us; 4: 18 us).
+int bwd_splits(int64_t BHc, int NQ) {
+  int best = 1;
+  double cost = 1e30;
+  for (int n = 1; n <= std::min(NQ, 128); ++n) {
+    const int per = ceil_div(NQ, n);
+    if (ceil_div(NQ, per) != n) continue;               // the same range length with fewer ranges
+    const double c = (double)((BHc * n + 511) / 512) * (per + 3) + 0.015 * (double)BHc * n;
+    if (c < cost) {
+      cost = c;
+      best = n;
+    }
+  }
+  return best;
+}
 BwLayout bwd_layout(int B, int H, int TQ, int TKV) {
   const int64_t BH = (int64_t)B * H;
   const int NQ = ceil_div(TQ, ICSA_BLOCK), NKV = ceil_div(TKV, ICSA_BLOCK);
   const int nc = ceil_div(NKV, 64), NKVp = nc * 64;
   BwLayout L;
-  // interval workgroups: about five rounds of the 512 that fit on the GPU (two per CU), so
-  // the last round's tail is small (1,080 workgroups, 2.1 rounds, measured 2 % slower)
-  const int want = std::max(1, ceil_div(2560, (int)std::max<int64_t>(1, BH * nc)));
-  int qbps = std::max(8, ceil_div(NQ, want));
-  qbps = std::min(qbps, std::min(NQ, 1024));
+  const int qbps = ceil_div(NQ, bwd_splits(BH * nc, NQ));
   L.qb_per_split = qbps;
   L.nsplit = ceil_div(NQ, qbps);
   int64_t o = 0;
@@ -835,6 +848,7 @@ BwLayout bwd_layout(int B, int H, int TQ, int TKV) {
   L.vsum = o; o += align256(BH * NKV * ICSA_D * 4);
   L.dvec = o; o += align256(BH * (int64_t)NQ * ICSA_BLOCK * 4);   // D rows padded to whole blocks
   L.selbits = o; o += align256(BH * NQ * (int64_t)nc * 8);
+  L.seltr = o; o += align256(BH * NKV * (int64_t)ceil_div(NQ, 64) * 8);
   L.kcb = o; o += align256(BH * NKVp * ICSA_D * 2);
   L.vcb = o; o += align256(BH * NKVp * ICSA_D * 2);
   L.dkc = o; o += align256((int64_t)L.nsplit * BH * NKVp * ICSA_D * 4);
@@ -912,6 +926,7 @@ int icsa_sparse_piecewise_attn_bwd(
   p.ksum = pk.sums[1]; p.vsum = pk.sums[2];
   p.dvec = reinterpret_cast<float*>(ws + L.dvec);
   p.selbits = reinterpret_cast<unsigned long long*>(ws + L.selbits);
+  p.seltr = reinterpret_cast<unsigned long long*>(ws + L.seltr);
   p.kcb = reinterpret_cast<bf16*>(ws + L.kcb);
   p.vcb = reinterpret_cast<bf16*>(ws + L.vcb);
   p.dkc_part = reinterpret_cast<float*>(ws + L.dkc);

@@ -46,6 +46,34 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, in
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
+// LDS DMA issued from inline assembly: the compiler does not track these loads, so it
+// inserts no waits for them before LDS reads of other tiles (it cannot tell the buffers of a
+// ring apart, and takes every transposing read for a read of the tile in flight); the kernel
+// waits itself.  Lane l of one instruction lands at lds_addr + 16 l (4 l).  The resource
+// words are those of make_rsrc (raw buffer, no stride), in scalar registers.
+__device__ __forceinline__ u32x4 dma_rsrc(const void* base, int64_t bytes) {
+  const unsigned long long a = (unsigned long long)base;
+  const int n = bytes > 0x7fffffffLL ? 0x7fffffff : (int)(bytes < 0 ? 0 : bytes);
+  u32x4 r;
+  r[0] = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a);
+  r[1] = (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)(a >> 32) & 0xffffu));
+  r[2] = (unsigned)__builtin_amdgcn_readfirstlane(n);
+  r[3] = 0x00020000u;
+  return r;
+}
+__device__ __forceinline__ void lds_dma16(unsigned lds_addr, int voff, u32x4 rs) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(lds_addr), "v"(voff), "s"(rs) : "memory", "m0");
+}
+__device__ __forceinline__ void lds_dma4(unsigned lds_addr, int voff, u32x4 rs) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+               :: "s"(lds_addr), "v"(voff), "s"(rs) : "memory", "m0");
+}
+__device__ __forceinline__ unsigned lds_u32(const void* p) {
+  return (unsigned)__builtin_amdgcn_readfirstlane(
+      (int)(unsigned)(size_t)(const __attribute__((address_space(3))) void*)p);
+}
+
 // Workgroup barrier without a memory fence.  __syncthreads() also waits for every
 // outstanding LDS-DMA load (vmcnt(0)), which would cut a tile prefetch short; kernels
 // using this wait for their tile DMA explicitly.  LDS reads and writes issued before the

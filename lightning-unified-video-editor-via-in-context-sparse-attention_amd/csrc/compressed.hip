@@ -384,29 +384,6 @@ __global__ void __launch_bounds__(256) icsa_vmean_split_kernel(CompressedParams 
   }
 }
 
-// LDS DMA issued from inline assembly: the compiler does not track these loads, so it
-// inserts no waits for them before LDS reads of the other stage; the kernel waits itself
-// (vmcnt(0) before the barrier that opens each chunk).  Lane l of one instruction lands at
-// lds_addr + 16 l.  The resource words are those of make_rsrc (raw buffer, no stride).
-__device__ __forceinline__ u32x4 rw_rsrc(const void* base, int64_t bytes) {
-  const unsigned long long a = (unsigned long long)base;
-  const int n = bytes > 0x7fffffffLL ? 0x7fffffff : (int)(bytes < 0 ? 0 : bytes);
-  u32x4 r;
-  r[0] = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a);
-  r[1] = (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)(a >> 32) & 0xffffu));
-  r[2] = (unsigned)__builtin_amdgcn_readfirstlane(n);
-  r[3] = 0x00020000u;
-  return r;
-}
-__device__ __forceinline__ void rw_dma16(unsigned lds_addr, int voff, u32x4 rs) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(lds_addr), "v"(voff), "s"(rs) : "memory", "m0");
-}
-__device__ __forceinline__ unsigned lds_u32(const void* p) {
-  return (unsigned)__builtin_amdgcn_readfirstlane(
-      (int)(unsigned)(size_t)(const __attribute__((address_space(3))) void*)p);
-}
-
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 icsa_compressed_rows_kernel(CompressedParams p, int NBp) {
   // two stages of the chunk operands as separate objects; 65 KB in all, two workgroups per CU
@@ -431,8 +408,8 @@ icsa_compressed_rows_kernel(CompressedParams p, int NBp) {
   // DMA sources: the strip's logit rows (rows past NB and keys past the last row are
   // outside the resource: no load, and P is zero there) and the head's value planes
   const float* Lbh = p.L + (int64_t)bh * NB * NB;
-  const u32x4 rs_l = rw_rsrc(Lbh + (int64_t)r_base * NB, (int64_t)max(0, min(64, NB - r_base)) * NB * 4);
-  const u32x4 rs_v = rw_rsrc(p.vmt + (int64_t)bh * 2 * ICSA_D * NBp, (int64_t)2 * ICSA_D * NBp * 2);
+  const u32x4 rs_l = dma_rsrc(Lbh + (int64_t)r_base * NB, (int64_t)max(0, min(64, NB - r_base)) * NB * 4);
+  const u32x4 rs_v = dma_rsrc(p.vmt + (int64_t)bh * 2 * ICSA_D * NBp, (int64_t)2 * ICSA_D * NBp * 2);
   // logits: wave w moves rows 8 w .. + 7 (128 bytes each), 16 bytes per lane
   const int l_off = ((8 * w + (lane >> 3)) * NB + 4 * (lane & 7)) * 4;
   // value planes: instruction j (0, 1) of wave w moves rows R = 16 (2 w + j) .. + 15 of the
@@ -445,9 +422,9 @@ icsa_compressed_rows_kernel(CompressedParams p, int NBp) {
     v_off[j] = ((R >> 7) * ICSA_D + (R & 127)) * NBp * 2 + 16 * ((lane & 3) ^ (R & 3));
   }
   auto issue = [&](int c, float* lc, bf16* vc) {
-    rw_dma16(lds_u32(lc + 256 * w), l_off + 128 * c, rs_l);
+    lds_dma16(lds_u32(lc + 256 * w), l_off + 128 * c, rs_l);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) rw_dma16(lds_u32(vc + 512 * (2 * w + j)), v_off[j] + 64 * c, rs_v);
+    for (int j = 0; j < 2; ++j) lds_dma16(lds_u32(vc + 512 * (2 * w + j)), v_off[j] + 64 * c, rs_v);
   };
 
   const int li = lane & 31, hl = lane >> 5;

@@ -219,6 +219,7 @@ struct SparseBwdParams {
   const float* ksum; const float* vsum;   // [BH, NKV, D] f32 block sums
   float* dvec;                       // [BH, TQ] rowsum(dO * O)
   unsigned long long* selbits;       // [BH, NQ, nc] selected key blocks per query block
+  unsigned long long* seltr;         // [BH, NKV, cdiv(NQ, 64)] the same by key block
   bf16* kcb; bf16* vcb;              // [BH, NKVp, D] bf16 block sums, rows >= NKV zero
   float* dkc_part; float* dvc_part;  // [nsplit, BH, NKVp, D] interval partials
   OutView dq, dk, dv;                // (sb, token stride, sh, dtype)

@@ -29,11 +29,26 @@
 // TKV are masked out of the exact part (triton_kernels.py:348), and gradient rows past TQ /
 // TKV are not stored.
 // P and dS are rounded to bf16 for the MFMA (the reference rounds P for dv and uses fp32
-// dots for dq / dk).  Workgroup = 2 waves; wave w owns queries (or keys) 32 w .. 32 w + 31.
+// dots for dq / dk).
+//
+// Workgroup = 4 waves on one 64 x 64 pair of blocks at a time: wave w computes the quadrant of
+// S and dP of 32 keys (or queries) it keeps in registers, w % 2, by 32 rows of the tile in LDS,
+// w / 2, and adds the products over its own quadrant.  At 228-256 registers two such
+// workgroups (at most 76 KB of LDS each) share a CU, so one wave's elementwise work and LDS
+// reads run beside another's MFMAs; with two waves per workgroup, 64 rows each and 308-412
+// registers, every SIMD held a single wave.  Measured at 40 heads, 7,800 tokens, 12 of 122
+// blocks, against that: dq 375 -> 300 us, dk / dv exact 500 -> 360 us, interval 90 -> 71 us
+// (4 heads, 2,048 tokens: 14.6 -> 11.7, 28 -> 21, 22 -> 11 us).  A step of the exact part then
+// takes 3,700 cycles with two workgroups on the CU, 55 % of them MFMA; about a third of a
+// workgroup's time is its start (first tiles, K and V) and its end (sums of the halves,
+// output), which is what bounds it at 12 steps.  Copies: all tiles from L2 5 % faster, no
+// tiles at all 17 %; no elementwise masks: the same.
+// Waits: the tile DMA is inline assembly (lds_dma16); behind the builtin the compiler waited
+// for the next step's tiles (vmcnt(0)) before every step's transposing reads.
 #include "attn_tile.h"
 #include "icsa_kernels.h"
 
-#define BW_THREADS 128
+#define BW_THREADS 256
 #define BW_MAX_TOPK 512
 #define BW_MAX_CHUNKS 32                 // NKV <= 2048
 #define BW_MAX_NQ 4096
@@ -75,7 +90,9 @@ __global__ void __launch_bounds__(256) icsa_sparse_bwd_rows_kernel(SparseBwdPara
   if (t < p.nc) p.selbits[((int64_t)bh * p.NQ + i) * p.nc + t] = sel[t];
 }
 
-// prep: bf16 block sums from the f32 sums (rows >= NKV zero)
+// prep: bf16 block sums from the f32 sums (rows >= NKV zero), and the chunk's part of the
+// selection bitmap by key block: the exact dk / dv workgroups then walk their query blocks with
+// scalar loads and bit scans alone, instead of listing them in LDS between two barriers.
 __global__ void __launch_bounds__(256) icsa_sparse_bwd_sums_kernel(SparseBwdParams p) {
   const int ch = blockIdx.x, bh = blockIdx.y;
   const int t = threadIdx.x;
@@ -97,6 +114,20 @@ __global__ void __launch_bounds__(256) icsa_sparse_bwd_sums_kernel(SparseBwdPara
       *reinterpret_cast<bf16x8*>(dst + 8 * g) = pack8_bf16(v);
     }
   }
+  // 64 x 64 bits at a time: lane l holds query block 64 w + l's word, then key block 64 ch + l's
+  const int lane = t & 63, n_qw = (p.NQ + 63) / 64;
+  for (int w = t >> 6; w < n_qw; w += 4) {
+    const int i = 64 * w + lane;
+    const unsigned long long word = i < p.NQ ? p.selbits[((int64_t)bh * p.NQ + i) * p.nc + ch] : 0ull;
+    unsigned long long mine = 0ull;
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {
+      const unsigned long long b = __ballot((word >> j) & 1ull);
+      if (lane == j) mine = b;
+    }
+    const int key = ch * ICSA_BLOCK + lane;
+    if (key < p.NKV) p.seltr[((int64_t)bh * p.NKV + key) * n_qw + w] = mine;
+  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -109,46 +140,29 @@ __global__ void __launch_bounds__(256) icsa_sparse_bwd_sums_kernel(SparseBwdPara
 // ------------------------------------------------------------------------------------------
 #define BW_WAIT(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
 
+// A wave-uniform word that an earlier kernel wrote, through the scalar cache.
+template <typename T>
+__device__ __forceinline__ T uniform_word(const T* p) {
+  return *(const __attribute__((address_space(4))) T*)(unsigned long long)p;
+}
+
 // Row tiles use the shared layout of attn_tile.h (rt_swz / rt_off).
 #define BW_PF 3                 // MFMA operand read-ahead (steps)
 
-// S^T (or S) for the 64 rows of a backward row tile: s[sub] covers rows 32 sub .. 32 sub + 31.
-// Step t uses sub = t % 2 and dims 16 (t / 2) .. + 15; operands are read BW_PF steps ahead
-// (with one wave per SIMD nothing else hides the LDS latency).
-__device__ __forceinline__ void qk_tile_bw(floatx16 s[2], const bf16* tile, const bf16x8 bf[8]) {
-  const int lane = threadIdx.x & 63;
-  const int li = lane & 31, hl = lane >> 5;
-  auto ld = [&](int t) -> bf16x8 {
-    return *reinterpret_cast<const bf16x8*>(tile + rt_off(32 * (t & 1) + li, 2 * (t >> 1) + hl));
-  };
-  bf16x8 a[16];
-#pragma unroll
-  for (int t = 0; t < BW_PF; ++t) a[t] = ld(t);
-  __builtin_amdgcn_sched_barrier(0);
-  floatx16 acc0 = {}, acc1 = {};
-#pragma unroll
-  for (int t = 0; t < 16; ++t) {
-    if (t + BW_PF < 16) a[t + BW_PF] = ld(t + BW_PF);
-    if (t & 1) acc1 = mfma32x32x16(a[t], bf[t >> 1], acc1);
-    else acc0 = mfma32x32x16(a[t], bf[t >> 1], acc0);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  s[0] = acc0;
-  s[1] = acc1;
-}
+// Byte offset of this lane's 16-byte chunk hl of tile row `row`; chunk 2 kk + hl is at that
+// offset ^ (kk << 5) (the swizzle only flips chunk bits).
+__device__ __forceinline__ int bw_row_off(int row, int hl) { return rt_off(row, hl) * 2; }
 
-// Rows >= valid lie outside the buffer range and land nothing: bw_fill_rows zeroes them once
-// the tile's loads have completed.
+// One wave's quarter of a tile: rows 16 w .. 16 w + 15.  Rows >= valid lie outside the buffer
+// range and land nothing: bw_fill_rows zeroes them once the tile's loads have completed.
 __device__ __forceinline__ void bw_dma_rows(unsigned char* tile, const bf16* base, int64_t rs, int wave,
                                             int lane, int valid = ICSA_BLOCK) {
-  const __amdgpu_buffer_rsrc_t rsrc =
-      make_rsrc(base, valid > 0 ? ((int64_t)(valid - 1) * rs + ICSA_D) * 2 : 0);
-  unsigned char* dst = tile + wave * 8192;
+  const u32x4 rs4 = dma_rsrc(base, valid > 0 ? ((int64_t)(valid - 1) * rs + ICSA_D) * 2 : 0);
+  const unsigned dst = lds_u32(tile + wave * 4096);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 32 * wave + 4 * i + (lane >> 4);
-    const int off = (int)(r * rs * 2) + (((lane & 15) ^ rt_swz(r)) << 4);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(dst + 1024 * i), 16, off, 0, 0, 0);
+  for (int i = 0; i < 4; ++i) {
+    const int r = 16 * wave + 4 * i + (lane >> 4);
+    lds_dma16(dst + 1024 * i, (int)(r * rs * 2) + (((lane & 15) ^ rt_swz(r)) << 4), rs4);
   }
 }
 
@@ -156,27 +170,95 @@ __device__ __forceinline__ void bw_dma_rows(unsigned char* tile, const bf16* bas
 __device__ __forceinline__ void bw_fill_rows(unsigned char* tile, int valid, int wave, int lane) {
   if (valid >= ICSA_BLOCK) return;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 32 * wave + 4 * i + (lane >> 4);
+  for (int i = 0; i < 4; ++i) {
+    const int r = 16 * wave + 4 * i + (lane >> 4);
     if (r >= valid) *reinterpret_cast<u32x4*>(tile + r * ICSA_D * 2 + (lane & 15) * 16) = u32x4{0u, 0u, 0u, 0u};
   }
 }
 
+// s = X Bx, d = Y By over 128 dims for 32 rows of the tiles x and y (this lane's row at byte
+// offset `ro`): 16 MFMAs, alternating, operands read BW_PF steps ahead.
+__device__ __forceinline__ void bw_scores(floatx16& s, floatx16& d, const unsigned char* x, const unsigned char* y,
+                                          int ro, const bf16x8 bx[8], const bf16x8 by[8]) {
+  auto ld = [&](int t) -> bf16x8 {
+    return *reinterpret_cast<const bf16x8*>(((t & 1) ? y : x) + (ro ^ ((t >> 1) << 5)));
+  };
+  bf16x8 a[16];
+#pragma unroll
+  for (int t = 0; t < BW_PF; ++t) a[t] = ld(t);
+  __builtin_amdgcn_sched_barrier(0);
+  s = d = floatx16{};
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    if (t + BW_PF < 16) a[t + BW_PF] = ld(t + BW_PF);
+    if (t & 1) d = mfma32x32x16(a[t], by[t >> 1], d);
+    else s = mfma32x32x16(a[t], bx[t >> 1], s);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// o[ND d-subtiles] += X^T P over NM 16-row steps from m0 of row tile X (p[m]: the bf16 B
+// operand of step m0 + m, straight from the score accumulators).  tro: the transposing read's
+// offset for the first d-subtile; the next 32 dims are 4 chunks on, byte bit 6 of the swizzled
+// offset flipped (64 dims: bit 7).
+template <int ND, int NM>
+__device__ __forceinline__ void bw_accum(floatx16* o, const unsigned char* tile, int tro, int m0,
+                                         const bf16x8* p) {
+  constexpr int N = ND * NM;
+  const unsigned char* base = tile + m0 * 16 * ICSA_D * 2;
+  auto ld = [&](int t) -> bf16x8 {
+    const int off = tro ^ ((t % ND) << 6);
+    const int st = (t / ND) * 16 * ICSA_D * 2;
+    const rt_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((rt_lds_v4s)(base + off + st));
+    const rt_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((rt_lds_v4s)(base + rt_tr_hi<false>(off) + st));
+    const short __attribute__((ext_vector_type(8))) a8 = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(bf16x8, a8);
+  };
+  bf16x8 a[N];
+#pragma unroll
+  for (int t = 0; t < BW_PF; ++t) a[t] = ld(t);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int t = 0; t < N; ++t) {
+    if (t + BW_PF < N) a[t + BW_PF] = ld(t + BW_PF);
+    o[t % ND] = mfma32x32x16(a[t], p[t / ND], o[t % ND]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Adds the accumulators of a wave pair (same rows / keys, the two halves of the summed
+// dimension) through LDS and leaves mul * sum as rows for store_rows: each wave hands over the
+// d-subtiles that the other one adds up.
+__device__ __forceinline__ void bw_reduce_stage(float* o_lds, const floatx16 o[4], int half, float mul) {
+  const int lane = threadIdx.x & 63, li = lane & 31;
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      o_lds[li * O_LDS_STRIDE + 32 * (2 * (half ^ 1) + d) + acc_row(i, lane)] = half ? o[d][i] : o[2 + d][i];
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float* x = &o_lds[li * O_LDS_STRIDE + 32 * (2 * half + d) + acc_row(i, lane)];
+      *x = ((half ? o[2 + d][i] : o[d][i]) + *x) * mul;
+    }
+  __syncthreads();
+}
 
 // ------------------------------------------------------------------------------------------
 // dq: one workgroup per query block.  Steps t = 0 .. n_ex + nc - 1: the valid selected
-// blocks, then the interval chunks.  Per step the K and V rows (16 DMA per wave) land in
+// blocks, then the interval chunks.  Per step the K and V rows (8 DMA per wave) land in
 // one of two buffers while the other step's S^T = K Q^T, dP^T = V dO^T and
-// dQ^T += K^T dS^T (K^T read transposed from the K rows) run.
+// dQ^T += K^T dS^T (K^T read transposed from the K rows) run.  Wave w: queries
+// 32 (w % 2) .. + 31 in registers, keys 32 (w / 2) .. + 31 of each step.
 // ------------------------------------------------------------------------------------------
-#define BWQ_LDS_BYTES (4 * K_TILE_BYTES + BW_MAX_TOPK * 4 + BW_MAX_CHUNKS * 8 + 16)
+#define BWQ_LDS_BYTES (4 * K_TILE_BYTES)
 
-__global__ void __launch_bounds__(BW_THREADS) icsa_sparse_bwd_dq_kernel(SparseBwdParams p) {
+__global__ void __launch_bounds__(BW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+icsa_sparse_bwd_dq_kernel(SparseBwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_q[];
-  int* src_l = reinterpret_cast<int*>(smem_q + 4 * K_TILE_BYTES);
-  unsigned long long* sel_l = reinterpret_cast<unsigned long long*>(src_l + BW_MAX_TOPK);
-  int* n_ex_l = reinterpret_cast<int*>(sel_l + BW_MAX_CHUNKS);
-
   const int n_work = p.B * p.H * p.NQ;
   const int work = xcd_remap(blockIdx.x, n_work);
   if (work < 0) return;
@@ -184,23 +266,44 @@ __global__ void __launch_bounds__(BW_THREADS) icsa_sparse_bwd_dq_kernel(SparseBw
   const int b = bh / p.H, h = bh % p.H;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int li = lane & 31;
-  const int qtok0 = qb * ICSA_BLOCK + 32 * wave;
+  const int li = lane & 31, hl = lane >> 5;
+  const int qh = wave & 1, kh = wave >> 1;
+  const int qtok0 = qb * ICSA_BLOCK + 32 * qh;
 
-  for (int c = tid; c < p.nc; c += BW_THREADS) sel_l[c] = p.selbits[((int64_t)bh * p.NQ + qb) * p.nc + c];
-  if (wave == 0) {                                     // valid selected blocks, list order kept
-    const int* row = p.idx + ((int64_t)bh * p.NQ + qb) * p.top_k;
-    int cnt = 0;
-    for (int base = 0; base < p.top_k; base += 64) {
-      const int u = base + lane;
-      const int j = u < p.top_k ? row[u] : -1;
-      const bool on = j >= 0 && j < p.NKV;            // out-of-range entries: zero blocks, no gradient
-      const unsigned long long bal = __ballot(on);
-      if (on) src_l[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = j;
-      cnt += __popcll(bal);
+  const bf16* kb = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh;
+  const bf16* vb = p.v + (int64_t)b * p.v_sb + (int64_t)h * p.v_sh;
+  const bf16* kcb = p.kcb + (int64_t)bh * p.NKVp * ICSA_D;
+  const bf16* vcb = p.vcb + (int64_t)bh * p.NKVp * ICSA_D;
+  // Steps: the listed blocks in list order (out-of-range entries are zero blocks without a
+  // gradient: skipped), then chunk ch as block -1 - ch.  Looked up one step ahead.
+  const int* row = p.idx + ((int64_t)bh * p.NQ + qb) * p.top_k;
+  const unsigned long long* selw = p.selbits + ((int64_t)bh * p.NQ + qb) * p.nc;
+  int at = 0;
+  auto next = [&]() -> int {
+    while (at < p.top_k) {
+      const int j = uniform_word(row + at++);
+      if (j >= 0 && j < p.NKV) return j;
     }
-    if (lane == 0) *n_ex_l = cnt;
-  }
+    return p.top_k - 1 - at++;                         // -1 - chunk
+  };
+  const int done = -1 - p.nc;
+  // real key rows of an exact step (the last block of a ragged TKV is partial)
+  auto key_rows = [&](int j) -> int { return j < 0 ? ICSA_BLOCK : min(ICSA_BLOCK, p.TKV - j * ICSA_BLOCK); };
+  // buffer u: K rows at 2 u tiles, V rows at 2 u + 1
+  auto issue = [&](int t, int j) {
+    unsigned char* kt = smem_q + (t & 1) * 2 * K_TILE_BYTES;
+    if (j >= 0) {
+      const int valid = key_rows(j);
+      bw_dma_rows(kt, kb + (int64_t)j * ICSA_BLOCK * p.k_st, p.k_st, wave, lane, valid);
+      bw_dma_rows(kt + K_TILE_BYTES, vb + (int64_t)j * ICSA_BLOCK * p.v_st, p.v_st, wave, lane, valid);
+    } else {
+      const int ch = -1 - j;
+      bw_dma_rows(kt, kcb + (int64_t)ch * ICSA_BLOCK * ICSA_D, ICSA_D, wave, lane);
+      bw_dma_rows(kt + K_TILE_BYTES, vcb + (int64_t)ch * ICSA_BLOCK * ICSA_D, ICSA_D, wave, lane);
+    }
+  };
+  int j = next();                                      // at least one chunk
+  issue(0, j);
   const int q_valid = max(0, min(32, p.TQ - qtok0));  // this wave's real query rows
   bf16x8 qf[8], dof[8];
   load_q_frags(qf, p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)qtok0 * p.q_st, p.q_st, q_valid);
@@ -210,86 +313,61 @@ __global__ void __launch_bounds__(BW_THREADS) icsa_sparse_bwd_dq_kernel(SparseBw
   const float dd = p.dvec[(int64_t)bh * p.NQ * ICSA_BLOCK + qtok0 + li];
   int tro[4];
   rt_tr_offsets<false>(tro, lane);
-  __syncthreads();
-  const int n_ex = *n_ex_l;
-  const int T = n_ex + p.nc;
-
-  const bf16* kb = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh;
-  const bf16* vb = p.v + (int64_t)b * p.v_sb + (int64_t)h * p.v_sh;
-  const bf16* kcb = p.kcb + (int64_t)bh * p.NKVp * ICSA_D;
-  const bf16* vcb = p.vcb + (int64_t)bh * p.NKVp * ICSA_D;
-  // real key rows of exact step t (the last block of a ragged TKV is partial)
-  auto key_rows = [&](int t) -> int {
-    return min(ICSA_BLOCK, p.TKV - __builtin_amdgcn_readfirstlane(src_l[t]) * ICSA_BLOCK);
-  };
-  // buffer u: K rows at 2 u tiles, V rows at 2 u + 1
-  auto issue = [&](int t) {
-    unsigned char* kt = smem_q + (t & 1) * 2 * K_TILE_BYTES;
-    if (t < n_ex) {
-      const int j = __builtin_amdgcn_readfirstlane(src_l[t]);
-      const int valid = key_rows(t);
-      bw_dma_rows(kt, kb + (int64_t)j * ICSA_BLOCK * p.k_st, p.k_st, wave, lane, valid);
-      bw_dma_rows(kt + K_TILE_BYTES, vb + (int64_t)j * ICSA_BLOCK * p.v_st, p.v_st, wave, lane, valid);
-    } else {
-      const int ch = t - n_ex;
-      bw_dma_rows(kt, kcb + (int64_t)ch * ICSA_BLOCK * ICSA_D, ICSA_D, wave, lane);
-      bw_dma_rows(kt + K_TILE_BYTES, vcb + (int64_t)ch * ICSA_BLOCK * ICSA_D, ICSA_D, wave, lane);
-    }
-  };
+  const int ro = bw_row_off(32 * kh + li, hl);
 
   floatx16 dq[4] = {};
-  floatx16 s[2], dp[2];
-  bf16x8 dsf[4];
+  floatx16 s, dp;
+  bf16x8 dsf[2];
   const float c64 = p.scale_log2 * (1.0f / 64.0f);
-  issue(0);                                            // T >= nc >= 1
-  for (int t = 0; t < T; ++t) {
-    const int kvalid = t < n_ex ? key_rows(t) : ICSA_BLOCK;
+  for (int t = 0; j != done; ++t) {
+    const int kvalid = key_rows(j), jn = next();
     BW_WAIT(0);                                        // step t's tiles, the only loads in flight
     if (kvalid < ICSA_BLOCK) {                         // zero key / value rows past TKV
       bw_fill_rows(smem_q + (t & 1) * 2 * K_TILE_BYTES, kvalid, wave, lane);
       bw_fill_rows(smem_q + (t & 1) * 2 * K_TILE_BYTES + K_TILE_BYTES, kvalid, wave, lane);
     }
-    ATT_BARRIER();                                     // step t complete; step t - 1's buffer read by both waves
-    if (t + 1 < T) issue(t + 1);                       // into that buffer
+    ATT_BARRIER();                                     // step t complete; step t - 1's buffer read by all waves
+    if (jn != done) issue(t + 1, jn);                  // into that buffer
     const unsigned char* ks = smem_q + (t & 1) * 2 * K_TILE_BYTES;
-    qk_tile_bw(s, reinterpret_cast<const bf16*>(ks), qf);                  // S^T[key][query]
-    qk_tile_bw(dp, reinterpret_cast<const bf16*>(ks + K_TILE_BYTES), dof); // dP^T
-    if (t < n_ex) {
-      const int thr = mask_threshold(kvalid, lane);
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const bool masked = acc_row_const(sub, e) >= thr;           // keys past TKV
-          const float pr = masked ? 0.f : __builtin_amdgcn_exp2f(fmaf(s[sub][e], p.scale_log2, -lse));
-          dsf[2 * sub + (e >> 3)][e & 7] = (bf16)(pr * (dp[sub][e] - dd));
-        }
+    bw_scores(s, dp, ks, ks + K_TILE_BYTES, ro, qf, dof);              // S^T[key][query], dP^T
+    // masked keys (past TKV; a chunk's selected blocks and blocks >= NKV) as one word: element
+    // e is bit 8 (e / 4) + e % 4 of the word's bits from 4 hl + 32 kh on
+    unsigned long long mb;
+    float c, dmul, dsmul;
+    if (j >= 0) {
+      mb = kvalid < ICSA_BLOCK ? ~0ull << kvalid : 0ull;
+      c = p.scale_log2; dmul = 1.f; dsmul = 1.f;
     } else {                                           // unselected block sums: score / 64, dS / 64
-      const int ch = t - n_ex;
-      // masked blocks of the chunk (selected, or >= NKV) as one word; element e of sub-tile
-      // sub is bit 8 (e / 4) + e % 4 of word sub of that word >> 4 hl
-      unsigned long long mb = sel_l[ch];
+      const int ch = -1 - j;
+      mb = uniform_word(selw + ch);
       const int n_real = p.NKV - ch * ICSA_BLOCK;
       if (n_real < ICSA_BLOCK) mb |= ~0ull << n_real;
-      const unsigned long long ml = mb >> (4 * (lane >> 5));
-      const unsigned wd[2] = {(unsigned)ml, (unsigned)(ml >> 32)};
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const bool masked = (wd[sub] >> (8 * (e >> 2) + (e & 3))) & 1u;
-          const float pr = masked ? 0.f : __builtin_amdgcn_exp2f(fmaf(s[sub][e], c64, -lse));
-          dsf[2 * sub + (e >> 3)][e & 7] = (bf16)(pr * (dp[sub][e] - 64.0f * dd) * (1.0f / 64.0f));
-        }
+      c = c64; dmul = 64.f; dsmul = 1.0f / 64.0f;
     }
-    pv_tile_tr<BW_PF, false>(dq, ks, tro, dsf);                      // dQ^T += K^T dS^T
+    if (mb == 0ull && j >= 0) {                      // the common case: a whole exact block
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        dsf[e >> 3][e & 7] = (bf16)(__builtin_amdgcn_exp2f(fmaf(s[e], c, -lse)) * (dp[e] - dd));
+    } else {
+      const unsigned wd = (unsigned)(mb >> (4 * hl + 32 * kh));
+      const float ddm = dmul * dd;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const unsigned keep = ~(unsigned)((int)(wd << (31 - 8 * (e >> 2) - (e & 3))) >> 31);
+        const float x = __builtin_amdgcn_exp2f(fmaf(s[e], c, -lse));
+        const float pr = __uint_as_float(__float_as_uint(x) & keep);
+        dsf[e >> 3][e & 7] = (bf16)(pr * (dp[e] - ddm) * dsmul);
+      }
+    }
+    bw_accum<4, 2>(dq, ks, tro[0], 2 * kh, dsf);          // dQ^T += K^T dS^T
+    j = jn;
   }
 
-  // ---- epilogue: dq = scale * acc ----
+  // ---- epilogue: dq = scale * (sum over both key halves) ----
   __syncthreads();
-  float* o_lds = reinterpret_cast<float*>(smem_q + wave * BW_STAGE_BYTES);
-  stage_o(o_lds, dq, p.scale);
-  __syncthreads();
+  float* o_lds = reinterpret_cast<float*>(smem_q + qh * BW_STAGE_BYTES);
+  bw_reduce_stage(o_lds, dq, kh, p.scale);
+  if (kh == 1) return;
   AlphaView none;
   none.p = nullptr; none.scalar = 0.f; none.sb = none.ss = none.sh = none.sd = 0; none.dtype = ICSA_DT_F32;
   store_rows(o_lds, p.dq, b, h, qtok0, q_valid, nullptr, none);
@@ -298,22 +376,25 @@ __global__ void __launch_bounds__(BW_THREADS) icsa_sparse_bwd_dq_kernel(SparseBw
 // ------------------------------------------------------------------------------------------
 // dk / dv: kInterval = true -> interval partials per (chunk, query range);
 //          kInterval = false -> exact part per key block + the summed partials.
-// Per visited query block: its Q and dO rows plus lse (wave 0) / D (wave 1), 17 DMA per
-// wave, land in one of two buffers while the previous block's S = Q K^T, dP = dO V^T,
-// dV^T += dO^T P and dK^T += Q^T dS run (Q^T, dO^T read transposed from the rows).
+// Per visited query block: its Q and dO rows plus lse (wave 0) / D (wave 1) land in one of two
+// buffers while the previous block's S = Q K^T, dP = dO V^T, dV^T += dO^T P and
+// dK^T += Q^T dS run (Q^T, dO^T read transposed from the rows).  Wave w: keys
+// 32 (w % 2) .. + 31 in registers, rows 32 (w / 2) .. + 31 of each query block.  dK sums the
+// wave's own rows over all 128 dims (the two row halves are added at the end); dV takes all
+// 64 rows for dims 64 (w / 2) .. + 63, with the other half's P read from LDS: keeping both
+// over all dims would need more than 256 registers.
 // ------------------------------------------------------------------------------------------
 #define BWKV_BUF_BYTES (2 * K_TILE_BYTES + 2 * 64 * 4)      // Q rows, dO rows, lse, D
-#define BWKV_LIST_BYTES 8192                 // exact: u16 query list; interval: u64 selection words
-#define BWKV_LDS_BYTES (2 * BWKV_BUF_BYTES + 2 * ICSA_D * 4 + BWKV_LIST_BYTES + 16)
+#define BWKV_P_BYTES (4 * 2 * 1024)                         // each wave's P: two 16-row operands
+#define BWKV_LDS_BYTES (2 * BWKV_BUF_BYTES + BWKV_P_BYTES + 2 * ICSA_D * 4)
+#define BWKV_SUM_AHEAD 16                                   // interval partials requested together
 
 template <bool kInterval>
-__global__ void __launch_bounds__(BW_THREADS) icsa_sparse_bwd_dkv_kernel(SparseBwdParams p) {
+__global__ void __launch_bounds__(BW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+icsa_sparse_bwd_dkv_kernel(SparseBwdParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_dyn[];
-  float* ivec = reinterpret_cast<float*>(smem_dyn + 2 * BWKV_BUF_BYTES);   // [2][128] interval sums
-  unsigned char* list = reinterpret_cast<unsigned char*>(ivec + 2 * ICSA_D);
-  unsigned short* qlist = reinterpret_cast<unsigned short*>(list);
-  unsigned long long* wlist = reinterpret_cast<unsigned long long*>(list);
-  int* qcount = reinterpret_cast<int*>(list + BWKV_LIST_BYTES);
+  unsigned char* pbuf = smem_dyn + 2 * BWKV_BUF_BYTES;
+  float* ivec = reinterpret_cast<float*>(pbuf + BWKV_P_BYTES);    // [2][128] interval sums
 
   const int n_work = kInterval ? p.B * p.H * p.nc * p.nsplit : p.B * p.H * p.NKV;
   const int work = xcd_remap(blockIdx.x, n_work);
@@ -322,8 +403,8 @@ __global__ void __launch_bounds__(BW_THREADS) icsa_sparse_bwd_dkv_kernel(SparseB
   if (kInterval) {
     bh = work / (p.nc * p.nsplit);
     const int rem = work % (p.nc * p.nsplit);
-    blk = rem / p.nsplit;                              // chunk of 64 compressed blocks
-    split = rem % p.nsplit;
+    split = rem / p.nc;                                // neighbours read the same query blocks
+    blk = rem % p.nc;                                  // chunk of 64 compressed blocks
   } else {
     bh = work / p.NKV;
     blk = work % p.NKV;                                // key block
@@ -331,9 +412,66 @@ __global__ void __launch_bounds__(BW_THREADS) icsa_sparse_bwd_dkv_kernel(SparseB
   const int b = bh / p.H, h = bh % p.H;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int li = lane & 31;
-  const int key0 = blk * ICSA_BLOCK + 32 * wave;       // this wave's first key (or compressed block)
+  const int li = lane & 31, hl = lane >> 5;
+  const int kh = wave & 1, rh = wave >> 1;
+  const int key0 = blk * ICSA_BLOCK + 32 * kh;         // this wave's first key (or compressed block)
 
+  int tro[4];
+  rt_tr_offsets<false>(tro, lane);
+  const int ro = bw_row_off(32 * rh + li, hl);
+
+  const int ckey = key0 + li;                          // interval: this lane's compressed block
+  const float cexp = kInterval ? p.scale_log2 * (1.0f / 64.0f) : p.scale_log2;
+  const float dmul = kInterval ? 64.0f : 1.0f;
+
+  const bf16* qb0 = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
+  const bf16* dob0 = p.dout + (int64_t)b * p.do_sb + (int64_t)h * p.do_sh;
+  const float* rowvec = wave == 0 ? p.lse + (int64_t)bh * p.TQ : p.dvec + (int64_t)bh * p.NQ * ICSA_BLOCK;
+  // Query blocks to visit, ascending, looked up one ahead: the interval's range (with the
+  // chunk's selection word of each), or the set bits of the key block's row of the bitmap.
+  const int i_end = kInterval ? min(p.NQ, (split + 1) * p.qb_per_split) : p.NQ;
+  const int n_qw = (p.NQ + 63) / 64;
+  const unsigned long long* bits = kInterval ? p.selbits + (int64_t)bh * p.NQ * p.nc + blk
+                                             : p.seltr + ((int64_t)bh * p.NKV + blk) * n_qw;
+  int at = kInterval ? split * p.qb_per_split : 0;     // next query block / current word
+  unsigned long long cur = kInterval ? 0ull : uniform_word(bits);
+  auto next = [&]() -> int {
+    if (kInterval) {
+      if (at >= i_end) return -1;
+      cur = uniform_word(bits + (int64_t)at * p.nc);
+      return at++;
+    }
+    while (cur == 0ull) {
+      if (++at >= n_qw) return -1;
+      cur = uniform_word(bits + at);
+    }
+    const int i = 64 * at + __builtin_ctzll(cur);
+    cur &= cur - 1ull;
+    return i;
+  };
+  auto issue = [&](int n, int i) {
+    const int valid = min(ICSA_BLOCK, p.TQ - i * ICSA_BLOCK);   // ragged TQ: partial last block
+    unsigned char* buf = smem_dyn + (n & 1) * BWKV_BUF_BYTES;
+    bw_dma_rows(buf, qb0 + (int64_t)i * ICSA_BLOCK * p.q_st, p.q_st, wave, lane, valid);
+    bw_dma_rows(buf + K_TILE_BYTES, dob0 + (int64_t)i * ICSA_BLOCK * p.do_st, p.do_st, wave, lane, valid);
+    if (wave < 2)
+      lds_dma4(lds_u32(buf + 2 * K_TILE_BYTES + wave * 256), lane * 4,
+               dma_rsrc(rowvec + (int64_t)i * ICSA_BLOCK, valid * 4));
+  };
+  // Everything the prologue reads is requested before any of it is waited for: the first
+  // tiles, the interval partials (exact part), K and V.
+  int i = next();
+  unsigned long long sel = cur;                        // interval: block i's word
+  if (i >= 0) issue(0, i);
+  float px[BWKV_SUM_AHEAD];
+  const float* part = kInterval ? nullptr : (tid < ICSA_D ? p.dkc_part : p.dvc_part) +
+                                                ((int64_t)bh * p.NKVp + blk) * ICSA_D + (tid & 127);
+  const int64_t part_st = (int64_t)p.B * p.H * p.NKVp * ICSA_D;
+  auto load_parts = [&](int sp0) {
+#pragma unroll
+    for (int u = 0; u < BWKV_SUM_AHEAD; ++u) px[u] = part[min(sp0 + u, p.nsplit - 1) * part_st];
+  };
+  if (!kInterval) load_parts(0);
   bf16x8 kf[8], vf[8];
   if (kInterval) {
     load_q_frags(kf, p.kcb + ((int64_t)bh * p.NKVp + key0) * ICSA_D, ICSA_D, 32);
@@ -343,176 +481,90 @@ __global__ void __launch_bounds__(BW_THREADS) icsa_sparse_bwd_dkv_kernel(SparseB
     load_q_frags(kf, p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh + (int64_t)key0 * p.k_st, p.k_st, kv);
     load_q_frags(vf, p.v + (int64_t)b * p.v_sb + (int64_t)h * p.v_sh + (int64_t)key0 * p.v_st, p.v_st, kv);
   }
-  int tro[4];
-  rt_tr_offsets<false>(tro, lane);
-
-  // query blocks to visit, ascending
-  int i_begin = 0, i_count;
-  if (kInterval) {
-    i_begin = split * p.qb_per_split;
-    i_count = max(0, min(p.NQ, i_begin + p.qb_per_split) - i_begin);
-    for (int u = tid; u < i_count; u += BW_THREADS)
-      wlist[u] = p.selbits[((int64_t)bh * p.NQ + i_begin + u) * p.nc + blk];
-    __syncthreads();
-  } else {
-    if (wave == 0) {
-      const int w = blk >> 6;
-      const unsigned long long bit = 1ull << (blk & 63);
-      int cnt = 0;
-      for (int base = 0; base < p.NQ; base += 64) {
-        const int i = base + lane;
-        const bool on = i < p.NQ && (p.selbits[((int64_t)bh * p.NQ + i) * p.nc + w] & bit) != 0ull;
-        const unsigned long long bal = __ballot(on);
-        if (on) qlist[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = (unsigned short)i;
-        cnt += __popcll(bal);
-      }
-      if (lane == 0) *qcount = cnt;
+  if (!kInterval) {                                    // interval sums of the block, in split order
+    float sum = 0.f;
+    for (int sp0 = 0;;) {
+#pragma unroll
+      for (int u = 0; u < BWKV_SUM_AHEAD; ++u)
+        if (sp0 + u < p.nsplit) sum += px[u];
+      sp0 += BWKV_SUM_AHEAD;
+      if (sp0 >= p.nsplit) break;
+      load_parts(sp0);
     }
-    __syncthreads();
-    i_count = *qcount;
+    ivec[tid] = tid < ICSA_D ? sum * p.scale : sum;
   }
 
-  const int ckey = key0 + li;                          // this lane's key (interval: compressed block)
-  const bool key_valid = ckey < (kInterval ? p.NKV : p.TKV);
-  const float cexp = kInterval ? p.scale_log2 * (1.0f / 64.0f) : p.scale_log2;
-  const float dmul = kInterval ? 64.0f : 1.0f;
-  const float dsmul = kInterval ? (1.0f / 64.0f) : 1.0f;
+  floatx16 dk[4] = {}, dv[2] = {};
+  floatx16 s, dp;
+  bf16x8 pf[4], dsf[2];
 
-  const bf16* qb0 = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh;
-  const bf16* dob0 = p.dout + (int64_t)b * p.do_sb + (int64_t)h * p.do_sh;
-  const float* rowvec = wave == 0 ? p.lse + (int64_t)bh * p.TQ : p.dvec + (int64_t)bh * p.NQ * ICSA_BLOCK;
-  auto qblock = [&](int n) -> int {
-    return kInterval ? i_begin + n : __builtin_amdgcn_readfirstlane((int)qlist[n]);
-  };
-  // real query rows of block qblock(n) (the last block of a ragged TQ is partial)
-  auto q_rows = [&](int n) -> int { return min(ICSA_BLOCK, p.TQ - qblock(n) * ICSA_BLOCK); };
-  auto issue = [&](int n) {
-    const int i = qblock(n), valid = q_rows(n);
+  for (int n = 0; i >= 0; ++n) {
+    // exact: a key past TKV (zero K and V rows) only reaches its own dk / dv row, not stored
+    const bool on = !kInterval || (ckey < p.NKV && ((sel >> (32 * kh + li)) & 1ull) == 0ull);
+    const int in = next();
     unsigned char* buf = smem_dyn + (n & 1) * BWKV_BUF_BYTES;
-    bw_dma_rows(buf, qb0 + (int64_t)i * ICSA_BLOCK * p.q_st, p.q_st, wave, lane, valid);
-    bw_dma_rows(buf + K_TILE_BYTES, dob0 + (int64_t)i * ICSA_BLOCK * p.do_st, p.do_st, wave, lane, valid);
-    const __amdgpu_buffer_rsrc_t rr = make_rsrc(rowvec + (int64_t)i * ICSA_BLOCK, valid * 4);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rr, (lds_ptr)(buf + 2 * K_TILE_BYTES + wave * 256), 4,
-                                             lane * 4, 0, 0, 0);
-  };
-
-  floatx16 dk[4] = {}, dv[4] = {};
-  floatx16 s[2], dp[2];
-  bf16x8 pf[4], dsf[4];
-  if (i_count > 0) issue(0);
-  for (int n = 0; n < i_count; ++n) {
-    bool on = key_valid;
-    if (kInterval) on = on && ((wlist[n] >> (32 * wave + li)) & 1ull) == 0ull;
-    BW_WAIT(0);                                        // block n's tiles, the only loads in flight
-    const int qvalid = q_rows(n);
-    if (qvalid < ICSA_BLOCK) {                         // zero Q / dO rows and lse / D past TQ
-      unsigned char* buf = smem_dyn + (n & 1) * BWKV_BUF_BYTES;
+    BW_WAIT(0);                                      // block n's tiles, the only loads in flight
+    const int qvalid = min(ICSA_BLOCK, p.TQ - i * ICSA_BLOCK);
+    if (qvalid < ICSA_BLOCK) {                       // zero Q / dO rows and lse / D past TQ
       bw_fill_rows(buf, qvalid, wave, lane);
       bw_fill_rows(buf + K_TILE_BYTES, qvalid, wave, lane);
-      if (lane >= qvalid) reinterpret_cast<float*>(buf + 2 * K_TILE_BYTES + wave * 256)[lane] = 0.f;
+      if (wave < 2 && lane >= qvalid) reinterpret_cast<float*>(buf + 2 * K_TILE_BYTES + wave * 256)[lane] = 0.f;
     }
-    ATT_BARRIER();                                     // block n complete; block n - 1's buffer read by both waves
-    if (n + 1 < i_count) issue(n + 1);                 // into that buffer
-    const unsigned char* qs = smem_dyn + (n & 1) * BWKV_BUF_BYTES;
-    const unsigned char* dos = qs + K_TILE_BYTES;
-    const float* lse_l = reinterpret_cast<const float*>(qs + 2 * K_TILE_BYTES);
-    const float* dd_l = lse_l + 64;
-    // One stream of 64 MFMAs, operands read BW_PF steps ahead, with the elementwise work
-    // slotted between MFMAs that do not depend on it (one wave per SIMD: nothing else
-    // fills the matrix pipe while this wave runs VALU code):
-    //   t  0..15  S and dP of query rows 0-31   (t even: S = Q K^T, odd: dP = dO V^T; kk = t / 2 % 8)
-    //   t 16..31  S and dP of rows 32-63        + P, dS of rows 0-31 (one element per MFMA)
-    //   t 32..63  u = t - 32: m = u / 8, ds = u / 2 % 4; u even: dV^T += dO^T P, odd:
-    //             dK^T += Q^T dS                + P, dS of rows 32-63 during u < 16
-    const bf16* qsb = reinterpret_cast<const bf16*>(qs);
-    const bf16* dosb = reinterpret_cast<const bf16*>(dos);
-    const int hl = lane >> 5;
-    auto ld = [&](int t) -> bf16x8 {
-      if (t < 32) {
-        const int sub = t >> 4, kk = (t & 15) >> 1;
-        return *reinterpret_cast<const bf16x8*>(((t & 1) ? dosb : qsb) + rt_off(32 * sub + li, 2 * kk + hl));
-      }
-      const int u = t - 32, m = u >> 3, ds = (u >> 1) & 3;
-      const unsigned char* tile = (u & 1) ? qs : dos;
-      const rt_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((rt_lds_v4s)(tile + tro[ds] + m * 16 * ICSA_D * 2));
-      const rt_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((rt_lds_v4s)(tile + rt_tr_hi<false>(tro[ds]) + m * 16 * ICSA_D * 2));
-      const short __attribute__((ext_vector_type(8))) a8 = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      return __builtin_bit_cast(bf16x8, a8);
-    };
-    floatx4 l4[2][4], d4[2][4];                        // lse / D of the rows each lane holds
-    auto ld_rows = [&](int sub) {
+    ATT_BARRIER();                                   // block n complete; block n - 1's buffer and P read by all
+    if (in >= 0) issue(n + 1, in);                   // into that buffer
+    const unsigned char* dos = buf + K_TILE_BYTES;
+    bw_scores(s, dp, buf, dos, ro, kf, vf);          // S[row][key], dP
+    const float* lse_l = reinterpret_cast<const float*>(buf + 2 * K_TILE_BYTES) + 32 * rh + 4 * hl;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int r0 = 32 * sub + 8 * g + 4 * (lane >> 5);  // acc_row(4 g + x, lane) = r0 + x
-        l4[sub][g] = *reinterpret_cast<const floatx4*>(lse_l + r0);
-        d4[sub][g] = *reinterpret_cast<const floatx4*>(dd_l + r0);
-      }
-    };
-    auto elem = [&](int sub, int e) {
-      const float pr = on ? __builtin_amdgcn_exp2f(fmaf(s[sub][e], cexp, -l4[sub][e >> 2][e & 3])) : 0.f;
-      pf[2 * sub + (e >> 3)][e & 7] = (bf16)pr;
-      dsf[2 * sub + (e >> 3)][e & 7] = (bf16)(pr * (dp[sub][e] - dmul * d4[sub][e >> 2][e & 3]) * dsmul);
-    };
-    bf16x8 a[64];
-    ld_rows(0);
+    for (int g = 0; g < 4; ++g) {                    // acc_row(4 g + x, lane) = 8 g + 4 hl + x
+      const floatx4 l4 = *reinterpret_cast<const floatx4*>(lse_l + 8 * g);
+      const floatx4 d4 = *reinterpret_cast<const floatx4*>(lse_l + 64 + 8 * g);
 #pragma unroll
-    for (int t = 0; t < BW_PF; ++t) a[t] = ld(t);
-    s[0] = s[1] = dp[0] = dp[1] = floatx16{};
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int t = 0; t < 64; ++t) {
-      if (t + BW_PF < 64) a[t + BW_PF] = ld(t + BW_PF);
-      if (t < 32) {
-        const int sub = t >> 4, kk = (t & 15) >> 1;
-        if (t & 1) dp[sub] = mfma32x32x16(a[t], vf[kk], dp[sub]);
-        else s[sub] = mfma32x32x16(a[t], kf[kk], s[sub]);
-      } else {
-        const int u = t - 32, m = u >> 3, ds = (u >> 1) & 3;
-        if (u & 1) dk[ds] = mfma32x32x16(a[t], dsf[m], dk[ds]);
-        else dv[ds] = mfma32x32x16(a[t], pf[m], dv[ds]);
+      for (int x = 0; x < 4; ++x) {
+        const int e = 4 * g + x;
+        const float ex = __builtin_amdgcn_exp2f(fmaf(s[e], cexp, -l4[x]));
+        const float pr = !kInterval || on ? ex : 0.f;
+        pf[e >> 3][e & 7] = (bf16)pr;
+        dsf[e >> 3][e & 7] = (bf16)(pr * (dp[e] - dmul * d4[x]));
       }
-      if (t == 16) ld_rows(1);
-      if (t >= 16 && t < 32) elem(0, t - 16);
-      if (t >= 32 && t < 48) elem(1, t - 32);
-      __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+      *reinterpret_cast<bf16x8*>(pbuf + ((2 * wave + m) * 64 + lane) * 16) = pf[m];
+    bw_accum<4, 2>(dk, buf, tro[0], 2 * rh, dsf);       // dK^T += Q^T dS, own rows
+    ATT_BARRIER();                                   // P of both row halves in LDS
+    // P operands by 16-row step: own rows from registers, the other half's from LDS
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+      pf[2 + m] = *reinterpret_cast<const bf16x8*>(pbuf + ((2 * (wave ^ 2) + m) * 64 + lane) * 16);
+    bw_accum<2, 2>(dv, dos, tro[0] ^ (rh << 7), 2 * rh, pf);     // dV^T += dO^T P, dims 64 rh ..
+    bw_accum<2, 2>(dv, dos, tro[0] ^ (rh << 7), 2 * (rh ^ 1), pf + 2);
+    i = in;
+    sel = cur;
   }
 
   __syncthreads();
-  float* o_lds = reinterpret_cast<float*>(smem_dyn + wave * BW_STAGE_BYTES);
+  float* o_lds = reinterpret_cast<float*>(smem_dyn + kh * BW_STAGE_BYTES);
+  float* v_lds = reinterpret_cast<float*>(smem_dyn + (2 + kh) * BW_STAGE_BYTES);
   AlphaView one;
   one.p = nullptr; one.scalar = 1.f; one.sb = one.ss = one.sh = one.sd = 0; one.dtype = ICSA_DT_F32;
+  {
+    const int lr = lane & 31;
+#pragma unroll
+    for (int ds = 0; ds < 2; ++ds)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) v_lds[lr * O_LDS_STRIDE + 64 * rh + 32 * ds + acc_row(e, lane)] = dv[ds][e];
+  }
+  // dK: both row halves; the interval's dS lacked its 1 / 64 (partials: dk without the scale)
+  bw_reduce_stage(o_lds, dk, rh, kInterval ? 1.0f / 64.0f : p.scale);
+  const float* src = rh == 0 ? o_lds : v_lds;          // waves 0, 1 store dk, waves 2, 3 dv
   if (kInterval) {
-    // partials [split][bh][NKVp][D] (dk part without the scale; dS already carries 1/64)
     const int64_t base = (((int64_t)split * p.B * p.H + bh) * p.NKVp) * ICSA_D;
-    stage_o(o_lds, dk, 1.f);
-    __syncthreads();
-    store_rows(o_lds, OutView{p.dkc_part + base, 0, ICSA_D, 0, ICSA_DT_F32}, 0, 0, key0, 32, nullptr, one);
-    __syncthreads();
-    stage_o(o_lds, dv, 1.f);
-    __syncthreads();
-    store_rows(o_lds, OutView{p.dvc_part + base, 0, ICSA_D, 0, ICSA_DT_F32}, 0, 0, key0, 32, nullptr, one);
+    store_rows(src, OutView{(rh == 0 ? p.dkc_part : p.dvc_part) + base, 0, ICSA_D, 0, ICSA_DT_F32}, 0, 0, key0, 32,
+               nullptr, one);
   } else {
-    // interval contributions of this block, summed over the splits in order
-    {
-      const int d = tid;                               // 128 threads = 128 dims
-      float sk = 0.f, sv = 0.f;
-      for (int sp = 0; sp < p.nsplit; ++sp) {
-        const int64_t off = ((((int64_t)sp * p.B * p.H + bh) * p.NKVp) + blk) * ICSA_D + d;
-        sk += p.dkc_part[off];
-        sv += p.dvc_part[off];
-      }
-      ivec[d] = sk * p.scale;
-      ivec[ICSA_D + d] = sv;
-    }
     const int kv = max(0, min(32, p.TKV - key0));     // rows past TKV are not stored
-    stage_o(o_lds, dk, p.scale);
-    __syncthreads();
-    store_rows(o_lds, p.dk, b, h, key0, kv, ivec, one);
-    __syncthreads();
-    stage_o(o_lds, dv, 1.f);
-    __syncthreads();
-    store_rows(o_lds, p.dv, b, h, key0, kv, ivec + ICSA_D, one);
+    store_rows(src, rh == 0 ? p.dk : p.dv, b, h, key0, kv, ivec + rh * ICSA_D, one);
   }
 }
 
@@ -529,7 +581,7 @@ hipError_t launch_sparse_bwd(const SparseBwdParams& p, hipStream_t stream) {
   const int BH = p.B * p.H;
   if (BH == 0 || p.NQ == 0) return hipSuccess;
   if (p.top_k < 1 || p.top_k > BW_MAX_TOPK || p.NKV < 1 || p.nc > BW_MAX_CHUNKS ||
-      p.NKVp != p.nc * ICSA_BLOCK || p.NQ > BW_MAX_NQ || p.nsplit < 1 || p.qb_per_split > 1024 ||
+      p.NKVp != p.nc * ICSA_BLOCK || p.NQ > BW_MAX_NQ || p.nsplit < 1 ||
       (int64_t)p.nsplit * p.qb_per_split < p.NQ)
     return hipErrorInvalidValue;
   static std::atomic<unsigned> set_q{0u}, set_i{0u}, set_e{0u};
