@@ -820,7 +820,7 @@ struct BwLayout {
 // and every further range 0.015 steps per (head, chunk) for the f32 partials it writes and
 // the exact part reads (1 KB each way per block sum at the copy rate, a step being 1.8 us).
 // The cheapest count at 40 heads, 122 query blocks, 2 chunks: 6 ranges (one round of 480
-// workgroups, 71 us; 16 ranges: 92 us); at 4 heads, 32 query blocks: 32 (11 us; 4: 18 us).
+// workgroups, 61 us; 16 ranges: 92 us before the waits for K and V left the loop); at 4 heads, 32 query blocks: 32 (11 us; 4: 18 us).
 int bwd_splits(int64_t BHc, int NQ) {
   int best = 1;
   double cost = 1e30;

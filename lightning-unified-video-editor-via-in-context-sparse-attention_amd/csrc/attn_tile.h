@@ -162,6 +162,17 @@ __device__ __forceinline__ void load_q_frags(bf16x8 qf[8], const bf16* qrow0, in
   }
 }
 
+// Waits for loaded operands here.  In a loop whose tile DMA the compiler does not see, its own
+// wait at their first use would sit inside the loop and wait for the DMA in flight each time.
+__device__ __forceinline__ void settle_frags(bf16x8 f[8]) {
+  u32x4 x[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] = __builtin_bit_cast(u32x4, f[i]);
+  asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]));
+#pragma unroll
+  for (int i = 0; i < 8; ++i) f[i] = __builtin_bit_cast(bf16x8, x[i]);
+}
+
 // S^T for the 64 keys of an LDS K tile: s[ks] covers keys 32*ks .. 32*ks + 31.
 __device__ __forceinline__ void qk_tile(floatx16 s[2], const bf16* ks, const bf16x8 qf[8]) {
   const int lane = threadIdx.x & 63;

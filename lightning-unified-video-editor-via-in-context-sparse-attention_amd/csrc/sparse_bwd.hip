@@ -37,14 +37,15 @@
 // workgroups (at most 76 KB of LDS each) share a CU, so one wave's elementwise work and LDS
 // reads run beside another's MFMAs; with two waves per workgroup, 64 rows each and 308-412
 // registers, every SIMD held a single wave.  Measured at 40 heads, 7,800 tokens, 12 of 122
-// blocks, against that: dq 375 -> 300 us, dk / dv exact 500 -> 360 us, interval 90 -> 71 us
-// (4 heads, 2,048 tokens: 14.6 -> 11.7, 28 -> 21, 22 -> 11 us).  A step of the exact part then
+// blocks, against that: dq 375 -> 298 us, dk / dv exact 500 -> 355 us, interval 90 -> 61 us
+// (4 heads, 2,048 tokens: 14.6 -> 11.7, 28 -> 21, 22 -> 10 us).  A step of the exact part then
 // takes 3,700 cycles with two workgroups on the CU, 55 % of them MFMA; about a third of a
 // workgroup's time is its start (first tiles, K and V) and its end (sums of the halves,
 // output), which is what bounds it at 12 steps.  Copies: all tiles from L2 5 % faster, no
 // tiles at all 17 %; no elementwise masks: the same.
 // Waits: the tile DMA is inline assembly (lds_dma16); behind the builtin the compiler waited
-// for the next step's tiles (vmcnt(0)) before every step's transposing reads.
+// for the next step's tiles (vmcnt(0)) before every step's transposing reads; settle_frags keeps its
+// waits for the register operands out of the loop (interval 70 -> 61 us).
 #include "attn_tile.h"
 #include "icsa_kernels.h"
 
@@ -309,11 +310,15 @@ icsa_sparse_bwd_dq_kernel(SparseBwdParams p) {
   load_q_frags(qf, p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)qtok0 * p.q_st, p.q_st, q_valid);
   load_q_frags(dof, p.dout + (int64_t)b * p.do_sb + (int64_t)h * p.do_sh + (int64_t)qtok0 * p.do_st, p.do_st,
                q_valid);
-  const float lse = li < q_valid ? p.lse[(int64_t)bh * p.TQ + qtok0 + li] : 0.f;
-  const float dd = p.dvec[(int64_t)bh * p.NQ * ICSA_BLOCK + qtok0 + li];
+  float lse = li < q_valid ? p.lse[(int64_t)bh * p.TQ + qtok0 + li] : 0.f;
+  float dd = p.dvec[(int64_t)bh * p.NQ * ICSA_BLOCK + qtok0 + li];
   int tro[4];
   rt_tr_offsets<false>(tro, lane);
   const int ro = bw_row_off(32 * kh + li, hl);
+
+  settle_frags(qf);
+  settle_frags(dof);
+  asm volatile("" : "+v"(lse), "+v"(dd));
 
   floatx16 dq[4] = {};
   floatx16 s, dp;
@@ -493,6 +498,8 @@ icsa_sparse_bwd_dkv_kernel(SparseBwdParams p) {
     }
     ivec[tid] = tid < ICSA_D ? sum * p.scale : sum;
   }
+  settle_frags(kf);
+  settle_frags(vf);
 
   floatx16 dk[4] = {}, dv[2] = {};
   floatx16 s, dp;
