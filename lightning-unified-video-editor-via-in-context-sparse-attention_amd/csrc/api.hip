@@ -71,6 +71,17 @@ bool row_ok(const void* p, int dtype, int64_t s0, int64_t s1, int64_t s2) {
   return aligned16(p) && s0 % m == 0 && s1 % m == 0 && s2 % m == 0;
 }
 
+// q of Sq tokens, k / v of Sk tokens
+void pool_sizes(PoolParams& p, int B, int H, int Sq, int Sk) {
+  p.B = B;
+  p.H = H;
+  for (int i = 0; i < 3; ++i) {
+    p.S[i] = i == 0 ? Sq : Sk;
+    p.NB[i] = ceil_div(p.S[i], ICSA_BLOCK);
+    p.NBp[i] = ceil_div(p.NB[i], 64) * 64;
+  }
+}
+
 int check_dtype(int dt, const char* name) {
   if (dt != ICSA_BF16 && dt != ICSA_F32) return fail(ICSA_EINVAL, "%s: dtype %d is not bf16 (0) or f32 (1)", name, dt);
   return ICSA_OK;
@@ -271,7 +282,7 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
   // V^T holds the new KV's tiles only: the pooling pass transposes the target blocks (block
   // n at columns 64 n ..), the selected source blocks follow after the selection
   pp.vt_limit = 1; pp.vt_nblk = ceil_div(t_seq_len, ICSA_BLOCK);
-  pp.B = B; pp.S = S; pp.H = H; pp.NB = z.NB;
+  pool_sizes(pp, B, H, S, S);
   ICSA_HIP_TRY(mark(ICSA_STAGE_START), "event");
   ICSA_HIP_TRY(launch_pool(pp, stream), "pool");
   ICSA_HIP_TRY(mark(ICSA_STAGE_POOL), "event");
@@ -334,7 +345,7 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
   np.vc = unaligned ? reinterpret_cast<bf16*>(WS(ICSA_WS_VC)) : nullptr;
   np.BH = BH; np.NKV = z.NKV; np.NKVp = z.NKVp;
   np.ksum = ksum; np.vsum = pp.sums[2];
-  np.kvmap = sp.kvmap; np.map_identity = 0; np.Nsrc = z.NB;
+  np.kvmap = sp.kvmap; np.Nsrc = z.NB;
   np.k = TokTensor{k, k_sb, k_ss, k_sh, k_dtype};
   np.v = TokTensor{v, v_sb, v_ss, v_sh, v_dtype};
   np.seg_a = seg_a; np.seg_from = z.n_t; np.S = S; np.H = H;
@@ -625,7 +636,7 @@ int icsa_wan_qk_prologue(
 
 namespace {
 struct SpLayout {
-  int64_t qsum, ksum, vsum, kc32, kc, vc, idx, scores, total;
+  int64_t qsum, ksum, kc, vc, idx, scores, total;
 };
 // Sizes for TQ / TKV rounded up to whole blocks (the Triton host's ragged lengths); the
 // index buffer holds max(1, int(sparsity * NKV)) entries per query block, which is at
@@ -639,8 +650,6 @@ SpLayout sparse_layout(int B, int H, int TQ, int TKV, double sparsity) {
   int64_t o = 0;
   L.qsum = o; o += align256(BH * NQ * ICSA_D * 4);
   L.ksum = o; o += align256(BH * NKV * ICSA_D * 4);
-  L.vsum = o; o += align256(BH * NKV * ICSA_D * 4);
-  L.kc32 = o; o += align256(BH * NKV * ICSA_D * 4);
   L.kc = o; o += align256(BH * NKVp * ICSA_D * 2);
   L.vc = o; o += align256(BH * NKVp * ICSA_D * 2);
   L.idx = o; o += align256(BH * NQ * top_k * 4);
@@ -696,45 +705,30 @@ static int sparse_piecewise_impl(
   char* ws = reinterpret_cast<char*>(workspace);
   const int BH = B * H;
 
-  PoolParams pq;
-  std::memset(&pq, 0, sizeof(pq));
-  pq.x[0] = TokTensor{q, q_sb, q_st, q_sh, ICSA_BF16};
-  pq.sums[0] = reinterpret_cast<float*>(ws + L.qsum);
-  pq.B = B; pq.S = TQ; pq.H = H; pq.NB = NQ;
-  ICSA_HIP_TRY(launch_pool(pq, stream), "pool q");
-  PoolParams pk;
-  std::memset(&pk, 0, sizeof(pk));
-  pk.x[1] = TokTensor{k, k_sb, k_st, k_sh, ICSA_BF16};
-  pk.x[2] = TokTensor{v, v_sb, v_st, v_sh, ICSA_BF16};
-  pk.sums[1] = reinterpret_cast<float*>(ws + L.ksum);
-  pk.sums[2] = reinterpret_cast<float*>(ws + L.vsum);
-  pk.B = B; pk.S = TKV; pk.H = H; pk.NB = NKV;
-  ICSA_HIP_TRY(launch_pool(pk, stream), "pool k/v");
+  // one pass: the f32 sums of q and k (scores), the bf16 ones of k and v (KC / VC)
+  PoolParams pp;
+  std::memset(&pp, 0, sizeof(pp));
+  pp.x[0] = TokTensor{q, q_sb, q_st, q_sh, ICSA_BF16};
+  pp.x[1] = TokTensor{k, k_sb, k_st, k_sh, ICSA_BF16};
+  pp.x[2] = TokTensor{v, v_sb, v_st, v_sh, ICSA_BF16};
+  pp.sums[0] = reinterpret_cast<float*>(ws + L.qsum);
+  pp.sums[1] = reinterpret_cast<float*>(ws + L.ksum);
+  pp.sb[1] = reinterpret_cast<bf16*>(ws + L.kc);
+  pp.sb[2] = reinterpret_cast<bf16*>(ws + L.vc);
+  pool_sizes(pp, B, H, TQ, TKV);
+  ICSA_HIP_TRY(launch_pool(pp, stream), "pool");
 
-  NewKvSumsParams np;
-  std::memset(&np, 0, sizeof(np));  // seg_a = 0: no straddling blocks
-  np.ksum = pk.sums[1]; np.vsum = pk.sums[2]; np.kvmap = nullptr; np.map_identity = 1;
-  np.kc32 = reinterpret_cast<float*>(ws + L.kc32);
-  np.kc = reinterpret_cast<bf16*>(ws + L.kc);
-  np.vct = nullptr;
-  np.vc = reinterpret_cast<bf16*>(ws + L.vc);
-  np.BH = BH; np.Nsrc = NKV; np.NKV = NKV; np.NKVp = NKVp;
-  ICSA_HIP_TRY(launch_newkv_sums(np, stream), "block sums");
-
-  int32_t* idx = reinterpret_cast<int32_t*>(ws + L.idx);
+  int32_t* idx = idx_out ? idx_out : reinterpret_cast<int32_t*>(ws + L.idx);
   if (inject_idx) {
     ICSA_HIP_TRY(hipMemcpyAsync(idx, inject_idx, (size_t)BH * NQ * top_k * 4, hipMemcpyDeviceToDevice,
                                 stream), "inject idx");
   } else {
     Level3Params lp;
-    lp.qsum = pq.sums[0]; lp.rows = nullptr; lp.rows_offset = 0; lp.rows_stride = 0;
-    lp.kc32 = np.kc32; lp.idx = idx; lp.scores = reinterpret_cast<float*>(ws + L.scores);
+    lp.qsum = pp.sums[0]; lp.rows = nullptr; lp.rows_offset = 0; lp.rows_stride = 0;
+    lp.kc32 = pp.sums[1]; lp.idx = idx; lp.scores = reinterpret_cast<float*>(ws + L.scores);
     lp.BH = BH; lp.NQsrc = NQ; lp.n_rows = NQ; lp.NKV = NKV; lp.top_k = top_k;
     ICSA_HIP_TRY(launch_level3(lp, stream), "block top-k");
   }
-  if (idx_out)
-    ICSA_HIP_TRY(hipMemcpyAsync(idx_out, idx, (size_t)BH * NQ * top_k * 4, hipMemcpyDeviceToDevice, stream),
-                 "copy idx");
 
   SparseParams s;
   std::memset(&s, 0, sizeof(s));   // seg_a = 0: the caller's new KV is contiguous
@@ -747,7 +741,7 @@ static int sparse_piecewise_impl(
   s.qblocks = nullptr; s.qb_offset = 0; s.qb_stride = 0; s.n_qblk = NQ;
   s.kvmap = nullptr; s.kvmap_identity = 1;
   s.idx = idx; s.top_k = top_k; s.NKV = NKV; s.NKVp = NKVp;
-  s.kc = np.kc; s.vct = nullptr; s.vc = np.vc;
+  s.kc = pp.sb[1]; s.vct = nullptr; s.vc = pp.sb[2];
   s.out_c = nullptr; s.nb_q = NQ;
   s.alpha = make_alpha(nullptr, ICSA_F32, 0, 0, 0, 0, 0.f);
   s.out = OutView{out, o_sb, o_st, o_sh, ICSA_BF16};
@@ -759,7 +753,7 @@ static int sparse_piecewise_impl(
   // |KC_j| bound of the interval pass
   if (interval_skip_enabled()) {
     s.kc_bound = reinterpret_cast<float*>(ws + L.scores);
-    ICSA_HIP_TRY(launch_kc_bound(np.kc, BH, NKV, NKVp, reinterpret_cast<float*>(ws + L.scores),
+    ICSA_HIP_TRY(launch_kc_bound(pp.sb[1], BH, NKV, NKVp, reinterpret_cast<float*>(ws + L.scores),
                                  &s.kc_bound_n, stream), "interval bound");
   }
   ICSA_HIP_TRY(launch_sparse(s, stream), "sparse attention");
@@ -812,7 +806,7 @@ int icsa_sparse_piecewise_attn_fwd(
 
 namespace {
 struct BwLayout {
-  int64_t ksum, vsum, dvec, selbits, seltr, kcb, vcb, dkc, dvc, total;
+  int64_t dvec, selbits, seltr, kcb, vcb, dkc, dvc, total;
   int nsplit, qb_per_split;
 };
 // Interval partials: the query blocks are cut in nsplit ranges, one workgroup per (chunk,
@@ -844,8 +838,6 @@ BwLayout bwd_layout(int B, int H, int TQ, int TKV) {
   L.qb_per_split = qbps;
   L.nsplit = ceil_div(NQ, qbps);
   int64_t o = 0;
-  L.ksum = o; o += align256(BH * NKV * ICSA_D * 4);
-  L.vsum = o; o += align256(BH * NKV * ICSA_D * 4);
   L.dvec = o; o += align256(BH * (int64_t)NQ * ICSA_BLOCK * 4);   // D rows padded to whole blocks
   L.selbits = o; o += align256(BH * NQ * (int64_t)nc * 8);
   L.seltr = o; o += align256(BH * NKV * (int64_t)ceil_div(NQ, 64) * 8);
@@ -902,13 +894,13 @@ int icsa_sparse_piecewise_attn_bwd(
   char* ws = reinterpret_cast<char*>(workspace);
   const int nc = ceil_div(NKV, 64);
 
-  PoolParams pk;                                   // f32 block sums of k / v (the forward's)
+  PoolParams pk;                                   // bf16 block sums of k / v (the forward's)
   std::memset(&pk, 0, sizeof(pk));
   pk.x[1] = TokTensor{k, k_sb, k_st, k_sh, ICSA_BF16};
   pk.x[2] = TokTensor{v, v_sb, v_st, v_sh, ICSA_BF16};
-  pk.sums[1] = reinterpret_cast<float*>(ws + L.ksum);
-  pk.sums[2] = reinterpret_cast<float*>(ws + L.vsum);
-  pk.B = B; pk.S = TKV; pk.H = H; pk.NB = NKV;
+  pk.sb[1] = reinterpret_cast<bf16*>(ws + L.kcb);
+  pk.sb[2] = reinterpret_cast<bf16*>(ws + L.vcb);
+  pool_sizes(pk, B, H, 0, TKV);
   ICSA_HIP_TRY(launch_pool(pk, stream), "pool k/v");
 
   SparseBwdParams p;
@@ -923,18 +915,16 @@ int icsa_sparse_piecewise_attn_bwd(
   p.top_k = top_k; p.nsplit = L.nsplit; p.qb_per_split = L.qb_per_split;
   p.scale = 1.0f / std::sqrt((float)ICSA_D);
   p.scale_log2 = kLog2e / std::sqrt((float)ICSA_D);
-  p.ksum = pk.sums[1]; p.vsum = pk.sums[2];
   p.dvec = reinterpret_cast<float*>(ws + L.dvec);
   p.selbits = reinterpret_cast<unsigned long long*>(ws + L.selbits);
   p.seltr = reinterpret_cast<unsigned long long*>(ws + L.seltr);
-  p.kcb = reinterpret_cast<bf16*>(ws + L.kcb);
-  p.vcb = reinterpret_cast<bf16*>(ws + L.vcb);
+  p.kcb = pk.sb[1];
+  p.vcb = pk.sb[2];
   p.dkc_part = reinterpret_cast<float*>(ws + L.dkc);
   p.dvc_part = reinterpret_cast<float*>(ws + L.dvc);
   p.dq = OutView{dq, dq_sb, dq_st, dq_sh, dq_dtype == ICSA_F32 ? ICSA_DT_F32 : ICSA_DT_BF16};
   p.dk = OutView{dk, dk_sb, dk_st, dk_sh, dk_dtype == ICSA_F32 ? ICSA_DT_F32 : ICSA_DT_BF16};
   p.dv = OutView{dv, dv_sb, dv_st, dv_sh, dv_dtype == ICSA_F32 ? ICSA_DT_F32 : ICSA_DT_BF16};
-  ICSA_HIP_TRY(launch_sparse_bwd_prep(p, stream), "backward prep");
   ICSA_HIP_TRY(launch_sparse_bwd(p, stream), "backward");
   return ICSA_OK;
 }
@@ -975,7 +965,7 @@ int icsa_flash_attn(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
   pv.vt = reinterpret_cast<bf16*>(workspace);
   pv.vt_sb = (int64_t)H * ICSA_D * Skp; pv.vt_sh = ICSA_D * Skp; pv.vt_sd = Skp;
   pv.vt_src = 2;
-  pv.B = B; pv.S = Sk; pv.H = H; pv.NB = NBk;
+  pool_sizes(pv, B, H, Sk, Sk);
   ICSA_HIP_TRY(launch_pool(pv, stream), "transpose v");
   FlashParams f;
   f.q = reinterpret_cast<const bf16*>(q); f.q_sb = q_sb; f.q_ss = q_ss; f.q_sh = q_sh;
@@ -1022,7 +1012,7 @@ int icsa_pool(const void* q, int q_dtype, int64_t q_sb, int64_t q_ss, int64_t q_
   pp.vt = reinterpret_cast<bf16*>(vt);
   pp.vt_sb = (int64_t)H * ICSA_D * Sp; pp.vt_sh = ICSA_D * Sp; pp.vt_sd = Sp;
   pp.vt_src = 2;
-  pp.B = B; pp.S = S; pp.H = H; pp.NB = NB;
+  pool_sizes(pp, B, H, S, S);
   ICSA_HIP_TRY(launch_pool(pp, reinterpret_cast<hipStream_t>(stream_)), "pool");
   return ICSA_OK;
 }

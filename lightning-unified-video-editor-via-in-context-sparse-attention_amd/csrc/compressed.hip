@@ -643,7 +643,7 @@ __global__ void __launch_bounds__(128) icsa_newkv_sums_kernel(NewKvSumsParams p)
   for (int i = 0; i < 16; ++i) {
     const int j = j0 + i;
     int src = -1;
-    if (j < p.NKV) src = p.map_identity ? j : p.kvmap[(int64_t)bh * p.NKV + j];
+    if (j < p.NKV) src = p.kvmap[(int64_t)bh * p.NKV + j];
     ks[i] = 0.f;
     vs[i] = 0.f;
     if (src >= 0) {

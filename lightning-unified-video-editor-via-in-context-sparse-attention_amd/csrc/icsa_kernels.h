@@ -7,14 +7,16 @@
 // ---------------------------------------------------------------- stage 1 (pool.hip)
 struct PoolParams {
   TokTensor x[3];       // inputs (p == nullptr -> skipped)
-  float* sums[3];       // [B, H, NB, D] fp32 block sums (nullptr -> skipped)
+  float* sums[3];       // [B, H, NB[i], D] fp32 block sums (nullptr -> skipped)
+  bf16* sb[3];          // [B, H, NBp[i], D] the same rounded to bf16, rows >= NB[i] zero (nullptr -> skipped)
   bf16* xb[3];          // bf16 copies, strides xb_* (nullptr -> skipped)
   int64_t xb_sb, xb_ss, xb_sh;
   bf16* vt;             // transposed copy of x[vt_src] (nullptr -> skipped)
   int64_t vt_sb, vt_sh, vt_sd;
   int vt_src;
   int vt_limit, vt_nblk;  // vt_limit: only blocks n < vt_nblk are transposed
-  int B, S, H, NB;      // S tokens, NB = ceil(S / 64) blocks
+  int B, H;
+  int S[3], NB[3], NBp[3];   // per input: S tokens, NB = ceil(S / 64) blocks
 };
 hipError_t launch_pool(const PoolParams& p, hipStream_t stream);
 // V^T of a list of blocks only: block base + list[bh * stride + r], r < n, of x[vt_src],
@@ -58,7 +60,6 @@ struct NewKvSumsParams {
   const float* ksum;    // [BH, Nsrc, D] source block sums
   const float* vsum;
   const int* kvmap;     // [BH, NKV]  source block index (token start / 64) or -1
-  int map_identity;     // 1: kvmap ignored, block j -> j
   float* kc32;          // [BH, NKV, D]   fp32 sums of new-KV blocks
   bf16* kc;             // [BH, NKVp, D]  bf16 sums (rows >= NKV zero)
   bf16* vct;            // [BH, D, NKVp]  bf16 sums of v transposed, kv_slot() order (nullptr: none)
@@ -216,13 +217,11 @@ struct SparseBwdParams {
   int B, H, TQ, TKV, NQ, NKV, NKVp, nc, top_k, nsplit, qb_per_split;
   float scale, scale_log2;
   // workspace
-  const float* ksum; const float* vsum;   // [BH, NKV, D] f32 block sums
   float* dvec;                       // [BH, TQ] rowsum(dO * O)
   unsigned long long* selbits;       // [BH, NQ, nc] selected key blocks per query block
   unsigned long long* seltr;         // [BH, NKV, cdiv(NQ, 64)] the same by key block
-  bf16* kcb; bf16* vcb;              // [BH, NKVp, D] bf16 block sums, rows >= NKV zero
+  const bf16* kcb; const bf16* vcb;  // [BH, NKVp, D] bf16 block sums, rows >= NKV zero
   float* dkc_part; float* dvc_part;  // [nsplit, BH, NKVp, D] interval partials
   OutView dq, dk, dv;                // (sb, token stride, sh, dtype)
 };
-hipError_t launch_sparse_bwd_prep(const SparseBwdParams& p, hipStream_t stream);
 hipError_t launch_sparse_bwd(const SparseBwdParams& p, hipStream_t stream);

@@ -11,10 +11,10 @@
 //
 // The reference adds dk / dv (and dq) with fp32 atomics, so its sums depend on timing.  Here
 // every gradient is a fixed-order sum:
-//   * icsa_sparse_bwd_dq_kernel: one workgroup per query block (dq rows are owned);
-//   * icsa_sparse_bwd_dkv_kernel<true>: one workgroup per (chunk of 64 compressed blocks,
+//   * bw_dq: one workgroup per query block (dq rows are owned);
+//   * bw_dkv<true>: one workgroup per (chunk of 64 compressed blocks,
 //     range of query blocks) -> interval partials dKC / dVC, summed later in split order;
-//   * icsa_sparse_bwd_dkv_kernel<false>: one workgroup per key block; it walks the query
+//   * bw_dkv<false>: one workgroup per key block; it walks the query
 //     blocks that selected it in ascending order (from the selection bitmap) and adds the
 //     interval partials in its epilogue.
 //
@@ -91,32 +91,12 @@ __global__ void __launch_bounds__(256) icsa_sparse_bwd_rows_kernel(SparseBwdPara
   if (t < p.nc) p.selbits[((int64_t)bh * p.NQ + i) * p.nc + t] = sel[t];
 }
 
-// prep: bf16 block sums from the f32 sums (rows >= NKV zero), and the chunk's part of the
-// selection bitmap by key block: the exact dk / dv workgroups then walk their query blocks with
-// scalar loads and bit scans alone, instead of listing them in LDS between two barriers.
-__global__ void __launch_bounds__(256) icsa_sparse_bwd_sums_kernel(SparseBwdParams p) {
-  const int ch = blockIdx.x, bh = blockIdx.y;
-  const int t = threadIdx.x;
-  const int r = t >> 2, qq = t & 3;
-  const int c = ch * ICSA_BLOCK + r;              // block index (< NKVp)
-#pragma unroll
-  for (int part = 0; part < 2; ++part) {
-    const float* src = (part == 0 ? p.ksum : p.vsum) + ((int64_t)bh * p.NKV + c) * ICSA_D + 32 * qq;
-    bf16* dst = (part == 0 ? p.kcb : p.vcb) + ((int64_t)bh * p.NKVp + c) * ICSA_D + 32 * qq;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      float v[8];
-      if (c < p.NKV) {
-        load8_f32<float>(src + 8 * g, v);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = 0.f;
-      }
-      *reinterpret_cast<bf16x8*>(dst + 8 * g) = pack8_bf16(v);
-    }
-  }
-  // 64 x 64 bits at a time: lane l holds query block 64 w + l's word, then key block 64 ch + l's
-  const int lane = t & 63, n_qw = (p.NQ + 63) / 64;
+// The selection bitmap by key block, for 64 key blocks (ch) of one head: the exact dk / dv
+// workgroups walk their query blocks with scalar loads and bit scans alone, instead of listing
+// them in LDS between two barriers.  64 x 64 bits at a time: lane l holds query block 64 w +
+// l's word, then key block 64 ch + l's.
+__device__ __forceinline__ void bw_transpose_bits(const SparseBwdParams& p, int bh, int ch) {
+  const int t = threadIdx.x, lane = t & 63, n_qw = (p.NQ + 63) / 64;
   for (int w = t >> 6; w < n_qw; w += 4) {
     const int i = 64 * w + lane;
     const unsigned long long word = i < p.NQ ? p.selbits[((int64_t)bh * p.NQ + i) * p.nc + ch] : 0ull;
@@ -255,14 +235,7 @@ __device__ __forceinline__ void bw_reduce_stage(float* o_lds, const floatx16 o[4
 // dQ^T += K^T dS^T (K^T read transposed from the K rows) run.  Wave w: queries
 // 32 (w % 2) .. + 31 in registers, keys 32 (w / 2) .. + 31 of each step.
 // ------------------------------------------------------------------------------------------
-#define BWQ_LDS_BYTES (4 * K_TILE_BYTES)
-
-__global__ void __launch_bounds__(BW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
-icsa_sparse_bwd_dq_kernel(SparseBwdParams p) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_q[];
-  const int n_work = p.B * p.H * p.NQ;
-  const int work = xcd_remap(blockIdx.x, n_work);
-  if (work < 0) return;
+__device__ __forceinline__ void bw_dq(const SparseBwdParams& p, unsigned char* smem_q, int work) {
   const int bh = work / p.NQ, qb = work % p.NQ;
   const int b = bh / p.H, h = bh % p.H;
   const int tid = threadIdx.x;
@@ -391,19 +364,14 @@ icsa_sparse_bwd_dq_kernel(SparseBwdParams p) {
 // ------------------------------------------------------------------------------------------
 #define BWKV_BUF_BYTES (2 * K_TILE_BYTES + 2 * 64 * 4)      // Q rows, dO rows, lse, D
 #define BWKV_P_BYTES (4 * 2 * 1024)                         // each wave's P: two 16-row operands
-#define BWKV_LDS_BYTES (2 * BWKV_BUF_BYTES + BWKV_P_BYTES + 2 * ICSA_D * 4)
+#define BW_LDS_BYTES (2 * BWKV_BUF_BYTES + BWKV_P_BYTES + 2 * ICSA_D * 4)
 #define BWKV_SUM_AHEAD 16                                   // interval partials requested together
 
 template <bool kInterval>
-__global__ void __launch_bounds__(BW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
-icsa_sparse_bwd_dkv_kernel(SparseBwdParams p) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_dyn[];
+__device__ __forceinline__ void bw_dkv(const SparseBwdParams& p, unsigned char* smem_dyn, int work) {
   unsigned char* pbuf = smem_dyn + 2 * BWKV_BUF_BYTES;
   float* ivec = reinterpret_cast<float*>(pbuf + BWKV_P_BYTES);    // [2][128] interval sums
 
-  const int n_work = kInterval ? p.B * p.H * p.nc * p.nsplit : p.B * p.H * p.NKV;
-  const int work = xcd_remap(blockIdx.x, n_work);
-  if (work < 0) return;
   int bh, blk, split = 0;
   if (kInterval) {
     bh = work / (p.nc * p.nsplit);
@@ -575,13 +543,34 @@ icsa_sparse_bwd_dkv_kernel(SparseBwdParams p) {
   }
 }
 
-hipError_t launch_sparse_bwd_prep(const SparseBwdParams& p, hipStream_t stream) {
-  const int BH = p.B * p.H;
-  if (BH == 0 || p.NQ == 0) return hipSuccess;
-  if (p.nc > BW_MAX_CHUNKS || p.NKVp != p.nc * ICSA_BLOCK) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(icsa_sparse_bwd_rows_kernel, dim3(p.NQ, BH), dim3(256), 0, stream, p);
-  hipLaunchKernelGGL(icsa_sparse_bwd_sums_kernel, dim3(p.nc, BH), dim3(256), 0, stream, p);
-  return hipGetLastError();
+// Two launches: the query-major part with the interval part and the transposed bitmap (which
+// do not depend on each other: their last rounds overlap; 345 us against 295 + 61 + 8 us one
+// after another at 40 heads, 7,800 tokens), then the exact key-major part, which needs the
+// other two.
+__global__ void __launch_bounds__(BW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+icsa_sparse_bwd_query_kernel(SparseBwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_bw[];
+  const int BH = p.B * p.H, n_iv = BH * p.nc * p.nsplit, n_tr = BH * p.nc;
+  int blk = blockIdx.x;
+  if (blk < xcd_grid(n_iv)) {                          // the longest workgroups first
+    const int work = xcd_remap(blk, n_iv);
+    if (work >= 0) bw_dkv<true>(p, smem_bw, work);
+    return;
+  }
+  blk -= xcd_grid(n_iv);
+  if (blk < xcd_grid(n_tr)) {
+    if (blk < n_tr) bw_transpose_bits(p, blk / p.nc, blk % p.nc);
+    return;
+  }
+  const int work = xcd_remap(blk - xcd_grid(n_tr), BH * p.NQ);
+  if (work >= 0) bw_dq(p, smem_bw, work);
+}
+
+__global__ void __launch_bounds__(BW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+icsa_sparse_bwd_key_kernel(SparseBwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_bw[];
+  const int work = xcd_remap(blockIdx.x, p.B * p.H * p.NKV);
+  if (work >= 0) bw_dkv<false>(p, smem_bw, work);
 }
 
 hipError_t launch_sparse_bwd(const SparseBwdParams& p, hipStream_t stream) {
@@ -591,18 +580,14 @@ hipError_t launch_sparse_bwd(const SparseBwdParams& p, hipStream_t stream) {
       p.NKVp != p.nc * ICSA_BLOCK || p.NQ > BW_MAX_NQ || p.nsplit < 1 ||
       (int64_t)p.nsplit * p.qb_per_split < p.NQ)
     return hipErrorInvalidValue;
-  static std::atomic<unsigned> set_q{0u}, set_i{0u}, set_e{0u};
-  hipError_t attr = ensure_lds_limit(reinterpret_cast<const void*>(icsa_sparse_bwd_dq_kernel), BWQ_LDS_BYTES, &set_q);
+  static std::atomic<unsigned> set_q{0u}, set_k{0u};
+  hipError_t attr = ensure_lds_limit(reinterpret_cast<const void*>(icsa_sparse_bwd_query_kernel), BW_LDS_BYTES, &set_q);
   if (attr != hipSuccess) return attr;
-  attr = ensure_lds_limit(reinterpret_cast<const void*>(icsa_sparse_bwd_dkv_kernel<true>), BWKV_LDS_BYTES, &set_i);
+  attr = ensure_lds_limit(reinterpret_cast<const void*>(icsa_sparse_bwd_key_kernel), BW_LDS_BYTES, &set_k);
   if (attr != hipSuccess) return attr;
-  attr = ensure_lds_limit(reinterpret_cast<const void*>(icsa_sparse_bwd_dkv_kernel<false>), BWKV_LDS_BYTES, &set_e);
-  if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(icsa_sparse_bwd_dq_kernel, dim3(xcd_grid(BH * p.NQ)), dim3(BW_THREADS), BWQ_LDS_BYTES,
-                     stream, p);
-  hipLaunchKernelGGL(icsa_sparse_bwd_dkv_kernel<true>, dim3(xcd_grid(BH * p.nc * p.nsplit)), dim3(BW_THREADS),
-                     BWKV_LDS_BYTES, stream, p);
-  hipLaunchKernelGGL(icsa_sparse_bwd_dkv_kernel<false>, dim3(xcd_grid(BH * p.NKV)), dim3(BW_THREADS),
-                     BWKV_LDS_BYTES, stream, p);
+  hipLaunchKernelGGL(icsa_sparse_bwd_rows_kernel, dim3(p.NQ, BH), dim3(256), 0, stream, p);
+  const int grid = xcd_grid(BH * p.nc * p.nsplit) + xcd_grid(BH * p.nc) + xcd_grid(BH * p.NQ);
+  hipLaunchKernelGGL(icsa_sparse_bwd_query_kernel, dim3(grid), dim3(BW_THREADS), BW_LDS_BYTES, stream, p);
+  hipLaunchKernelGGL(icsa_sparse_bwd_key_kernel, dim3(xcd_grid(BH * p.NKV)), dim3(BW_THREADS), BW_LDS_BYTES, stream, p);
   return hipGetLastError();
 }
