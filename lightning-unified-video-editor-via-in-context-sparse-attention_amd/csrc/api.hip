@@ -96,6 +96,10 @@ struct Layout {
 // then the topK selected source blocks (tile j at columns 64 j .. 64 j + 63)
 int64_t vt_columns(const Sizes& z, int t) { return ((int64_t)ceil_div(t, ICSA_BLOCK) + z.topK) * ICSA_BLOCK; }
 
+int64_t l3_bound_off(int BH, const Sizes& z) {
+  return align256(std::max((int64_t)BH * std::max(z.n_diffuse, 1) * z.NKV * 4, compressed_vmt_bytes(BH, z.NB)));
+}
+
 Layout editing_layout(int B, int S, int H, const Sizes& z, int t, int q_dtype, int k_dtype, int v_dtype) {
   const int64_t BH = (int64_t)B * H;
   const int64_t D = ICSA_D;
@@ -121,8 +125,9 @@ Layout editing_layout(int B, int S, int H, const Sizes& z, int t, int q_dtype, i
   sz[ICSA_WS_L3] = BH * std::max(z.n_diffuse, 1) * z.top_k * 4;
   sz[ICSA_WS_VC] = unaligned ? BH * z.NKVp * D * 2 : 0;
   sz[ICSA_WS_COLP] = BH * ceil_div(z.n_t, ICSA_BLOCK) * std::max(z.n_s, 1) * 4;
-  // the level-3 scores, and before them the compressed stage's split value means
-  sz[ICSA_WS_L3S] = std::max(BH * std::max(z.n_diffuse, 1) * z.NKV * 4, compressed_vmt_bytes((int)BH, z.NB));
+  // the level-3 scores, and before them the compressed stage's split value means; then the
+  // interval bound
+  sz[ICSA_WS_L3S] = l3_bound_off((int)BH, z) + BH * kc_bound_groups(z.NKV) * 4;
   sz[ICSA_WS_RSTAT] = BH * z.NB * 2 * 4;
   sz[ICSA_WS_FLASHP] = flash_plan(flash_items((int)BH, z.n_peaked), ceil_div(t, ICSA_BLOCK) + z.topK, true).part_bytes;
   Layout L;
@@ -329,17 +334,15 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
   sp.inject_sel = inject_sel ? 1 : 0;
   sp.inject_order = inject_order ? 1 : 0;
   ICSA_HIP_TRY(launch_select(sp, stream), "select");
-  ICSA_HIP_TRY(launch_vt_blocks(pp, sel, z.n_t, std::max(z.topK, 1), z.topK, pp.vt_nblk, stream),
-               "V^T of the selected blocks");
 
-  // ---- new-KV block sums ----
+  // ---- new-KV block sums, V^T of the selected blocks ----
   // The new KV is read in place.  For t % 64 != 0 its blocks from n_t on straddle two
   // blocks of the sequence (the t % 64 target-tail tokens, or the tail of the previous
   // selected block, then the head of the next one); their sums come from the token rows.
   const int seg_a = t_seq_len % ICSA_BLOCK;
-  NewKvSumsParams np;
+  NewKvParams np;
   std::memset(&np, 0, sizeof(np));
-  np.kc32 = reinterpret_cast<float*>(WS(ICSA_WS_KC32));
+  np.kc32 = z.n_diffuse > 0 ? reinterpret_cast<float*>(WS(ICSA_WS_KC32)) : nullptr;
   np.kc = reinterpret_cast<bf16*>(WS(ICSA_WS_KC));
   np.vct = unaligned ? nullptr : reinterpret_cast<bf16*>(WS(ICSA_WS_VCT));
   np.vc = unaligned ? reinterpret_cast<bf16*>(WS(ICSA_WS_VC)) : nullptr;
@@ -354,21 +357,24 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
   const int64_t vr_sb = v_dtype == ICSA_BF16 ? v_sb : pp.xb_sb;
   const int64_t vr_ss = v_dtype == ICSA_BF16 ? v_ss : pp.xb_ss;
   const int64_t vr_sh = v_dtype == ICSA_BF16 ? v_sh : pp.xb_sh;
-  if (z.n_diffuse > 0) ICSA_HIP_TRY(launch_newkv_sums(np, stream), "new-KV sums");
+  np.sel = sel; np.sel_stride = std::max(z.topK, 1); np.n_sel = z.topK; np.sel_base = z.n_t;
+  np.vt_dst0 = pp.vt_nblk; np.vt = pp.vt; np.vt_sb = pp.vt_sb; np.vt_sh = pp.vt_sh; np.vt_sd = pp.vt_sd;
+  ICSA_HIP_TRY(launch_newkv(np, stream), "new-KV tables");
 
   // ---- level-3 selection for the diffuse blocks ----
   int32_t* l3 = reinterpret_cast<int32_t*>(WS(ICSA_WS_L3));
+  float* bound = reinterpret_cast<float*>(WS(ICSA_WS_L3S) + l3_bound_off(BH, z));
   if (z.n_diffuse > 0) {
-    if (inject_l3) {
+    if (inject_l3)
       ICSA_HIP_TRY(hipMemcpyAsync(l3, inject_l3, (size_t)BH * z.n_diffuse * z.top_k * 4,
                                   hipMemcpyDeviceToDevice, stream), "inject l3");
-    } else {
-      Level3Params lp;
-      lp.qsum = qsum; lp.rows = order; lp.rows_offset = z.n_peaked; lp.rows_stride = z.NB;
-      lp.kc32 = np.kc32; lp.idx = l3; lp.scores = reinterpret_cast<float*>(WS(ICSA_WS_L3S));
-      lp.BH = BH; lp.NQsrc = z.NB; lp.n_rows = z.n_diffuse; lp.NKV = z.NKV; lp.top_k = z.top_k;
-      ICSA_HIP_TRY(launch_level3(lp, stream), "level-3 top-k");
-    }
+    Level3Params lp;
+    lp.qsum = qsum; lp.rows = order; lp.rows_offset = z.n_peaked; lp.rows_stride = z.NB;
+    lp.kc32 = np.kc32; lp.idx = l3; lp.scores = reinterpret_cast<float*>(WS(ICSA_WS_L3S));
+    lp.BH = BH; lp.NQsrc = z.NB; lp.n_rows = z.n_diffuse; lp.NKV = z.NKV; lp.top_k = z.top_k;
+    lp.given = inject_l3 ? 1 : 0;
+    lp.kc = np.kc; lp.NKVp = z.NKVp; lp.bound = interval_skip_enabled() ? bound : nullptr;
+    ICSA_HIP_TRY(launch_level3(lp, stream), "level-3 top-k");
   }
 
   ICSA_HIP_TRY(mark(ICSA_STAGE_SELECT), "event");
@@ -398,13 +404,8 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
     s.out_c = cp.out_c; s.nb_q = z.NB;
     s.alpha = av; s.out = ov; s.scale_log2 = scale_log2; s.lse = nullptr;
     s.mask_tail = 0;                   // zero-padded new KV attended with logit 0 (TileLang)
-    // the level-3 score rows are free again: BH * min(8, cdiv(NKV, 16)) floats of them hold the |KC_j|
-    // bound of the interval pass
-    if (interval_skip_enabled()) {
-      s.kc_bound = reinterpret_cast<float*>(WS(ICSA_WS_L3S));
-      ICSA_HIP_TRY(launch_kc_bound(np.kc, BH, z.NKV, z.NKVp, reinterpret_cast<float*>(WS(ICSA_WS_L3S)),
-                                   &s.kc_bound_n, stream), "interval bound");
-    }
+    s.kc_bound = interval_skip_enabled() ? bound : nullptr;
+    s.kc_bound_n = kc_bound_groups(z.NKV);
     ICSA_HIP_TRY(launch_sparse(s, stream), "sparse attention");
   }
   ICSA_HIP_TRY(mark(ICSA_STAGE_SPARSE), "event");
@@ -636,7 +637,7 @@ int icsa_wan_qk_prologue(
 
 namespace {
 struct SpLayout {
-  int64_t qsum, ksum, kc, vc, idx, scores, total;
+  int64_t qsum, ksum, kc, vc, idx, scores, bound, total;
 };
 // Sizes for TQ / TKV rounded up to whole blocks (the Triton host's ragged lengths); the
 // index buffer holds max(1, int(sparsity * NKV)) entries per query block, which is at
@@ -654,6 +655,7 @@ SpLayout sparse_layout(int B, int H, int TQ, int TKV, double sparsity) {
   L.vc = o; o += align256(BH * NKVp * ICSA_D * 2);
   L.idx = o; o += align256(BH * NQ * top_k * 4);
   L.scores = o; o += align256(BH * NQ * (int64_t)NKV * 4);
+  L.bound = o; o += align256(BH * kc_bound_groups(NKV) * 4);
   L.total = o;
   return L;
 }
@@ -722,8 +724,12 @@ static int sparse_piecewise_impl(
   if (inject_idx) {
     ICSA_HIP_TRY(hipMemcpyAsync(idx, inject_idx, (size_t)BH * NQ * top_k * 4, hipMemcpyDeviceToDevice,
                                 stream), "inject idx");
-  } else {
+  }
+  float* bound = interval_skip_enabled() ? reinterpret_cast<float*>(ws + L.bound) : nullptr;
+  {
     Level3Params lp;
+    lp.given = inject_idx ? 1 : 0;
+    lp.kc = pp.sb[1]; lp.NKVp = NKVp; lp.bound = bound;
     lp.qsum = pp.sums[0]; lp.rows = nullptr; lp.rows_offset = 0; lp.rows_stride = 0;
     lp.kc32 = pp.sums[1]; lp.idx = idx; lp.scores = reinterpret_cast<float*>(ws + L.scores);
     lp.BH = BH; lp.NQsrc = NQ; lp.n_rows = NQ; lp.NKV = NKV; lp.top_k = top_k;
@@ -749,13 +755,8 @@ static int sparse_piecewise_impl(
   s.lse = lse_out;
   s.mask_tail = triton;
   s.interval_bn = interval_bn;
-  // the block top-k score rows are free again: BH * min(8, cdiv(NKV, 16)) floats of them hold the
-  // |KC_j| bound of the interval pass
-  if (interval_skip_enabled()) {
-    s.kc_bound = reinterpret_cast<float*>(ws + L.scores);
-    ICSA_HIP_TRY(launch_kc_bound(pp.sb[1], BH, NKV, NKVp, reinterpret_cast<float*>(ws + L.scores),
-                                 &s.kc_bound_n, stream), "interval bound");
-  }
+  s.kc_bound = bound;
+  s.kc_bound_n = kc_bound_groups(NKV);
   ICSA_HIP_TRY(launch_sparse(s, stream), "sparse attention");
   return ICSA_OK;
 }

@@ -10,6 +10,8 @@
 // Every ranked decision uses the rule "larger value first, lower index first on ties".
 // All score arithmetic is fp32 with fixed reduction orders, so repeated runs are bitwise
 // identical and no float atomics are used.
+#include <algorithm>
+
 #include "attn_tile.h"
 #include "icsa_kernels.h"
 
@@ -31,15 +33,15 @@ __device__ __forceinline__ float block_size_f(int blk, int NB, int S) {
 //     accumulator.  So the logits carry fp32-level rounding while the matrix work takes
 //     6 bf16 MFMAs (32x32x16, 32 cycles) per 16 dims instead of 8 fp32 ones (32x32x2, 64).
 //     Workgroup = 4 waves = 128 query rows (wave w: rows 32 w .. 32 w + 31) against one of
-//     LG_SPLIT column ranges.  A wave's split A operands stay in registers for the whole
+//     lg_split() column ranges.  A wave's split A operands stay in registers for the whole
 //     range (lane (li, hl) holds row li's dims 16 s + 8 hl .. + 7, s = 0 .. 7); 32-column K
 //     tiles pass through a double-buffered LDS ring of split tiles, the next tile prefetched
 //     into registers while the current one is multiplied.  A fixed order of MFMAs, so
 //     repeated runs are bitwise identical.
 // ---------------------------------------------------------------------------------------
-#define LG_SPLIT 3
 #define LG_ROWS 128
 #define LG_COLS 32
+#define LG_MIN_WG 256
 #define LG_KST 136            // bf16 row stride of a split K tile (272 B: conflict-free reads)
 
 __device__ __forceinline__ void split3_bf16(float x, bf16& h, bf16& m, bf16& l) {
@@ -62,12 +64,77 @@ struct Split3Gemm {
   float* C;                 // [BH, n_rows, n_cols]
   int NB, S;                // block sizes (block_mean)
   float div;
+  int n_split;              // column ranges
 };
 
+// Column ranges per 128 rows: three (each range splits the rows' operands again; two and four
+// were slower at 40 heads, 1,024 blocks), more where that leaves CUs without a workgroup, down
+// to one 32-column tile a range: 5 heads, 1,024 blocks, logits 42 -> 32 us and level-3 scores
+// 20 -> 12 us with 7 and 13 ranges; 2 heads, 128 blocks, 12.9 -> 10.5 us with 4.
+static int lg_split(int n_rows, int n_cols, int BH) {
+  const int64_t row_wg = (int64_t)BH * ((n_rows + LG_ROWS - 1) / LG_ROWS);
+  const int n_ct = (n_cols + LG_COLS - 1) / LG_COLS;
+  return std::max(1, std::min<int>(n_ct, (int)std::max<int64_t>(3, (LG_MIN_WG + row_wg - 1) / row_wg)));
+}
+
+// The value means for the strip pass (c), by workgroups of the logits' launch past its n_rt row
+// tiles (they need nothing of the logits; as a launch of its own this cost 4-5 us).
+struct VmeanParams {
+  const float* vsum;        // [BH, NB, D]
+  bf16* vmt;                // CompressedParams::vmt
+  int NB, NBp, S, n_rt;
+};
+
+// Vm = Vsum / block size, transposed and split in two bf16 parts, for keys k0 .. k0 + 63:
+// vmt[((bh * 2 + part) * D + d) * NBp + key], zero for keys >= NB.
+__device__ __forceinline__ void vmean_split(const VmeanParams& p, int bh, int k0, float (*tile)[ICSA_D + 4]) {
+  const int NB = p.NB, NBp = p.NBp, t = threadIdx.x;
+  const float* V = p.vsum + (int64_t)bh * NB * ICSA_D;
+  floatx4 v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {                 // float4 f = t + 256 j: key f / 32, dims 4 (f % 32)
+    const int f = t + 256 * j, key = k0 + (f >> 5);
+    v[j] = key < NB ? *reinterpret_cast<const floatx4*>(V + (int64_t)key * ICSA_D + 4 * (f & 31))
+                    : floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int f = t + 256 * j, key = k0 + (f >> 5);
+    if (key < NB) {
+      const float inv = 1.f / block_size_f(key, NB, p.S);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[j][e] *= inv;
+    }
+    *reinterpret_cast<floatx4*>(&tile[f >> 5][4 * (f & 31)]) = v[j];
+  }
+  __syncthreads();
+  const int d = t >> 1, kh = t & 1;             // dim d, keys 32 kh .. + 31
+  bf16* dst = p.vmt + ((int64_t)bh * 2 * ICSA_D + d) * NBp + k0 + 32 * kh;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    bf16x8 hi, lo;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float x = tile[32 * kh + 8 * g + i][d];
+      const bf16 h = f2bf(x);
+      hi[i] = h;
+      lo[i] = f2bf(x - bf2f(h));
+    }
+    *reinterpret_cast<bf16x8*>(dst + 8 * g) = hi;
+    *reinterpret_cast<bf16x8*>(dst + (int64_t)ICSA_D * NBp + 8 * g) = lo;
+  }
+}
+
 template <bool BLOCK_MEAN>
-__global__ void __launch_bounds__(256) icsa_split3_gemm_kernel(Split3Gemm g) {
+__global__ void __launch_bounds__(256) icsa_split3_gemm_kernel(Split3Gemm g, VmeanParams vm) {
   __shared__ __attribute__((aligned(16))) bf16 ks[2][3][LG_COLS][LG_KST];
   const int rt = blockIdx.x, cs = blockIdx.y, bh = blockIdx.z;
+  if (BLOCK_MEAN && rt >= vm.n_rt) {
+    static_assert(sizeof(ks) >= 64 * (ICSA_D + 4) * sizeof(float), "the value tile shares the K tiles' LDS");
+    const int k0 = ((rt - vm.n_rt) * (int)gridDim.y + cs) * 64;
+    if (k0 < vm.NBp) vmean_split(vm, bh, k0, reinterpret_cast<float (*)[ICSA_D + 4]>(&ks[0][0][0][0]));
+    return;
+  }
   const int NC = g.n_cols;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
   const int li = l & 31, hl = l >> 5;
@@ -102,7 +169,7 @@ __global__ void __launch_bounds__(256) icsa_split3_gemm_kernel(Split3Gemm g) {
   }
 
   const int n_ct = (NC + LG_COLS - 1) / LG_COLS;
-  const int per = (n_ct + LG_SPLIT - 1) / LG_SPLIT;
+  const int per = (n_ct + g.n_split - 1) / g.n_split;
   const int t0 = cs * per, t1 = min(n_ct, t0 + per);
   if (t0 >= t1) return;                                // uniform for the workgroup
 
@@ -328,7 +395,7 @@ __global__ void __launch_bounds__(256) icsa_compressed_stats_kernel(CompressedPa
 // (c) one 64-row strip of P per workgroup of 8 waves, in 32-key chunks: out_c = P Vm with
 //     P = exp(L - m) / z, on the bf16 matrix pipe from split operands.  Per chunk:
 //       * the chunk's logits (64 x 32 fp32) and its split, transposed value means (two bf16
-//         planes of 128 dims x 32 keys, icsa_vmean_split_kernel) arrive by LDS DMA, double
+//         planes of 128 dims x 32 keys, vmean_split) arrive by LDS DMA, double
 //         buffered: chunk c + 1 is in flight while chunk c is computed, and two workgroups
 //         share each CU (65 KB of LDS each);
 //       * P is formed once in fp32 and kept as its two bf16 parts P = Ph + Pl (to 2^-17 of
@@ -341,48 +408,6 @@ __global__ void __launch_bounds__(256) icsa_compressed_stats_kernel(CompressedPa
 //     Fixed orders throughout, so repeated runs are bitwise identical.
 // ---------------------------------------------------------------------------------------
 #define RW_PB_LD 36                             // floats per P row in LDS (16-byte skew)
-
-// Vm = Vsum / block size, transposed and split in two bf16 parts:
-// vmt[((bh * 2 + part) * D + d) * NBp + key], zero for keys >= NB.
-__global__ void __launch_bounds__(256) icsa_vmean_split_kernel(CompressedParams p, int NBp) {
-  __shared__ float tile[64][ICSA_D + 4];
-  const int k0 = blockIdx.x * 64, bh = blockIdx.y;
-  const int NB = p.NB, t = threadIdx.x;
-  const float* V = p.vsum + (int64_t)bh * NB * ICSA_D;
-  floatx4 v[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {                 // float4 f = t + 256 j: key f / 32, dims 4 (f % 32)
-    const int f = t + 256 * j, key = k0 + (f >> 5);
-    v[j] = key < NB ? *reinterpret_cast<const floatx4*>(V + (int64_t)key * ICSA_D + 4 * (f & 31))
-                    : floatx4{0.f, 0.f, 0.f, 0.f};
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int f = t + 256 * j, key = k0 + (f >> 5);
-    if (key < NB) {
-      const float inv = 1.f / block_size_f(key, NB, p.S);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[j][e] *= inv;
-    }
-    *reinterpret_cast<floatx4*>(&tile[f >> 5][4 * (f & 31)]) = v[j];
-  }
-  __syncthreads();
-  const int d = t >> 1, kh = t & 1;             // dim d, keys 32 kh .. + 31
-  bf16* dst = p.vmt + ((int64_t)bh * 2 * ICSA_D + d) * NBp + k0 + 32 * kh;
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    bf16x8 hi, lo;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float x = tile[32 * kh + 8 * g + i][d];
-      const bf16 h = f2bf(x);
-      hi[i] = h;
-      lo[i] = f2bf(x - bf2f(h));
-    }
-    *reinterpret_cast<bf16x8*>(dst + 8 * g) = hi;
-    *reinterpret_cast<bf16x8*>(dst + (int64_t)ICSA_D * NBp + 8 * g) = lo;
-  }
-}
 
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 icsa_compressed_rows_kernel(CompressedParams p, int NBp) {
@@ -509,8 +534,11 @@ hipError_t launch_compressed(const CompressedParams& p, hipStream_t stream) {
   g.A = p.qsum; g.rows = nullptr; g.rows_stride = 0; g.rows_offset = 0; g.a_rows = p.NB;
   g.n_rows = p.NB; g.B = p.ksum; g.n_cols = p.NB; g.C = p.L; g.NB = p.NB; g.S = p.S;
   g.div = sqrtf((float)ICSA_D);
-  hipLaunchKernelGGL(icsa_split3_gemm_kernel<true>, dim3((p.NB + LG_ROWS - 1) / LG_ROWS, LG_SPLIT, p.BH),
-                     dim3(256), 0, stream, g);
+  g.n_split = lg_split(p.NB, p.NB, p.BH);
+  const int NBp = compressed_nbp(p.NB), n_rt = (p.NB + LG_ROWS - 1) / LG_ROWS;
+  const VmeanParams vm{p.vsum, p.vmt, p.NB, NBp, p.S, n_rt};
+  const int n_vm = (NBp / 64 + g.n_split - 1) / g.n_split;
+  hipLaunchKernelGGL(icsa_split3_gemm_kernel<true>, dim3(n_rt + n_vm, g.n_split, p.BH), dim3(256), 0, stream, g, vm);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int64_t rows = (int64_t)p.BH * p.NB;
@@ -527,10 +555,6 @@ hipError_t launch_compressed(const CompressedParams& p, hipStream_t stream) {
     hipLaunchKernelGGL(icsa_compressed_stats_kernel<40>, sgrid, dim3(256), 0, stream, p);
   else
     hipLaunchKernelGGL(icsa_compressed_stats_kernel<64>, sgrid, dim3(256), 0, stream, p);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int NBp = compressed_nbp(p.NB);
-  hipLaunchKernelGGL(icsa_vmean_split_kernel, dim3(NBp / 64, p.BH), dim3(256), 0, stream, p, NBp);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(icsa_compressed_rows_kernel, dim3(nt, p.BH), dim3(512), 0, stream, p, NBp);
@@ -630,120 +654,48 @@ hipError_t launch_select(const SelectParams& p, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------------------
-// (e) sums of the new-KV blocks (fp32 for scoring; bf16 rows / transposed for the kernel)
-// ---------------------------------------------------------------------------------------
-// One workgroup per 16 consecutive new-KV blocks, thread d: dim d of each (the 32 source
-// sums of a thread are requested together).  The 16 blocks' V sums of dim d are one
-// 16-slot group of V^T row d, written as 32 contiguous bytes in kv_slot() order (kv_slot
-// swaps two index bits, so it is its own inverse).
-__global__ void __launch_bounds__(128) icsa_newkv_sums_kernel(NewKvSumsParams p) {
-  const int j0 = 16 * blockIdx.x, bh = blockIdx.y, d = threadIdx.x;
-  float ks[16], vs[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int j = j0 + i;
-    int src = -1;
-    if (j < p.NKV) src = p.kvmap[(int64_t)bh * p.NKV + j];
-    ks[i] = 0.f;
-    vs[i] = 0.f;
-    if (src >= 0) {
-      ks[i] = p.ksum[((int64_t)bh * p.Nsrc + src) * ICSA_D + d];
-      vs[i] = p.vsum[((int64_t)bh * p.Nsrc + src) * ICSA_D + d];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int j = j0 + i;
-    if (p.seg_a > 0 && j >= p.seg_from && j < p.NKV) continue;   // icsa_newkv_straddle_kernel
-    if (j < p.NKV) p.kc32[((int64_t)bh * p.NKV + j) * ICSA_D + d] = ks[i];
-    p.kc[((int64_t)bh * p.NKVp + j) * ICSA_D + d] = f2bf(ks[i]);
-    if (p.vc) p.vc[((int64_t)bh * p.NKVp + j) * ICSA_D + d] = f2bf(vs[i]);
-  }
-  if (p.vct) {                    // no straddling blocks where V^T sums are wanted (seg_a == 0)
-    bf16x8 a, b;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      a[s] = f2bf(vs[kv_slot(s)]);
-      b[s] = f2bf(vs[kv_slot(s + 8)]);
-    }
-    bf16* dst = p.vct + ((int64_t)bh * ICSA_D + d) * p.NKVp + j0;
-    *reinterpret_cast<bf16x8*>(dst) = a;
-    *reinterpret_cast<bf16x8*>(dst + 8) = b;
-  }
-}
-
-// Straddling new-KV block j (the pipeline's new KV when t % 64 != 0; see SparseParams):
-// rows r < a from tokens segA + r, rows r >= a from 64 kvmap[j] + r - a, summed straight
-// from the token rows.  Thread t: 8 dims 8 (t % 16) .. + 7 of rows t / 16 + 8 m; the 8
-// row groups are added in fixed order.
-template <typename TK, typename TV>
-__global__ void __launch_bounds__(128) icsa_newkv_straddle_kernel(NewKvSumsParams p) {
-  __shared__ float red[2][8][ICSA_D + 4];
-  const int j = p.seg_from + blockIdx.x, bh = blockIdx.y;
-  const int b = bh / p.H, h = bh % p.H;
-  const int t = threadIdx.x, c = t & 15, g = t >> 4;
-  const int a = p.seg_a;
-  const int* map = p.kvmap + (int64_t)bh * p.NKV;
-  int tokA = -1;
-  if (j == p.seg_from) tokA = ICSA_BLOCK * p.seg_from;
-  else if (map[j - 1] >= 0) tokA = ICSA_BLOCK * map[j - 1] + ICSA_BLOCK - a;
-  const int tokB = map[j] >= 0 ? ICSA_BLOCK * map[j] - a : -1;    // token of row r >= a: tokB + r
-  const TK* kb = reinterpret_cast<const TK*>(p.k.p) + (int64_t)b * p.k.sb + (int64_t)h * p.k.sh;
-  const TV* vb = reinterpret_cast<const TV*>(p.v.p) + (int64_t)b * p.v.sb + (int64_t)h * p.v.sh;
-  float ks[8], vs[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) { ks[e] = 0.f; vs[e] = 0.f; }
-#pragma unroll
-  for (int m = 0; m < 8; ++m) {
-    const int r = g + 8 * m;
-    const int tok = r < a ? (tokA < 0 ? -1 : tokA + r) : (tokB < 0 ? -1 : tokB + r);
-    if (tok >= 0 && tok < p.S) {
-      float x[8];
-      load8_f32(kb + (int64_t)tok * p.k.ss + 8 * c, x);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ks[e] += x[e];
-      load8_f32(vb + (int64_t)tok * p.v.ss + 8 * c, x);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vs[e] += x[e];
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) { red[0][g][8 * c + e] = ks[e]; red[1][g][8 * c + e] = vs[e]; }
-  __syncthreads();
-  const int d = t;
-  float k_sum = 0.f, v_sum = 0.f;
-#pragma unroll
-  for (int gg = 0; gg < 8; ++gg) { k_sum += red[0][gg][d]; v_sum += red[1][gg][d]; }
-  p.kc32[((int64_t)bh * p.NKV + j) * ICSA_D + d] = k_sum;
-  p.kc[((int64_t)bh * p.NKVp + j) * ICSA_D + d] = f2bf(k_sum);
-  if (p.vct) p.vct[((int64_t)bh * ICSA_D + d) * p.NKVp + (j & ~15) + kv_slot(j & 15)] = f2bf(v_sum);
-  if (p.vc) p.vc[((int64_t)bh * p.NKVp + j) * ICSA_D + d] = f2bf(v_sum);
-}
-
-hipError_t launch_newkv_sums(const NewKvSumsParams& p, hipStream_t stream) {
-  if (p.NKVp % 16 != 0 || (p.vct && p.seg_a > 0)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(icsa_newkv_sums_kernel, dim3(p.NKVp / 16, p.BH), dim3(128), 0, stream, p);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || p.seg_a <= 0 || p.seg_from >= p.NKV) return e;
-  if (!p.kvmap || !p.k.p || !p.v.p) return hipErrorInvalidValue;
-  const dim3 grid(p.NKV - p.seg_from, p.BH);
-  const bool kf = p.k.dtype == ICSA_DT_F32, vf = p.v.dtype == ICSA_DT_F32;
-  if (kf && vf) hipLaunchKernelGGL((icsa_newkv_straddle_kernel<float, float>), grid, dim3(128), 0, stream, p);
-  else if (kf) hipLaunchKernelGGL((icsa_newkv_straddle_kernel<float, bf16>), grid, dim3(128), 0, stream, p);
-  else if (vf) hipLaunchKernelGGL((icsa_newkv_straddle_kernel<bf16, float>), grid, dim3(128), 0, stream, p);
-  else hipLaunchKernelGGL((icsa_newkv_straddle_kernel<bf16, bf16>), grid, dim3(128), 0, stream, p);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------------------
-// (f) level-3: per query block, top_k new-KV blocks by QCsum . KCsum (fp32), ascending list.
+// (e) level-3: per query block, top_k new-KV blocks by QCsum . KCsum (fp32), ascending list.
 //     Scores: the fp32-accurate split-bf16 product of (a) on the raw sums (128 query blocks
-//     of the list per workgroup, a third of the new-KV blocks), written to a scratch row
+//     of the list per workgroup, a range of the new-KV blocks), written to a scratch row
 //     per query block.  Selection: one wave per query block, bisection over the float keys
-//     (ballot counts), then compaction in ascending block order.
+//     (ballot counts), then compaction in ascending block order.  The interval bound of the
+//     sparse kernel (largest |KC_j| of each head) takes the launch's last workgroups: as a
+//     launch of its own it cost 4-5 us.
 // ---------------------------------------------------------------------------------------
+// Workgroup y of G per head: rows j = 16 (y + G i) + r, r = 0 .. 15 (i = 0, 1, ...); 16 lanes
+// per row, one 16-byte chunk each, the squared norm summed over the 16 lanes with lane
+// shuffles; the workgroup maximum goes through an LDS atomic (non-negative floats order like
+// their bit patterns).
+__device__ __forceinline__ void kc_bound(const Level3Params& p, int bh, int y, int G) {
+  __shared__ unsigned mx;
+  const int r = threadIdx.x >> 4, ch = threadIdx.x & 15;
+  if (threadIdx.x == 0) mx = 0u;
+  __syncthreads();
+  float best = 0.f;
+  for (int j0 = 16 * y; j0 < p.NKV; j0 += 16 * G) {
+    const int j = j0 + r;
+    float n2 = 0.f;
+    if (j < p.NKV) {
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(p.kc + ((int64_t)bh * p.NKVp + j) * ICSA_D + 8 * ch);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) n2 = fmaf(bf2f(v[e]), bf2f(v[e]), n2);
+    }
+#pragma unroll
+    for (int w = 1; w < 16; w <<= 1) n2 += __shfl_xor(n2, w);
+    best = fmaxf(best, n2);
+  }
+  atomicMax(&mx, __float_as_uint(best));
+  __syncthreads();
+  if (threadIdx.x == 0) p.bound[(int64_t)bh * G + y] = sqrtf(__uint_as_float(mx));
+}
+
 template <int VPL>   // scores per lane: NKV <= 64 * VPL
-__global__ void __launch_bounds__(256) icsa_level3_select_kernel(Level3Params p) {
+__global__ void __launch_bounds__(256) icsa_level3_select_kernel(Level3Params p, int n_sel_wg) {
+  if ((int)blockIdx.x >= n_sel_wg) {
+    const int G = kc_bound_groups(p.NKV), u = blockIdx.x - n_sel_wg;
+    kc_bound(p, u / G, u % G, G);
+    return;
+  }
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + w;          // over BH * n_rows
   if (row >= (int64_t)p.BH * p.n_rows) return;
@@ -789,25 +741,29 @@ __global__ void __launch_bounds__(256) icsa_level3_select_kernel(Level3Params p)
 }
 
 hipError_t launch_level3(const Level3Params& p, hipStream_t stream) {
-  if (p.NKV > ICSA_MAX_NKV || p.top_k > p.NKV || p.top_k < 1) return hipErrorInvalidValue;
+  if (!p.given && (p.NKV > ICSA_MAX_NKV || p.top_k > p.NKV || p.top_k < 1)) return hipErrorInvalidValue;
   if (p.n_rows <= 0) return hipSuccess;
-  Split3Gemm g;
-  g.A = p.qsum; g.rows = p.rows; g.rows_stride = p.rows_stride; g.rows_offset = p.rows_offset;
-  g.a_rows = p.NQsrc; g.n_rows = p.n_rows; g.B = p.kc32; g.n_cols = p.NKV; g.C = p.scores;
-  g.NB = 0; g.S = 0; g.div = 1.f;
-  hipLaunchKernelGGL(icsa_split3_gemm_kernel<false>, dim3((p.n_rows + LG_ROWS - 1) / LG_ROWS, LG_SPLIT, p.BH),
-                     dim3(256), 0, stream, g);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int64_t rows = (int64_t)p.BH * p.n_rows;
-  const dim3 grid((unsigned)((rows + 3) / 4));
+  if (!p.given) {
+    Split3Gemm g;
+    g.A = p.qsum; g.rows = p.rows; g.rows_stride = p.rows_stride; g.rows_offset = p.rows_offset;
+    g.a_rows = p.NQsrc; g.n_rows = p.n_rows; g.B = p.kc32; g.n_cols = p.NKV; g.C = p.scores;
+    g.NB = 0; g.S = 0; g.div = 1.f; g.n_split = lg_split(p.n_rows, p.NKV, p.BH);
+    hipLaunchKernelGGL(icsa_split3_gemm_kernel<false>, dim3((p.n_rows + LG_ROWS - 1) / LG_ROWS, g.n_split, p.BH),
+                       dim3(256), 0, stream, g, VmeanParams{});
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  const int n_sel_wg = p.given ? 0 : (int)(((int64_t)p.BH * p.n_rows + 3) / 4);
+  const int n_wg = n_sel_wg + (p.bound ? p.BH * kc_bound_groups(p.NKV) : 0);
+  if (n_wg == 0) return hipSuccess;
+  const dim3 grid((unsigned)n_wg);
   if (p.NKV <= 256)
-    hipLaunchKernelGGL(icsa_level3_select_kernel<4>, grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(icsa_level3_select_kernel<4>, grid, dim3(256), 0, stream, p, n_sel_wg);
   else if (p.NKV <= 512)
-    hipLaunchKernelGGL(icsa_level3_select_kernel<8>, grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(icsa_level3_select_kernel<8>, grid, dim3(256), 0, stream, p, n_sel_wg);
   else if (p.NKV <= 1024)
-    hipLaunchKernelGGL(icsa_level3_select_kernel<16>, grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(icsa_level3_select_kernel<16>, grid, dim3(256), 0, stream, p, n_sel_wg);
   else
-    hipLaunchKernelGGL(icsa_level3_select_kernel<32>, grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(icsa_level3_select_kernel<32>, grid, dim3(256), 0, stream, p, n_sel_wg);
   return hipGetLastError();
 }

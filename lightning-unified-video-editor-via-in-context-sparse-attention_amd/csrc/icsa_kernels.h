@@ -19,11 +19,6 @@ struct PoolParams {
   int S[3], NB[3], NBp[3];   // per input: S tokens, NB = ceil(S / 64) blocks
 };
 hipError_t launch_pool(const PoolParams& p, hipStream_t stream);
-// V^T of a list of blocks only: block base + list[bh * stride + r], r < n, of x[vt_src],
-// stored as V^T block dst0 + r (the selected source blocks, transposed after the selection
-// into the columns that follow the target blocks)
-hipError_t launch_vt_blocks(const PoolParams& p, const int* list, int base, int stride, int n,
-                            int dst0, hipStream_t stream);
 
 // ---------------------------------------------------------------- stage 2 (compressed.hip)
 struct CompressedParams {
@@ -56,11 +51,12 @@ struct SelectParams {
 };
 hipError_t launch_select(const SelectParams& p, hipStream_t stream);
 
-struct NewKvSumsParams {
+// The new KV's tables, once the selection is known (newkv.hip): block sums and V^T.
+struct NewKvParams {
   const float* ksum;    // [BH, Nsrc, D] source block sums
   const float* vsum;
   const int* kvmap;     // [BH, NKV]  source block index (token start / 64) or -1
-  float* kc32;          // [BH, NKV, D]   fp32 sums of new-KV blocks
+  float* kc32;          // [BH, NKV, D]   fp32 sums of new-KV blocks (nullptr: no block sums at all)
   bf16* kc;             // [BH, NKVp, D]  bf16 sums (rows >= NKV zero)
   bf16* vct;            // [BH, D, NKVp]  bf16 sums of v transposed, kv_slot() order (nullptr: none)
   bf16* vc;             // [BH, NKVp, D]  bf16 sums of v, row-major (nullptr: none)
@@ -69,8 +65,12 @@ struct NewKvSumsParams {
   // token rows of k / v (dtype as given, rows >= S zero) instead of copied from ksum / vsum
   TokTensor k, v;
   int seg_a, seg_from, S, H;
+  // V^T of the selected source blocks: block sel_base + sel[bh * sel_stride + r], r < n_sel,
+  // of v goes to V^T block vt_dst0 + r (the columns that follow the target blocks)
+  const int* sel; int sel_stride, n_sel, sel_base, vt_dst0;
+  bf16* vt; int64_t vt_sb, vt_sh, vt_sd;
 };
-hipError_t launch_newkv_sums(const NewKvSumsParams& p, hipStream_t stream);
+hipError_t launch_newkv(const NewKvParams& p, hipStream_t stream);
 
 struct Level3Params {
   const float* qsum;    // [BH, NQsrc, D]
@@ -80,7 +80,13 @@ struct Level3Params {
   int* idx;             // [BH, n_rows, top_k]  ascending block indices
   float* scores;        // [BH, n_rows, NKV]  scratch
   int BH, NQsrc, n_rows, NKV, top_k;
+  int given;            // 1: idx holds the caller's lists (only the bound is computed)
+  // optional interval bound (SparseParams::kc_bound), not in `scores`: bound[bh * G + y] = max
+  // over the blocks j < NKV with (j / 16) % G == y of the L2 norm of the bf16 row kc[bh, j, :]
+  const bf16* kc; int NKVp;
+  float* bound;
 };
+__host__ __device__ inline int kc_bound_groups(int NKV) { return (NKV + 15) / 16 < 8 ? (NKV + 15) / 16 : 8; }
 hipError_t launch_level3(const Level3Params& p, hipStream_t stream);
 
 // ---------------------------------------------------------------- new-KV gather (gather.hip)
@@ -189,7 +195,7 @@ struct SparseParams {
   OutView out;
   float scale_log2;
   float* lse;                        // optional [BH, Sq]: m + log2(l + g_l) per query (log2 units)
-  // optional [BH, kc_bound_n] partial maxima of |KC_j| (launch_kc_bound): a workgroup whose
+  // optional [BH, kc_bound_n] partial maxima of |KC_j| (Level3Params::bound): a workgroup whose
   // rows all satisfy |q| max |KC_j| c / 64 < exact max skips the interval max pass
   const float* kc_bound; int kc_bound_n;
   // blocks per interval chunk of the reference (BN): the running max of the non-rescaled
@@ -197,11 +203,6 @@ struct SparseParams {
   int interval_bn;
 };
 hipError_t launch_sparse(const SparseParams& p, hipStream_t stream);
-// out[bh * G + y] = max over the new-KV blocks j < NKV with (j / 16) % G == y of the L2
-// norm of the bf16 row kc[bh, j, :] (fp32 arithmetic); G = min(8, cdiv(NKV, 16)) is
-// returned in *G (at most NKV, so BH * G floats fit wherever BH * NKV do)
-hipError_t launch_kc_bound(const bf16* kc, int BH, int NKV, int NKVp, float* out, int* G,
-                           hipStream_t stream);
 
 // ---------------------------------------------------------------- backward (sparse_bwd.hip)
 // Gradients of the sparse piecewise attention (triton_kernels.py:265-486, 541-598) without

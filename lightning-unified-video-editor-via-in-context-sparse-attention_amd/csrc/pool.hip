@@ -10,41 +10,14 @@
 //     backward 213 -> 198 us with the launches this saves)
 //   * optional bf16 copy     -> xb[i]    same strides as a contiguous [B, S, H, D]
 //   * optional V transposed  -> vt       [B, H, D, Sp] bf16, kv_slot() order, zero padded;
-//     with vt_limit only blocks n < vt_nblk (the pipeline's target blocks), and
-//     icsa_vt_blocks_kernel transposes a list of further blocks (the selected source
-//     blocks) once the selection is known
+//     with vt_limit only blocks n < vt_nblk (the pipeline's target blocks; newkv.hip
+//     transposes the selected source blocks once the selection is known)
 // Token rows at or beyond S read as zeros, so the partial last block sums only real tokens
 // and the transposed copy is zero for padding tokens.
 #include <algorithm>
 
 #include "icsa_kernels.h"
-
-// Raw storage of 8 consecutive elements of one row (one thread's share of a 64-token row).
-template <typename T> struct Raw8;
-template <> struct Raw8<bf16> {
-  bf16x8 v;
-  __device__ __forceinline__ void load(const bf16* p) { v = *reinterpret_cast<const bf16x8*>(p); }
-  __device__ __forceinline__ void zero() {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = (bf16)0.f;
-  }
-  __device__ __forceinline__ void to_f32(float o[8]) const {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = (float)v[e];
-  }
-};
-template <> struct Raw8<float> {
-  floatx4 a, b;
-  __device__ __forceinline__ void load(const float* p) {
-    a = *reinterpret_cast<const floatx4*>(p);
-    b = *reinterpret_cast<const floatx4*>(p + 4);
-  }
-  __device__ __forceinline__ void zero() { a = floatx4{0.f, 0.f, 0.f, 0.f}; b = a; }
-  __device__ __forceinline__ void to_f32(float o[8]) const {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { o[e] = a[e]; o[4 + e] = b[e]; }
-  }
-};
+#include "pool_rows.h"
 
 // Thread t covers chunk c = t % 16 (8 of the 128 dims) of rows g + 16 j, g = t / 16.
 template <typename T>
@@ -57,27 +30,6 @@ __device__ __forceinline__ void pool_load(const PoolParams& p, int i, int n, int
     const int tok = n * ICSA_BLOCK + g + 16 * j;
     if (tok < p.S[i]) r[j].load(base + (int64_t)tok * p.x[i].ss + 8 * c);
     else r[j].zero();
-  }
-}
-
-// V^T of block n from the staged rows vtile[token][d]: thread -> (d, half), 32 consecutive
-// slots of V^T row d, in kv_slot order
-__device__ __forceinline__ void vt_store(const PoolParams& p, int n, int b, int h,
-                                         const bf16 (*vtile)[ICSA_D + 8]) {
-  const int t = threadIdx.x;
-  const int d = t >> 1;
-  const int half = t & 1;
-  bf16* dst = p.vt + (int64_t)b * p.vt_sb + (int64_t)h * p.vt_sh + (int64_t)d * p.vt_sd
-              + (int64_t)n * ICSA_BLOCK + 32 * half;
-#pragma unroll
-  for (int q4 = 0; q4 < 4; ++q4) {
-    bf16x8 o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int slot = 32 * half + 8 * q4 + e;
-      o[e] = vtile[kv_slot(slot)][d];
-    }
-    *reinterpret_cast<bf16x8*>(dst + 8 * q4) = o;
   }
 }
 
@@ -122,7 +74,8 @@ __device__ __forceinline__ void pool_one(const PoolParams& p, int i, int n, int 
     if (p.sums[i] != nullptr) p.sums[i][(bh * p.NB[i] + n) * ICSA_D + t] = s;
     if (p.sb[i] != nullptr) p.sb[i][(bh * p.NBp[i] + n) * ICSA_D + t] = f2bf(s);
   }
-  if (want_vt) vt_store(p, n, b, h, vtile);
+  if (want_vt)
+    vt_store(p.vt + (int64_t)b * p.vt_sb + (int64_t)h * p.vt_sh + (int64_t)n * ICSA_BLOCK, p.vt_sd, vtile);
   __syncthreads();
 }
 
@@ -176,45 +129,5 @@ hipError_t launch_pool(const PoolParams& p, hipStream_t stream) {
 #undef ICSA_POOL_CASE
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
-}
-
-// V^T of listed blocks: one workgroup per (b*h, list entry r), stored as V^T block dst0 + r
-// (an entry outside [0, NB) stores a zero block, so no column keeps stale workspace data)
-template <typename T>
-__global__ void __launch_bounds__(256) icsa_vt_blocks_kernel(PoolParams p, const int* list, int base,
-                                                             int stride, int dst0) {
-  __shared__ bf16 vtile[ICSA_BLOCK][ICSA_D + 8];
-  const int bh = blockIdx.x, r = blockIdx.y;
-  const int b = bh / p.H, h = bh % p.H;
-  const int n = base + list[(int64_t)bh * stride + r];
-  const bool real = n >= 0 && n < p.NB[p.vt_src];  // uniform for the workgroup
-  Raw8<T> rows[4];
-  if (real) {
-    pool_load<T>(p, p.vt_src, n, b, h, rows);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) rows[j].zero();
-  }
-  const int c = threadIdx.x & 15, g = threadIdx.x >> 4;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    float v[8];
-    rows[j].to_f32(v);
-    *reinterpret_cast<bf16x8*>(&vtile[g + 16 * j][8 * c]) = pack8_bf16(v);
-  }
-  __syncthreads();
-  vt_store(p, dst0 + r, b, h, vtile);
-}
-
-hipError_t launch_vt_blocks(const PoolParams& p, const int* list, int base, int stride, int n,
-                            int dst0, hipStream_t stream) {
-  if (n <= 0 || p.B * p.H == 0) return hipSuccess;
-  if (!p.vt || !p.x[p.vt_src].p) return hipErrorInvalidValue;
-  dim3 grid(p.B * p.H, n);
-  if (p.x[p.vt_src].dtype == ICSA_DT_F32)
-    hipLaunchKernelGGL(icsa_vt_blocks_kernel<float>, grid, dim3(256), 0, stream, p, list, base, stride, dst0);
-  else
-    hipLaunchKernelGGL(icsa_vt_blocks_kernel<bf16>, grid, dim3(256), 0, stream, p, list, base, stride, dst0);
   return hipGetLastError();
 }

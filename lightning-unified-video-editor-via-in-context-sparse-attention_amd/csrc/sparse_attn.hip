@@ -19,7 +19,7 @@
 // non-rescaled g terms straight into the output accumulator.  That costs one extra
 // Q.KC product per chunk and frees the separate g accumulator (64 registers), which is
 // what lets two waves share each SIMD.  Pass 1 is skipped when a Cauchy-Schwarz bound,
-// |q| max_j |KC_j| c / 64 (max_j |KC_j| per head from icsa_kc_bound_kernel), lies below the
+// |q| max_j |KC_j| c / 64 (max_j |KC_j| per head, computed beside the level-3 selection), lies below the
 // exact max of every row of the workgroup: then the running max cannot rise and
 // m_final = m_exact, bit for bit.
 //
@@ -596,43 +596,6 @@ icsa_sparse_kernel(SparseParams p) {
     const float* oc = p.out_c ? p.out_c + ((int64_t)bh * p.nb_q + qblk) * ICSA_D : nullptr;
     store_rows(o_lds, p.out, b, h, qtok0, q_valid, oc, p.alpha);
   }
-}
-
-// Workgroup (b, h, y) takes the rows j = 16 (y + G i) + r, r = 0 .. 15 (i = 0, 1, ...): 16
-// lanes per row, one 16-byte chunk each, the squared norm summed over the 16 lanes with
-// lane shuffles; the workgroup maximum goes through an LDS atomic (non-negative floats
-// order like their bit patterns).
-__global__ void __launch_bounds__(256) icsa_kc_bound_kernel(const bf16* kc, int NKV, int NKVp, float* out) {
-  __shared__ unsigned mx;
-  const int bh = blockIdx.x, y = blockIdx.y, G = gridDim.y;
-  const int r = threadIdx.x >> 4, ch = threadIdx.x & 15;
-  if (threadIdx.x == 0) mx = 0u;
-  __syncthreads();
-  float best = 0.f;
-  for (int j0 = 16 * y; j0 < NKV; j0 += 16 * G) {
-    const int j = j0 + r;
-    float n2 = 0.f;
-    if (j < NKV) {
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(kc + ((int64_t)bh * NKVp + j) * ICSA_D + 8 * ch);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) n2 = fmaf(bf2f(v[e]), bf2f(v[e]), n2);
-    }
-#pragma unroll
-    for (int w = 1; w < 16; w <<= 1) n2 += __shfl_xor(n2, w);
-    best = fmaxf(best, n2);
-  }
-  atomicMax(&mx, __float_as_uint(best));
-  __syncthreads();
-  if (threadIdx.x == 0) out[(int64_t)bh * G + y] = sqrtf(__uint_as_float(mx));
-}
-
-hipError_t launch_kc_bound(const bf16* kc, int BH, int NKV, int NKVp, float* out, int* G,
-                           hipStream_t stream) {
-  const int groups = (NKV + 15) / 16;                 // 16-row groups
-  *G = groups < 8 ? groups : 8;
-  if (BH <= 0 || NKV <= 0) return hipSuccess;
-  hipLaunchKernelGGL(icsa_kc_bound_kernel, dim3(BH, *G), dim3(256), 0, stream, kc, NKV, NKVp, out);
-  return hipGetLastError();
 }
 
 hipError_t launch_sparse(const SparseParams& p, hipStream_t stream) {

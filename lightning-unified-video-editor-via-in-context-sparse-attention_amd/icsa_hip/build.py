@@ -18,7 +18,7 @@ CSRC_DIR = os.path.join(os.path.dirname(PKG_DIR), "csrc")
 BUILD_DIR = os.path.join(CSRC_DIR, "_build")
 LIB_PATH = os.path.join(PKG_DIR, "libicsa.so")
 
-SOURCES = ["pool.hip", "compressed.hip", "gather.hip", "flash_attn.hip", "sparse_attn.hip", "sparse_bwd.hip",
+SOURCES = ["pool.hip", "compressed.hip", "newkv.hip", "gather.hip", "flash_attn.hip", "sparse_attn.hip", "sparse_bwd.hip",
            "wan_qk.hip", "wan_block.hip", "api.hip"]
 
 HIP_FLAGS = [
