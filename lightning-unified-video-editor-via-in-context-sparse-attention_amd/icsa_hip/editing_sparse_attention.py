@@ -22,7 +22,7 @@ import torch
 
 from . import _lib
 from .hip_host import (BLOCK_M, IcsaArgumentError, _require, check_index_lists, dtype_code,
-                       inner_contiguous, ptr, stream_ptr)
+                       inner_contiguous, on_device, ptr, stream_ptr)
 
 
 class Backend:
@@ -90,12 +90,15 @@ def _editing_sparse_attention_hip(q, k, v, t_seq_len, alpha_2=1.0, SPARSITY_RATI
     for t in (q, k, v):
         dtype_code(t)
     L = _lib.lib()
-    sizes = derived_sizes(B, S, H, D, t_seq_len, SPARSITY_RATIO, srr, flat_ratio)
     offs = (ctypes.c_int64 * len(_lib.WS_SLOTS))()
     ws_bytes = L.icsa_editing_workspace_layout(B, S, H, D, t_seq_len, float(SPARSITY_RATIO),
                                                float(srr), float(flat_ratio), dtype_code(q),
                                                dtype_code(k), dtype_code(v),
                                                ctypes.cast(offs, ctypes.c_void_p))
+    # the sizes themselves are only looked at by the options below (and name a bad argument)
+    sizes = None
+    if ws_bytes < 0 or presummed is not None or inject or keep_workspace:
+        sizes = derived_sizes(B, S, H, D, t_seq_len, SPARSITY_RATIO, srr, flat_ratio)
     if ws_bytes < 0:
         raise _lib.IcsaError("icsa_editing_workspace_layout", int(ws_bytes))
     _require(not noalloc or (not keep_workspace and stage_events is None and presummed is None),
@@ -112,13 +115,12 @@ def _editing_sparse_attention_hip(q, k, v, t_seq_len, alpha_2=1.0, SPARSITY_RATI
         _require(q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16,
                  "presummed q / k must be bfloat16")
     a, a_scalar, a_dt, a_st = _alpha_view(alpha_2, B, S, H, D, q.device)
-    inject = inject or {}
     inj = {}
     # injected decisions (a testing hook): the kernels index q rows with `order`, source
     # blocks with `sel` and new-KV blocks with `l3`, so their ranges are checked here
     for name, shape, hi in (("sel", (B, H, sizes["topK"]), sizes["n_s"]),
                             ("order", (B, H, sizes["NB"]), sizes["NB"]),
-                            ("l3", (B, H, sizes["n_diffuse"], sizes["top_k"]), sizes["NKV"])):
+                            ("l3", (B, H, sizes["n_diffuse"], sizes["top_k"]), sizes["NKV"])) if inject else ():
         if inject.get(name) is not None:
             t = inject[name].to(device=q.device, dtype=torch.int32).contiguous()
             _require(tuple(t.shape) == shape, f"inject[{name!r}] must have shape {shape}")
@@ -138,14 +140,14 @@ def _editing_sparse_attention_hip(q, k, v, t_seq_len, alpha_2=1.0, SPARSITY_RATI
     if noalloc:
         fn = L.icsa_editing_sparse_attention_noalloc
         ws_args = []
-    with torch.cuda.device(q.device):     # the library launches on the current device
+    with on_device(q.device):
         rc = fn(
-            ptr(q), dtype_code(q), q.stride(0), q.stride(1), q.stride(2),
-            ptr(k), dtype_code(k), k.stride(0), k.stride(1), k.stride(2),
-            ptr(v), dtype_code(v), v.stride(0), v.stride(1), v.stride(2),
+            ptr(q), dtype_code(q), *q.stride()[:3],
+            ptr(k), dtype_code(k), *k.stride()[:3],
+            ptr(v), dtype_code(v), *v.stride()[:3],
             B, S, H, D, int(t_seq_len), float(SPARSITY_RATIO), float(srr), float(flat_ratio),
             ptr(a), a_dt, a_st[0], a_st[1], a_st[2], a_st[3], float(a_scalar),
-            ptr(out), dtype_code(out), out.stride(0), out.stride(1), out.stride(2),
+            ptr(out), dtype_code(out), *out.stride()[:3],
             ptr(inj.get("sel")), ptr(inj.get("order")), ptr(inj.get("l3")),
             *ws_args, stream_ptr(q.device), *ev_args)
     _lib.check(fn.__name__, rc)

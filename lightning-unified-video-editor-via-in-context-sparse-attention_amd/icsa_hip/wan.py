@@ -22,7 +22,7 @@ import torch.nn as nn
 
 from . import _lib
 from .editing_sparse_attention import Backend, _editing_sparse_attention_hip, derived_sizes
-from .hip_host import _require, dtype_code, ptr, stream_ptr
+from .hip_host import _require, dtype_code, on_device, ptr, stream_ptr
 
 _rope_cache: dict = {}
 
@@ -61,11 +61,15 @@ def rope_tables(freqs: torch.Tensor, device) -> tuple[torch.Tensor, torch.Tensor
     return hit[0], hit[1]
 
 
+def _grid(row) -> list:
+    """One row of grid sizes as ints (a tensor's row in one copy, not one an element)."""
+    return [int(x) for x in (row.tolist() if isinstance(row, torch.Tensor) else row)]
+
+
 def _grids(grid_sizes, source_video_grid_sizes, B) -> ctypes.Array:
     g = (ctypes.c_int32 * (6 * B))()
     for b in range(B):
-        t = [int(x) for x in grid_sizes[b]]
-        s = [int(x) for x in source_video_grid_sizes[b]]
+        t, s = _grid(grid_sizes[b]), _grid(source_video_grid_sizes[b])
         _require(len(t) == 3 and len(s) == 3, "grid sizes are (frames, rows, columns)")
         for a in range(3):
             g[6 * b + a] = t[a]
@@ -123,7 +127,7 @@ def wan_qk_prologue(yq: torch.Tensor, yk, norm_q_weight: torch.Tensor, norm_k_we
         a_args = [ptr(a), dtype_code(a), a.stride(0), a.stride(1)]
     ws_bytes = L.icsa_wan_qk_workspace_size(B, S)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):     # the library launches on the current device
+    with on_device(dev):
         rc = L.icsa_wan_qk_prologue(
             ptr(yq), ptr(yk), dtype_code(yq), yq.stride(0), yq.stride(1),
             ptr(wq), ptr(wk), float(eps),
@@ -131,7 +135,7 @@ def wan_qk_prologue(yq: torch.Tensor, yk, norm_q_weight: torch.Tensor, norm_k_we
             ctypes.cast(_grids(grid_sizes, source_video_grid_sizes, B), ctypes.c_void_p), int(TAG),
             *a_args,
             B, S, H, D,
-            ptr(q), ptr(k), q.stride(0), q.stride(1), q.stride(2),
+            ptr(q), ptr(k), *q.stride()[:3],
             ptr(qsum), ptr(ksum), ptr(gate),
             ptr(ws), ws_bytes, stream_ptr(dev))
     _lib.check("icsa_wan_qk_prologue", rc)
@@ -154,7 +158,7 @@ def wan_self_attention_core(yq, yk, yv, alpha_logit, norm_q_weight, norm_k_weigh
     q, k, qsum, ksum, gate = wan_qk_prologue(yq, yk, norm_q_weight, norm_k_weight, grid_sizes,
                                              source_video_grid_sizes, TAG, freqs, H,
                                              alpha_logit, eps)
-    f, h, w = (int(x) for x in grid_sizes[0])
+    f, h, w = _grid(grid_sizes[0])
     t_seq_len = f * h * w
     v = yv.reshape(B, S, H, D)
     alpha_2 = gate.view(B, S, 1, 1) if gate is not None else 0.0
@@ -200,7 +204,7 @@ def ln_modulate(x: torch.Tensor, shift=None, scale=None, weight=None, bias=None,
     else:
         _require(x_out is None, "x_out needs y")
     o = torch.empty(B, S, dim, dtype=torch.bfloat16, device=x.device) if out else None
-    with torch.cuda.device(x.device):     # the library launches on the current device
+    with on_device(x.device):
         rc = _lib.lib().icsa_wan_ln_modulate(
             ptr(x), dtype_code(x), x.stride(0), x.stride(1),
             ptr(y), y.stride(0) if y is not None else 0, y.stride(1) if y is not None else 0,
