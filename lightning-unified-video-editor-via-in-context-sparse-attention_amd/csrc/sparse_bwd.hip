@@ -134,18 +134,38 @@ __device__ __forceinline__ T uniform_word(const T* p) {
 // offset ^ (kk << 5) (the swizzle only flips chunk bits).
 __device__ __forceinline__ int bw_row_off(int row, int hl) { return rt_off(row, hl) * 2; }
 
-// One wave's quarter of a tile: rows 16 w .. 16 w + 15.  Rows >= valid lie outside the buffer
-// range and land nothing: bw_fill_rows zeroes them once the tile's loads have completed.
-__device__ __forceinline__ void bw_dma_rows(unsigned char* tile, const bf16* base, int64_t rs, int wave,
-                                            int lane, int valid = ICSA_BLOCK) {
-  const u32x4 rs4 = dma_rsrc(base, valid > 0 ? ((int64_t)(valid - 1) * rs + ICSA_D) * 2 : 0);
-  const unsigned dst = lds_u32(tile + wave * 4096);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = 16 * wave + 4 * i + (lane >> 4);
-    lds_dma16(dst + 1024 * i, (int)(r * rs * 2) + (((lane & 15) ^ rt_swz(r)) << 4), rs4);
+// Row tiles of one tensor of a head: block j's 64 rows.  What a tile needs is kept to a product
+// and an add, and one select for the partial last block (rows past it lie outside the buffer
+// range and land nothing: bw_fill_rows zeroes them once the tile's loads have completed): with the
+// byte count worked out for each tile and generic LDS pointers, a step's two tiles took 145
+// instructions and about 800 of its 3,400 cycles; now 91 (40 heads, 7,800 tokens: query-major launch
+// 352 -> 341 us, exact key-major 368 -> 358 us at the best clock, forward and backward 993 -> 982).
+struct BwSrc {
+  unsigned long long base;
+  long long block_bytes;
+  int row_bytes, partial, n_partial;     // partial: index of the last block if it is not whole
+  __device__ __forceinline__ BwSrc(const bf16* head, int64_t stride, int rows)
+      : base((unsigned long long)head), block_bytes(stride * 2 * ICSA_BLOCK), row_bytes((int)(stride * 2)),
+        partial(rows % ICSA_BLOCK ? rows / ICSA_BLOCK : -1) {
+    const int64_t n = ((int64_t)(rows % ICSA_BLOCK - 1) * stride + ICSA_D) * 2;
+    n_partial = n > 0x7fffffffLL ? 0x7fffffff : (int)n;
   }
-}
+  // one wave's quarter of block j's tile (rows 16 w .. 16 w + 15) to LDS address `tile`
+  __device__ __forceinline__ void load(unsigned tile, int j, int wave, int lane) const {
+    const unsigned long long a = base + (unsigned long long)(unsigned)j * (unsigned long long)block_bytes;
+    u32x4 rs;
+    rs[0] = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a);
+    rs[1] = (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)(a >> 32) & 0xffffu));
+    rs[2] = (unsigned)__builtin_amdgcn_readfirstlane(j == partial ? n_partial : 0x7fffffff);
+    rs[3] = 0x00020000u;
+    const unsigned dst = tile + 4096u * wave;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * wave + 4 * i + (lane >> 4);
+      lds_dma16(dst + 1024 * i, r * row_bytes + (((lane & 15) ^ rt_swz(r)) << 4), rs);
+    }
+  }
+};
 
 // Zero this wave's rows >= valid of a row tile (the bytes its DMA lanes would have landed).
 __device__ __forceinline__ void bw_fill_rows(unsigned char* tile, int valid, int wave, int lane) {
@@ -263,17 +283,18 @@ __device__ __forceinline__ void bw_dq(const SparseBwdParams& p, unsigned char* s
   const int done = -1 - p.nc;
   // real key rows of an exact step (the last block of a ragged TKV is partial)
   auto key_rows = [&](int j) -> int { return j < 0 ? ICSA_BLOCK : min(ICSA_BLOCK, p.TKV - j * ICSA_BLOCK); };
+  const BwSrc k_src(kb, p.k_st, p.TKV), v_src(vb, p.v_st, p.TKV);
+  const BwSrc kc_src(kcb, ICSA_D, p.NKVp), vc_src(vcb, ICSA_D, p.NKVp);
+  const unsigned lds = lds_u32(smem_q);
   // buffer u: K rows at 2 u tiles, V rows at 2 u + 1
   auto issue = [&](int t, int j) {
-    unsigned char* kt = smem_q + (t & 1) * 2 * K_TILE_BYTES;
+    const unsigned kt = lds + (t & 1) * 2 * K_TILE_BYTES;
     if (j >= 0) {
-      const int valid = key_rows(j);
-      bw_dma_rows(kt, kb + (int64_t)j * ICSA_BLOCK * p.k_st, p.k_st, wave, lane, valid);
-      bw_dma_rows(kt + K_TILE_BYTES, vb + (int64_t)j * ICSA_BLOCK * p.v_st, p.v_st, wave, lane, valid);
+      k_src.load(kt, j, wave, lane);
+      v_src.load(kt + K_TILE_BYTES, j, wave, lane);
     } else {
-      const int ch = -1 - j;
-      bw_dma_rows(kt, kcb + (int64_t)ch * ICSA_BLOCK * ICSA_D, ICSA_D, wave, lane);
-      bw_dma_rows(kt + K_TILE_BYTES, vcb + (int64_t)ch * ICSA_BLOCK * ICSA_D, ICSA_D, wave, lane);
+      kc_src.load(kt, -1 - j, wave, lane);
+      vc_src.load(kt + K_TILE_BYTES, -1 - j, wave, lane);
     }
   };
   int j = next();                                      // at least one chunk
@@ -422,14 +443,15 @@ __device__ __forceinline__ void bw_dkv(const SparseBwdParams& p, unsigned char* 
     cur &= cur - 1ull;
     return i;
   };
+  const BwSrc q_src(qb0, p.q_st, p.TQ), do_src(dob0, p.do_st, p.TQ);
+  const unsigned lds = lds_u32(smem_dyn);
   auto issue = [&](int n, int i) {
-    const int valid = min(ICSA_BLOCK, p.TQ - i * ICSA_BLOCK);   // ragged TQ: partial last block
-    unsigned char* buf = smem_dyn + (n & 1) * BWKV_BUF_BYTES;
-    bw_dma_rows(buf, qb0 + (int64_t)i * ICSA_BLOCK * p.q_st, p.q_st, wave, lane, valid);
-    bw_dma_rows(buf + K_TILE_BYTES, dob0 + (int64_t)i * ICSA_BLOCK * p.do_st, p.do_st, wave, lane, valid);
+    const unsigned buf = lds + (n & 1) * BWKV_BUF_BYTES;
+    q_src.load(buf, i, wave, lane);
+    do_src.load(buf + K_TILE_BYTES, i, wave, lane);
     if (wave < 2)
-      lds_dma4(lds_u32(buf + 2 * K_TILE_BYTES + wave * 256), lane * 4,
-               dma_rsrc(rowvec + (int64_t)i * ICSA_BLOCK, valid * 4));
+      lds_dma4(buf + 2 * K_TILE_BYTES + wave * 256, lane * 4,
+               dma_rsrc(rowvec + (int64_t)i * ICSA_BLOCK, min(ICSA_BLOCK, p.TQ - i * ICSA_BLOCK) * 4));
   };
   // Everything the prologue reads is requested before any of it is waited for: the first
   // tiles, the interval partials (exact part), K and V.
