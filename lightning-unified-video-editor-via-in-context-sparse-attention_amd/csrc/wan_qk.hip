@@ -23,6 +23,17 @@
 // then the h axis and the w axis for D/2/3 pairs each (rope_apply's freqs.split).
 #include "icsa_kernels.h"
 
+// The alpha gate of token s: bf16 arithmetic of the reference, sigmoid, - 0.5 and * 0.5 each
+// round to bf16
+__device__ __forceinline__ void wan_gate(const WanRmsParams& p, int b, int s) {
+  const int64_t off = (int64_t)b * p.alpha_logit.sb + (int64_t)s * p.alpha_logit.ss;
+  const float a = p.alpha_logit.dtype == ICSA_DT_F32 ? reinterpret_cast<const float*>(p.alpha_logit.p)[off]
+                                                     : (float)reinterpret_cast<const bf16*>(p.alpha_logit.p)[off];
+  const float sg = (float)(bf16)(1.f / (1.f + expf(-a)));
+  const float g = (float)(bf16)(sg - 0.5f) * 0.5f;
+  p.gate[(int64_t)b * p.S + s] = g;
+}
+
 // ---- per-token RMS factors (+ alpha gate): one wave per token ----
 __global__ void __launch_bounds__(256) icsa_wan_rms_kernel(WanRmsParams p) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -47,15 +58,7 @@ __global__ void __launch_bounds__(256) icsa_wan_rms_kernel(WanRmsParams p) {
     ss = wave_sum(ss);
     if (lane == 0) p.rinv[i][tok_all] = 1.f / sqrtf(ss / (float)dim + p.eps);
   }
-  if (p.alpha_logit.p != nullptr && lane == 0) {
-    const int64_t off = (int64_t)b * p.alpha_logit.sb + (int64_t)s * p.alpha_logit.ss;
-    const float a = p.alpha_logit.dtype == ICSA_DT_F32 ? reinterpret_cast<const float*>(p.alpha_logit.p)[off]
-                                                       : (float)reinterpret_cast<const bf16*>(p.alpha_logit.p)[off];
-    // bf16 arithmetic of the reference: sigmoid, - 0.5 and * 0.5 each round to bf16
-    const float sg = (float)(bf16)(1.f / (1.f + expf(-a)));
-    const float g = (float)(bf16)(sg - 0.5f) * 0.5f;
-    p.gate[tok_all] = g;
-  }
+  if (p.alpha_logit.p != nullptr && lane == 0) wan_gate(p, b, s);
 }
 
 // RoPE position of token tok on axis a (0: frames, 1: height, 2: width); -1: not rotated
@@ -202,7 +205,145 @@ __global__ void __launch_bounds__(256) icsa_wan_qk_kernel(WanQkParams p) {
   }
 }
 
+// ---- the same in one pass over the projections (bf16, H <= 40) ----
+// The two kernels above read y twice, 104 of 345 us at 40 heads, 28,080 tokens.  Here a wave holds
+// whole rows: four of them (64 lanes x NCH chunks of 8 dims each), so the row's RMS needs no
+// other wave, and 40 KB a wave are in flight.  Workgroup = 4 waves = one 64-token block of q or
+// k, in 4 rounds: wave w takes rows 4 round + w + 16 j, j = 0 .. 3, which are the rows that the
+// thread group 4 round + w of icsa_wan_qk_kernel takes, so all sums run in the same order
+// and the results are the same bits.  A chunk's registers take the next round's load as soon
+// as it is stored.  The block sums go through LDS chunk by chunk (512 dims, two buffers, one
+// barrier each).  40 heads, 28,080 tokens: 352 -> 281 us.  Few blocks leave most CUs idle for four
+// rounds: this kernel takes over from WQ_MIN_BLOCKS 64-token blocks of one head (q and k both
+// counted).  Measured, two passes / one: 40 heads 93 / 109 us at 7,840 such blocks, 124 / 124 at
+// 10,240, 190 / 160 at 15,600, 339 / 281 at 31,200; 12 heads 59 / 71 at 6,144, 113 / 109 at 9,360,
+// 146 / 117 at 12,288.
+#define WQ_MIN_BLOCKS 12000
+#define WQ_MAX_CH 10
+
+template <int NCH>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+icsa_wan_qk_rows_kernel(WanRmsParams rp, WanQkParams p) {
+  __shared__ __attribute__((aligned(16))) float w_l[512 * NCH];
+  __shared__ __attribute__((aligned(16))) float run_l[512 * NCH];    // block sums of the rounds so far
+  __shared__ __attribute__((aligned(16))) float red[2][4][512];
+  __shared__ __attribute__((aligned(16))) float rope_l[4][4][2][ICSA_D / 2];   // [wave][row][cos, sin][pair]
+  const int n = blockIdx.x, i = blockIdx.y, b = blockIdx.z;
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int c = lane & 15, n_chunk = 16 * p.H, dim = p.H * ICSA_D;
+  const bf16* y = reinterpret_cast<const bf16*>(p.y[i].p) + (int64_t)b * p.y[i].sb;
+  bf16* out = reinterpret_cast<bf16*>(p.out[i].p) + (int64_t)b * p.out[i].sb;
+  const int64_t o_ss = p.out[i].ss, o_sh4 = 4 * p.out[i].sh;
+  const int64_t y_ss = p.y[i].ss;
+  bf16x8 raw[4][NCH];
+  auto row_token = [&](int round, int j) -> int { return n * ICSA_BLOCK + 4 * round + w + 16 * j; };
+  auto load = [&](int round, int j, int u, unsigned ln) {
+    const int tok = row_token(round, j);
+    if (tok < p.S && (int)ln + 64 * u < n_chunk)
+      raw[j][u] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(y + (int64_t)tok * y_ss + 512 * u) +
+                                                   16u * ln);
+    else
+      raw[j][u] = bf16x8{};
+  };
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) load(0, j, u, lane);
+  if (i == 0 && rp.alpha_logit.p != nullptr && t < ICSA_BLOCK && n * ICSA_BLOCK + t < p.S)
+    wan_gate(rp, b, n * ICSA_BLOCK + t);
+  for (int d = t; d < 512 * NCH; d += 256) w_l[d] = d < dim ? p.w[i][d] : 0.f;
+  __syncthreads();
+  const int npair = ICSA_D / 2, n_hw = npair / 3, n_f = npair - 2 * n_hw;
+  const int axis = lane < n_f ? 0 : (lane < n_f + n_hw ? 1 : 2);       // of pair `lane`
+  const bool want_sums = p.sums[i] != nullptr;
+  int buf = 0;
+#pragma unroll 1
+  for (int round = 0; round < 4; ++round) {
+    // lane values that every chunk's addresses and masks derive from: not to be hoisted out of
+    // the loop for all chunks at once, the rows take 160 registers
+    int ln = lane;
+    int64_t o_lane = (lane >> 4) * p.out[i].sh + 8 * c;
+    asm volatile("" : "+v"(ln), "+v"(o_lane));
+    float rr[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float ss = 0.f;
+#pragma unroll
+      for (int u = 0; u < NCH; ++u)
+        if (ln + 64 * u < n_chunk) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ss = fmaf((float)raw[j][u][e], (float)raw[j][u][e], ss);
+        }
+#pragma unroll
+      for (int u = 0; u < NCH; ++u) asm volatile("" : "+v"(raw[j][u]));   // the fp32 forms are not kept
+      ss = wave_sum(ss);
+      rr[j] = 1.f / sqrtf(ss / (float)dim + rp.eps);
+      int pos[3];
+      rope_pos(p, b, row_token(round, j), pos);
+      const int ps = pos[axis];
+      rope_l[w][j][0][lane] = ps >= 0 ? p.rope_cos[(int64_t)ps * npair + lane] : 1.f;
+      rope_l[w][j][1][lane] = ps >= 0 ? p.rope_sin[(int64_t)ps * npair + lane] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) {
+      const bool on = ln + 64 * u < n_chunk;
+      const floatx4 w0 = *reinterpret_cast<const floatx4*>(&w_l[512 * u + 8 * lane]);
+      const floatx4 w1 = *reinterpret_cast<const floatx4*>(&w_l[512 * u + 8 * lane + 4]);
+      float acc[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int tok = row_token(round, j);
+        if (tok < p.S) {                               // uniform for the wave
+          const floatx4 c4 = *reinterpret_cast<const floatx4*>(&rope_l[w][j][0][4 * c]);
+          const floatx4 s4 = *reinterpret_cast<const floatx4*>(&rope_l[w][j][1][4 * c]);
+          float m[8], o[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            m[e] = (float)(bf16)((float)raw[j][u][e] * rr[j]) * (e < 4 ? w0[e] : w1[e - 4]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            o[2 * e] = fmaf(m[2 * e], c4[e], -m[2 * e + 1] * s4[e]);
+            o[2 * e + 1] = fmaf(m[2 * e], s4[e], m[2 * e + 1] * c4[e]);
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] += o[e];
+          if (on) *reinterpret_cast<bf16x8*>(out + (int64_t)tok * o_ss + u * o_sh4 + o_lane) = pack8_bf16(o);
+        }
+        if (round < 3) load(round + 1, j, u, ln);
+        __builtin_amdgcn_sched_barrier(0);             // one row's values at a time
+      }
+      if (want_sums) {
+        *reinterpret_cast<floatx4*>(&red[buf][w][8 * lane]) = floatx4{acc[0], acc[1], acc[2], acc[3]};
+        *reinterpret_cast<floatx4*>(&red[buf][w][8 * lane + 4]) = floatx4{acc[4], acc[5], acc[6], acc[7]};
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // loads stay in flight
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          const int d = t + 256 * x, gd = 512 * u + d;
+          float s = round == 0 ? 0.f : run_l[gd];
+#pragma unroll
+          for (int g = 0; g < 4; ++g) s += red[buf][g][d];
+          if (round < 3) run_l[gd] = s;
+          else if (gd < dim)
+            p.sums[i][(((int64_t)b * p.H + gd / ICSA_D) * p.NB + n) * ICSA_D + gd % ICSA_D] = s;
+        }
+        buf ^= 1;
+      }
+    }
+  }
+}
+
 hipError_t launch_wan_qk(const WanRmsParams& rp, const WanQkParams& qp, hipStream_t stream) {
+  const int nt = qp.y[1].p != nullptr ? 2 : 1;
+  if (qp.y[0].dtype != ICSA_DT_F32 && qp.H <= 4 * WQ_MAX_CH && (int64_t)qp.NB * nt * qp.B * qp.H >= WQ_MIN_BLOCKS) {
+    const dim3 rows_grid(qp.NB, nt, qp.B);
+    if (qp.H <= 12) hipLaunchKernelGGL(icsa_wan_qk_rows_kernel<3>, rows_grid, dim3(256), 0, stream, rp, qp);
+    else if (qp.H <= 20) hipLaunchKernelGGL(icsa_wan_qk_rows_kernel<5>, rows_grid, dim3(256), 0, stream, rp, qp);
+    else hipLaunchKernelGGL(icsa_wan_qk_rows_kernel<WQ_MAX_CH>, rows_grid, dim3(256), 0, stream, rp, qp);
+    return hipGetLastError();
+  }
   const int64_t ntok = (int64_t)rp.B * rp.S;
   hipLaunchKernelGGL(icsa_wan_rms_kernel, dim3((unsigned)((ntok + 3) / 4)), dim3(256), 0, stream, rp);
   hipError_t e = hipGetLastError();
