@@ -93,11 +93,11 @@ enum icsa_ws_slot {
   ICSA_WS_COLP,       /* f32 [B*H, ceil(n_t/64), n_s] source-column mass per target strip */
   ICSA_WS_L3S,        /* f32 [B*H, n_diffuse, NKV] level-3 block scores (scratch;    */
                       /* before them, the compressed stage's split value means,      */
-                      /* bf16 [B*H, 2, D, ceil(NB/64)*64]; sized for the larger),    */
-                      /* then the interval bound, f32 [B*H, min(8, ceil(NKV/16))]    */
+                      /* bf16 [B*H, 2, D, ceil(NB/64)*64]; sized for the larger)     */
   ICSA_WS_RSTAT,      /* f32 [B*H, NB, 2]   row max and 1 / row sum of the compressed softmax */
-  ICSA_WS_FLASHP,     /* f32 partials of the peaked blocks whose keys are split (O, max, sum; */
-                      /* a workspace that ends before this slot is accepted: nothing is split) */
+  ICSA_WS_FLASHP,     /* f32 interval bound [B*H, min(8, ceil(NKV/16))], then the partials */
+                      /* of the peaked blocks whose keys are split (O, max, sum); a workspace */
+                      /* that ends before this slot is accepted: no bound, nothing is split */
   ICSA_WS_COUNT
 };
 

@@ -96,9 +96,8 @@ struct Layout {
 // then the topK selected source blocks (tile j at columns 64 j .. 64 j + 63)
 int64_t vt_columns(const Sizes& z, int t) { return ((int64_t)ceil_div(t, ICSA_BLOCK) + z.topK) * ICSA_BLOCK; }
 
-int64_t l3_bound_off(int BH, const Sizes& z) {
-  return align256(std::max((int64_t)BH * std::max(z.n_diffuse, 1) * z.NKV * 4, compressed_vmt_bytes(BH, z.NB)));
-}
+// bytes of the interval bound, at the head of the optional last slot
+int64_t l3_bound_bytes(int BH, const Sizes& z) { return align256((int64_t)BH * kc_bound_groups(z.NKV) * 4); }
 
 Layout editing_layout(int B, int S, int H, const Sizes& z, int t, int q_dtype, int k_dtype, int v_dtype) {
   const int64_t BH = (int64_t)B * H;
@@ -125,11 +124,11 @@ Layout editing_layout(int B, int S, int H, const Sizes& z, int t, int q_dtype, i
   sz[ICSA_WS_L3] = BH * std::max(z.n_diffuse, 1) * z.top_k * 4;
   sz[ICSA_WS_VC] = unaligned ? BH * z.NKVp * D * 2 : 0;
   sz[ICSA_WS_COLP] = BH * ceil_div(z.n_t, ICSA_BLOCK) * std::max(z.n_s, 1) * 4;
-  // the level-3 scores, and before them the compressed stage's split value means; then the
-  // interval bound
-  sz[ICSA_WS_L3S] = l3_bound_off((int)BH, z) + BH * kc_bound_groups(z.NKV) * 4;
+  // the level-3 scores, and before them the compressed stage's split value means
+  sz[ICSA_WS_L3S] = std::max(BH * std::max(z.n_diffuse, 1) * z.NKV * 4, compressed_vmt_bytes((int)BH, z.NB));
   sz[ICSA_WS_RSTAT] = BH * z.NB * 2 * 4;
-  sz[ICSA_WS_FLASHP] = flash_plan(flash_items((int)BH, z.n_peaked), ceil_div(t, ICSA_BLOCK) + z.topK, true).part_bytes;
+  sz[ICSA_WS_FLASHP] = l3_bound_bytes((int)BH, z) +
+                       flash_plan(flash_items((int)BH, z.n_peaked), ceil_div(t, ICSA_BLOCK) + z.topK, true).part_bytes;
   Layout L;
   int64_t o = 0;
   for (int i = 0; i < ICSA_WS_COUNT; ++i) {
@@ -255,7 +254,8 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
   if (z.NKV > 2048 || z.top_k > 512)
     return fail(ICSA_EUNSUPPORTED, "NKV=%d / top_k=%d exceed limits (2048 / 512)", z.NKV, z.top_k);
   const Layout L = editing_layout(B, S, H, z, t_seq_len, q_dtype, k_dtype, v_dtype);
-  // the last slot may be missing: the peaked blocks then run without being split
+  // the last slot may be missing: the peaked blocks then run without being split, and the sparse
+  // kernel without the bound that spares it the interval max pass (the same bits)
   if (workspace_bytes < L.off[ICSA_WS_FLASHP])
     return fail(ICSA_EWORKSPACE, "workspace %lld bytes < required %lld", (long long)workspace_bytes,
                 (long long)L.total);
@@ -363,7 +363,8 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
 
   // ---- level-3 selection for the diffuse blocks ----
   int32_t* l3 = reinterpret_cast<int32_t*>(WS(ICSA_WS_L3));
-  float* bound = reinterpret_cast<float*>(WS(ICSA_WS_L3S) + l3_bound_off(BH, z));
+  const int64_t bound_bytes = l3_bound_bytes(BH, z), spare = workspace_bytes - L.off[ICSA_WS_FLASHP];
+  float* bound = interval_skip_enabled() && spare >= bound_bytes ? reinterpret_cast<float*>(WS(ICSA_WS_FLASHP)) : nullptr;
   if (z.n_diffuse > 0) {
     if (inject_l3)
       ICSA_HIP_TRY(hipMemcpyAsync(l3, inject_l3, (size_t)BH * z.n_diffuse * z.top_k * 4,
@@ -373,7 +374,7 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
     lp.kc32 = np.kc32; lp.idx = l3; lp.scores = reinterpret_cast<float*>(WS(ICSA_WS_L3S));
     lp.BH = BH; lp.NQsrc = z.NB; lp.n_rows = z.n_diffuse; lp.NKV = z.NKV; lp.top_k = z.top_k;
     lp.given = inject_l3 ? 1 : 0;
-    lp.kc = np.kc; lp.NKVp = z.NKVp; lp.bound = interval_skip_enabled() ? bound : nullptr;
+    lp.kc = np.kc; lp.NKVp = z.NKVp; lp.bound = bound;
     ICSA_HIP_TRY(launch_level3(lp, stream), "level-3 top-k");
   }
 
@@ -404,7 +405,7 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
     s.out_c = cp.out_c; s.nb_q = z.NB;
     s.alpha = av; s.out = ov; s.scale_log2 = scale_log2; s.lse = nullptr;
     s.mask_tail = 0;                   // zero-padded new KV attended with logit 0 (TileLang)
-    s.kc_bound = interval_skip_enabled() ? bound : nullptr;
+    s.kc_bound = bound;
     s.kc_bound_n = kc_bound_groups(z.NKV);
     ICSA_HIP_TRY(launch_sparse(s, stream), "sparse attention");
   }
@@ -422,8 +423,8 @@ int editing_impl(ICSA_EDITING_ARGS, void* const* stage_events, const float* qsum
     f.sel = sel; f.sel_stride = std::max(z.topK, 1); f.n_sel = z.topK; f.sel_base = z.n_t;
     f.out_c = cp.out_c; f.nb_q = z.NB;
     f.alpha = av; f.out = ov; f.scale_log2 = scale_log2;
-    f.part = reinterpret_cast<float*>(WS(ICSA_WS_FLASHP));
-    f.part_bytes = workspace_bytes - L.off[ICSA_WS_FLASHP];
+    f.part = reinterpret_cast<float*>(WS(ICSA_WS_FLASHP) + bound_bytes);
+    f.part_bytes = std::max<int64_t>(0, spare - bound_bytes);
     ICSA_HIP_TRY(launch_flash(f, stream), "flash attention");
   }
   ICSA_HIP_TRY(mark(ICSA_STAGE_FLASH), "event");
