@@ -107,19 +107,29 @@ __device__ __forceinline__ void newkv_straddle(const NewKvParams& p, int bh, int
     const int tokB = map[j] >= 0 ? ICSA_BLOCK * map[j] - a : -1;    // token of row r >= a: tokB + r
     const TK* kb = reinterpret_cast<const TK*>(p.k.p) + (int64_t)b * p.k.sb + (int64_t)h * p.k.sh;
     const TV* vb = reinterpret_cast<const TV*>(p.v.p) + (int64_t)b * p.v.sb + (int64_t)h * p.v.sh;
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
+    Raw8<TK> kr[8];
+    Raw8<TV> vr[8];
+    auto token = [&](int m) -> int {
       const int r = g + 8 * m;
       const int tok = r < a ? (tokA < 0 ? -1 : tokA + r) : (tokB < 0 ? -1 : tokB + r);
-      if (tok >= 0 && tok < p.S) {
-        float x[8];
-        load8_f32(kb + (int64_t)tok * p.k.ss + 8 * c, x);
+      return tok < p.S ? tok : -1;
+    };
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ks[e] += x[e];
-        load8_f32(vb + (int64_t)tok * p.v.ss + 8 * c, x);
+    for (int m = 0; m < 8; ++m) {
+      const int tok = max(token(m), 0);
+      kr[m].load(kb + (int64_t)tok * p.k.ss + 8 * c);
+      vr[m].load(vb + (int64_t)tok * p.v.ss + 8 * c);
+    }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) vs[e] += x[e];
-      }
+    for (int m = 0; m < 8; ++m) {
+      const bool real = token(m) >= 0;
+      float x[8];
+      kr[m].to_f32(x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ks[e] += real ? x[e] : 0.f;
+      vr[m].to_f32(x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vs[e] += real ? x[e] : 0.f;
     }
   }
 #pragma unroll
