@@ -693,12 +693,14 @@ __global__ void __launch_bounds__(256) icsa_level3_select_kernel(Level3Params p,
   if (row >= (int64_t)p.BH * p.n_rows) return;
   const int NKV = p.NKV, k = p.top_k;
   const float* srow = p.scores + row * NKV;
+  // unconditional loads from a clamped place: a condition around each made VPL branches, each
+  // waiting for the load before it (5 heads, 1,024 blocks 13.5 -> 11.5 us, 40 heads 34.4 -> 31.3)
+  float score[VPL];
+#pragma unroll
+  for (int u = 0; u < VPL; ++u) score[u] = srow[min(lane + 64 * u, NKV - 1)];
   uint32_t key[VPL];
 #pragma unroll
-  for (int u = 0; u < VPL; ++u) {
-    const int j = lane + 64 * u;
-    key[u] = j < NKV ? f2key(srow[j]) : 0u;         // 0 is below every real key
-  }
+  for (int u = 0; u < VPL; ++u) key[u] = lane + 64 * u < NKV ? f2key(score[u]) : 0u;   // 0 is below every real key
   const int nu = (NKV + 63) / 64;
   const uint32_t lo = kth_largest_key<VPL>(key, k, nu);
   int cgt = 0;
