@@ -22,7 +22,7 @@
 // heads) unchanged at 20.0 ms.  The rate is then about 1.23 PFLOP/s at every size that
 // fills the chip, the engine clock under this load being 1.7-1.9 GHz; with 8 tiles an item,
 // timing copies without the output stores and without the Q loads take 693 and 755 us (both:
-// 641 us), so what is left there is mostly the first tiles' second pass and the stores.
+// 641 us).
 //
 // Workgroup = 8 waves = an item's query blocks (wave w: block w/2, rows 32*(w%2)..+31),
 // all sharing each K / V^T tile.  The waves form two groups, G0 = waves 0-3 and G1 = waves
@@ -41,13 +41,15 @@
 // once, the tile start is the scalar base of a buffer resource whose range covers only key
 // rows below Sk, and every LDS offset is hoisted out of the loop.
 //
-// Softmax state: probabilities are taken relative to a reference max m_ref, computed first
-// and checked afterwards: only when a lane's partial sum of the tile exceeds 2^64 (or is NaN,
-// as against the initial m_ref = -inf) is the row max of the tile taken, the reference
-// raised, O / l rescaled and the tile recomputed.  In the common case no per-tile max
-// reduction precedes the exponentials.  Exact in real arithmetic.
+// Softmax state: probabilities are taken relative to a reference max m_ref.  A segment starts
+// without one (its rows are other queries, maybe another head's) and takes its first tile's
+// row max, before any exponential.  From then on the probabilities come first and are checked
+// afterwards: only when a lane's partial sum of the tile exceeds 2^64 (or is NaN) is the row max
+// of the tile taken, the reference raised, O / l rescaled and the tile recomputed.  In the
+// common case no per-tile max reduction precedes the exponentials.  Exact in real arithmetic.
+// (The first tile by that check as well, two passes of exponentials: 8 tiles an item, forward
+// 811-823 us a call against 789-806.)
 #include <algorithm>
-
 
 #include "attn_tile.h"
 #include "icsa_kernels.h"
@@ -388,7 +390,7 @@ icsa_flash_kernel(FlashParams p) {
   // SOFT(k): mask, P(k) against the reference max, and -- only when some probability of the
   // tile left the allowed range -- a rescale to the tile's row max and a second pass.  The
   // wave's DMA segments go out one at a time between the exponentials of the first pass.
-  auto soft = [&](int tile) __attribute__((always_inline)) {
+  auto soft = [&](int tile, bool first) __attribute__((always_inline)) {
     const int mask_from = tile < p.n_tgt_tiles ? p.t_limit - tile * ATT_BN : ATT_BN;
     if (mask_from < ATT_BN) {
       // keys >= mask_from as one 64-bit word; element i of sub-tile sub is key
@@ -407,27 +409,32 @@ icsa_flash_kernel(FlashParams p) {
         }
       }
     }
-    // four partial sums: a single chain of 32 dependent adds measured 0.4 % slower
-    float rsv[4];
+    float rs = 0.f;
+    if (!first) {
+      // four partial sums: a single chain of 32 dependent adds measured 0.4 % slower
+      float rsv[4];
 #pragma unroll
-    for (int sb = 0; sb < 2; ++sb)
+      for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        if ((i & 7) == 0) {                // DMA segment 2 sb + i / 8 before every 8th exponential
-          __builtin_amdgcn_sched_barrier(0);
-          dma_seg(2 * sb + (i >> 3));
-          __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < 16; ++i) {
+          if ((i & 7) == 0) {                // DMA segment 2 sb + i / 8 before every 8th exponential
+            __builtin_amdgcn_sched_barrier(0);
+            dma_seg(2 * sb + (i >> 3));
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          const float e = __builtin_amdgcn_exp2f(fmaf(s[sb][i], c, -m_ref));
+          if (sb == 0 && i < 4) rsv[i] = e;      // no adds of 0.f (not foldable: signed zeros)
+          else rsv[i & 3] += e;
+          pf[2 * sb + (i >> 3)][i & 7] = (bf16)e;
         }
-        const float e = __builtin_amdgcn_exp2f(fmaf(s[sb][i], c, -m_ref));
-        if (sb == 0 && i < 4) rsv[i] = e;      // no adds of 0.f (not foldable: signed zeros)
-        else rsv[i & 3] += e;
-        pf[2 * sb + (i >> 3)][i & 7] = (bf16)e;
-      }
-    float rs = (rsv[0] + rsv[1]) + (rsv[2] + rsv[3]);
-    // The partial sum exceeds FA_PSUM_MAX (or is NaN) only in a segment's first tile and when
-    // a score rose far above the reference: then raise the reference of every row whose tile
-    // max exceeds it, rescale O and l, and recompute the tile's probabilities.
-    if (__ballot(!(rs <= FA_PSUM_MAX)) != 0ull) {
+      rs = (rsv[0] + rsv[1]) + (rsv[2] + rsv[3]);
+    } else {
+      issue_all();
+    }
+    // The partial sum exceeds FA_PSUM_MAX (or is NaN) only when a score rose far above the
+    // reference: then, and in a segment's first tile, raise the reference of every row whose
+    // tile max exceeds it, rescale O and l, and (re)compute the tile's probabilities.
+    if (first || __ballot(!(rs <= FA_PSUM_MAX)) != 0ull) {
       float mx = -INFINITY;
 #pragma unroll
       for (int sub = 0; sub < 2; ++sub)
@@ -525,7 +532,8 @@ icsa_flash_kernel(FlashParams p) {
   // Every segment goes through the general iteration below for its first and its last tile
   // and through the plain loop for those between.
   bool wrote = false;                      // the GEMM phase before this SOFT phase wrote a segment out
-  int last = len0 - 1;                     // the segment's last iteration
+  bool first = true;                       // the segment's first iteration
+  int last = len0 - 1;                     // and its last
   for (;;) {
     const bool ends = k == last, more = k + 1 < n_it;
     bool q_ahead = false, writes = false;
@@ -535,7 +543,7 @@ icsa_flash_kernel(FlashParams p) {
       __builtin_amdgcn_sched_barrier(0);
     }
     dma_setup();
-    soft(tile);
+    soft(tile, first);
     if (!lag) wait_tile(wrote || q_ahead);            // V(k)
     ATT_BARRIER();
     __builtin_amdgcn_s_setprio(1);
@@ -548,6 +556,7 @@ icsa_flash_kernel(FlashParams p) {
 #pragma unroll
       for (int ds = 0; ds < 4; ++ds) o[ds] = floatx16{};
       l_run = 0.f;
+      m_ref = FA_M_NONE;             // other rows: nothing of this segment's scores carries over
       tile = tile1 - 1;
       seg_len = len1;
       last = k + len1;
@@ -565,7 +574,7 @@ icsa_flash_kernel(FlashParams p) {
     if (!ends) {
       for (; k < last; ++k, ++tile) {
         dma_setup();
-        soft(tile);
+        soft(tile, false);
         if (!lag) wait_tile(false);
         ATT_BARRIER();
         __builtin_amdgcn_s_setprio(1);
@@ -577,6 +586,7 @@ icsa_flash_kernel(FlashParams p) {
       }
     }
     wrote = writes;
+    first = ends;
   }
   __builtin_amdgcn_s_setprio(0);
   if (!lag) ATT_BARRIER();       // group 1's last SOFT phase ends here
