@@ -679,6 +679,12 @@ FlashPlan flash_plan(int64_t n_work, int n_tiles, bool may_split) {
   const int64_t rounds = n_work / FA_CUS, rest = n_work % FA_CUS;
   f.n_whole = (int)n_work;
   f.n_chunk = 0;
+  if (n_tiles <= 0) {                    // a size query for a call without keys (refused later)
+    f.bundle = 1;
+    f.n_bundle = f.n_whole;
+    f.part_bytes = 0;
+    return f;
+  }
   if (may_split && rest > 0) {
     const int64_t g = std::min<int64_t>(FA_CUS, std::max<int64_t>(rest, rest * n_tiles / FA_MIN_CHUNK));
     if (n_tiles - (rest * n_tiles + g - 1) / g > FA_COMBINE_TILES) {

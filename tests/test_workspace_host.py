@@ -1,0 +1,25 @@
+"""CPU tests of the workspace size queries: arguments at which there is nothing to deal out."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from icsa_hip import _lib
+
+pytestmark = pytest.mark.cpu
+
+
+@pytest.mark.parametrize("B,H,S,t,srr", [
+    (1, 40, 65536, 0, 0.0),          # no target, no source blocks retained: no key tiles
+    (2, 200, 256, 0, 0.125),         # no target, a source too short for one retained block
+    (1, 40, 65536, 128, -2 / 1022),  # a negative share that takes the target's blocks away
+])
+def test_size_of_a_layer_without_keys(B, H, S, t, srr):
+    """A size, not an abort (in a process of its own: a division by zero would end it)."""
+    code = ("from icsa_hip import _lib\n"
+            f"print(_lib.lib().icsa_editing_workspace_size({B}, {S}, {H}, 128, {t}, 0.0625, {srr!r}, 0.5, 0, 0, 0))")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
+                       env=dict(os.environ, PYTHONPATH=os.path.dirname(os.path.dirname(_lib.__file__))))
+    assert r.returncode == 0, r.returncode
+    assert int(r.stdout) > 0
