@@ -478,10 +478,12 @@ icsa_flash_kernel(FlashParams p) {
   // A segment boundary costs no slot: Q of the next segment is requested in the SOFT phase
   // of the last tile (its registers are free since that tile's QK) and first used after the
   // next GEMM's PV and the output, which are written from the accumulators between that
-  // GEMM's PV and QK (the scores and probabilities are not live there).  Those at least 8
-  // loads or stores are newer than the tiles waited for next, so these waits (group 0's in
-  // the same SOFT phase for Q and in the following one for the output, group 1's in the
-  // writing GEMM phase and in the following one) allow 8 more in flight.
+  // GEMM's PV and QK (the scores and probabilities are not live there).  These loads and
+  // stores are newer than the tiles waited for next (group 0's in the same SOFT phase for Q and
+  // in the following one for the output, group 1's in the writing GEMM phase and in the
+  // following one), so the wait allows 8 more in flight where at least 8 are sure: Q is 8 loads
+  // of a wave with any row; the output at least 8 stores of a wave with more than 16 rows (of
+  // fewer, the bf16 form issues 4: its second store of a sub-tile, rows 16 .. 31, is skipped).
   // zero key rows >= k_valid of a group-1 wave's K segments (rows 16 dw .. 16 dw + 15)
   auto fill_tail4 = [&](int j, int k_valid) {
     if (k_valid >= ATT_BN) return;
@@ -531,7 +533,7 @@ icsa_flash_kernel(FlashParams p) {
   int k = 0;
   // Every segment goes through the general iteration below for its first and its last tile
   // and through the plain loop for those between.
-  bool wrote = false;                      // the GEMM phase before this SOFT phase wrote a segment out
+  bool wrote = false;                      // the GEMM phase before this SOFT phase issued 8 stores or more
   bool first = true;                       // the segment's first iteration
   int last = len0 - 1;                     // and its last
   for (;;) {
@@ -551,8 +553,8 @@ icsa_flash_kernel(FlashParams p) {
     if (!more) break;
     if (ends) {
       __builtin_amdgcn_s_setprio(0);
-      writes = sg.q_valid > 0;
-      if (writes) flush(seg_len != n_tiles);
+      writes = sg.q_valid > 16;
+      if (sg.q_valid > 0) flush(seg_len != n_tiles);
 #pragma unroll
       for (int ds = 0; ds < 4; ++ds) o[ds] = floatx16{};
       l_run = 0.f;

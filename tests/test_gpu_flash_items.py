@@ -78,13 +78,18 @@ def test_infinite_scores_stay_in_their_head(gpu, B, H, Sq, Sk):
     assert torch.equal(x[:, :, keep], y[:, :, keep])
 
 
-def test_layer_heads_as_alone(gpu):
-    """The layer's peaked blocks: 9 key tiles, two items a head, two items a workgroup."""
-    H, t = 140, 512
-    g = torch.Generator().manual_seed(3)
-    q, k, v = (torch.randn(1, 2 * t, H, 128, generator=g) for _ in range(3))
-    level = torch.tensor([40.0, 0.0, 1.0])[torch.randint(3, (1, 2 * t // 64, H, 1), generator=g)]
-    q = q * level.repeat_interleave(64, dim=1)
+@pytest.mark.parametrize("S,t", [
+    (1024, 512),            # 9 key tiles, two whole items a head
+    (649, 320),             # 5 key tiles; items of 4 and of 1 block, a last block of 9 rows that may
+                            # come anywhere among a head's 5 peaked ones
+])
+def test_layer_heads_as_alone(gpu, S, t):
+    """The layer's peaked blocks, two items a workgroup."""
+    H = 140
+    g = torch.Generator().manual_seed(S)
+    q, k, v = (torch.randn(1, S, H, 128, generator=g) for _ in range(3))
+    level = torch.tensor([40.0, 0.0, 1.0])[torch.randint(3, (1, (S + 63) // 64, H, 1), generator=g)]
+    q = q * level.repeat_interleave(64, dim=1)[:, :S]
     q, k, v = (x.to(torch.bfloat16).to(gpu) for x in (q, k, v))
     x, _ = _editing_sparse_attention_hip(q, k, v, t)
     assert x.isfinite().all()
