@@ -9,6 +9,7 @@
 #include <mutex>
 #include <string>
 
+#include "flash_plan.h"
 #include "icsa_kernels.h"
 #include "../../include/icsa.h"
 

@@ -49,14 +49,11 @@
 // common case no per-tile max reduction precedes the exponentials.  Exact in real arithmetic.
 // (The first tile by that check as well, two passes of exponentials: 8 tiles an item, forward
 // 811-823 us a call against 789-806.)
-#include <algorithm>
-
 #include "attn_tile.h"
+#include "flash_plan.h"
 #include "icsa_kernels.h"
 
-#define FA_WAVES 8
 #define FA_THREADS (FA_WAVES * 64)
-#define FA_QBLK_PER_WG (FA_WAVES / 2)
 #define FA_NBUF 4                                            // K and V^T tile buffers
 #define FA_TILE_BYTES (FA_NBUF * (K_TILE_BYTES + V_TILE_BYTES))
 #define FA_JUNK_OFF FA_TILE_BYTES                            // landing area of disabled DMA
@@ -73,8 +70,6 @@
 #ifndef FA_PF
 #define FA_PF 5             // operand prefetch depth (MFMA steps); 3, 4, 6 and 8 measured slower
 #endif
-#define FA_PART_WAVE (64 * 64 + 2 * 64)                      // floats of one wave's partial: O, m, l
-#define FA_PART_FLOATS (FA_WAVES * FA_PART_WAVE)
 
 namespace {
 
@@ -657,61 +652,6 @@ __global__ void __launch_bounds__(256) icsa_flash_combine_kernel(FlashParams p) 
   const float* oc = p.out_c ? p.out_c + ((int64_t)bh * p.nb_q + qblk) * ICSA_D : nullptr;
   store_subtile<kBf16, kAlphaD>(stage[ds], acc, ds, 1.f / xhalf_sum(l), p.out, bh / p.H, bh % p.H,
                 qblk * ICSA_BLOCK + 32 * (w & 1), q_valid, oc, p.alpha);
-}
-
-// ------------------------------------------------------------------------------------------
-// How the items are dealt out.  One workgroup fills a CU's LDS, so the chip runs FA_CUS of
-// them at a time, and a last round of r < FA_CUS items takes as long as a full one.
-//  * Those r items are cut into FA_CUS chunks of r n_tiles / FA_CUS tiles when that saves
-//    more than FA_COMBINE_TILES tiles: the sums' kernel takes 9-13 us and a tile 1.7 us of a
-//    workgroup, and a chunk's workgroup has a start of its own (about 5 us).  Chunks are not
-//    shorter than FA_MIN_CHUNK tiles.
-//  * Whole items go several to a workgroup, up to FA_BUNDLE_TILES tiles, in equal numbers:
-//    beyond that a workgroup's start no longer counts and many workgroups even out the
-//    CUs (220 tiles an item, 8.6 rounds: 4,710 us with bundles of 1 or 2 items, 4,870 us
-//    with 8; 8 tiles an item, 40 rounds: 783, 775 and 773 us with 14, 20 and 40 items).
-// ------------------------------------------------------------------------------------------
-#define FA_CUS 256
-#define FA_MIN_CHUNK 4
-#define FA_COMBINE_TILES 12
-#define FA_BUNDLE_TILES 512
-
-FlashPlan flash_plan(int64_t n_work, int n_tiles, bool may_split) {
-  FlashPlan f;
-  const int64_t rounds = n_work / FA_CUS, rest = n_work % FA_CUS;
-  f.n_whole = (int)n_work;
-  f.n_chunk = 0;
-  if (n_tiles <= 0) {                    // a size query for a call without keys (refused later)
-    f.bundle = 1;
-    f.n_bundle = f.n_whole;
-    f.part_bytes = 0;
-    return f;
-  }
-  if (may_split && rest > 0) {
-    const int64_t g = std::min<int64_t>(FA_CUS, std::max<int64_t>(rest, rest * n_tiles / FA_MIN_CHUNK));
-    if (n_tiles - (rest * n_tiles + g - 1) / g > FA_COMBINE_TILES) {
-      f.n_whole = (int)(rounds * FA_CUS);
-      f.n_chunk = (int)g;
-    }
-  }
-  int64_t m = 1;
-  if (f.n_whole > FA_CUS) {
-    const int64_t per_cu = (f.n_whole + FA_CUS - 1) / FA_CUS;
-    const int64_t want = std::max<int64_t>(1, std::min<int64_t>(per_cu, FA_BUNDLE_TILES / n_tiles));
-    const int64_t k = (per_cu + want - 1) / want;
-    m = (per_cu + k - 1) / k;
-
-  }
-  f.bundle = (int)m;
-  f.n_bundle = (int)((f.n_whole + m - 1) / m);
-  f.part_bytes = f.n_chunk ? (int64_t)(f.n_chunk + rest) * FA_PART_FLOATS * 4 : 0;
-  return f;
-}
-
-int64_t flash_items(int BH, int n_qblk) { return (int64_t)BH * ((n_qblk + FA_QBLK_PER_WG - 1) / FA_QBLK_PER_WG); }
-
-int64_t flash_part_bytes_max(int n_tiles) {
-  return n_tiles > FA_COMBINE_TILES ? (int64_t)(2 * FA_CUS - 1) * FA_PART_FLOATS * 4 : 0;
 }
 
 // kAlphaD: the residual weight varies along the head dim (its own instantiation: its gathers

@@ -114,15 +114,8 @@ struct FlashParams {
   OutView out;
   float scale_log2;                // log2(e) / sqrt(D)
   float* part; int64_t part_bytes; // room for the partials of split items (part_bytes 0: none)
-  // set by launch_flash: items (4 query blocks of one head) [0, n_whole) run whole, `bundle`
-  // consecutive ones per workgroup (n_bundle workgroups); the tiles of the others are cut
-  // into n_chunk equal ranges, one per workgroup, and combined
-  int n_whole, bundle, n_bundle, n_chunk;
+  int n_whole, bundle, n_bundle, n_chunk;   // FlashPlan, set by launch_flash
 };
-struct FlashPlan { int n_whole, bundle, n_bundle, n_chunk; int64_t part_bytes; };
-int64_t flash_items(int BH, int n_qblk);
-FlashPlan flash_plan(int64_t n_work, int n_tiles, bool may_split);
-int64_t flash_part_bytes_max(int n_tiles);      // over any number of items
 hipError_t launch_flash(FlashParams p, hipStream_t stream);
 
 // ---------------------------------------------------------------- Wan q/k producer (wan_qk.hip)
