@@ -176,13 +176,14 @@ icsa_flash_kernel(FlashParams p) {
   // (a window of n_tiles - chunk length tiles that L2 holds) instead of being spread over
   // all of them.
   int item0, tile0 = 0, len0 = n_tiles, tile1 = 0, len1 = n_tiles, step = 1, n_it, chunk = -1;
-  if ((int)blockIdx.x < xcd_grid(p.n_bundle)) {
-    const int u = xcd_remap(blockIdx.x, p.n_bundle);
-    if (u < 0) return;
-    item0 = u * p.bundle;
-    n_it = min(p.bundle, p.n_whole - item0) * n_tiles;
+  if ((int)blockIdx.x < FA_XCDS * p.n_bundle) {
+    const FlashRun run = flash_whole_run(blockIdx.x, p.n_whole, p.n_bundle);
+    if (run.count == 0) return;
+    item0 = run.first;
+    step = p.n_bundle;
+    n_it = run.count * n_tiles;
   } else {
-    chunk = xcd_remap(blockIdx.x - xcd_grid(p.n_bundle), p.n_chunk);
+    chunk = xcd_remap(blockIdx.x - FA_XCDS * p.n_bundle, p.n_chunk);
     if (chunk < 0) return;
     const int n_split = p.B * p.H * ngrp - p.n_whole;
     const int64_t lo = chunk_start(chunk, n_split, n_tiles, p.n_chunk);
@@ -662,7 +663,7 @@ static hipError_t run_flash(const FlashParams& p, int64_t n_work, hipStream_t st
   const hipError_t attr = ensure_lds_limit(reinterpret_cast<const void*>(icsa_flash_kernel<kBf16, kAlphaD>),
                                            FA_LDS_BYTES, &lds_set);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((icsa_flash_kernel<kBf16, kAlphaD>), dim3(xcd_grid(p.n_bundle) + xcd_grid(p.n_chunk)),
+  hipLaunchKernelGGL((icsa_flash_kernel<kBf16, kAlphaD>), dim3(FA_XCDS * p.n_bundle + xcd_grid(p.n_chunk)),
                      dim3(FA_THREADS), FA_LDS_BYTES, stream, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.n_chunk == 0) return e;
@@ -681,7 +682,7 @@ hipError_t launch_flash(FlashParams p, hipStream_t stream) {
     return hipErrorInvalidValue;
   FlashPlan f = flash_plan(n_work, n_tiles, true);
   if (f.part_bytes > p.part_bytes) f = flash_plan(n_work, n_tiles, false);
-  p.n_whole = f.n_whole; p.n_chunk = f.n_chunk; p.bundle = f.bundle; p.n_bundle = f.n_bundle;
+  p.n_whole = f.n_whole; p.n_chunk = f.n_chunk; p.n_bundle = f.n_bundle;
   const bool alpha_d = p.out_c != nullptr && p.alpha.p != nullptr && p.alpha.sd != 0;
   if (p.out.dtype == ICSA_DT_BF16)
     return alpha_d ? run_flash<true, true>(p, n_work, stream) : run_flash<true, false>(p, n_work, stream);

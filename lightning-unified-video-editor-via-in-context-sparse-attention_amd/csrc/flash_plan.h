@@ -10,9 +10,25 @@
 #define FA_PART_WAVE (64 * 64 + 2 * 64)                      // floats of one wave's partial: O, m, l
 #define FA_PART_FLOATS (FA_WAVES * FA_PART_WAVE)
 
-// Items [0, n_whole) run whole, `bundle` consecutive ones per workgroup (n_bundle workgroups); the
-// tiles of the others are cut into n_chunk equal ranges, one per workgroup, and combined.
+#define FA_XCDS 8
+
+// Items [0, n_whole) run whole, up to `bundle` of them per workgroup (n_bundle workgroups on each
+// XCD); the tiles of the others are cut into n_chunk equal ranges, one per workgroup, and combined.
 struct FlashPlan { int n_whole, bundle, n_bundle, n_chunk; int64_t part_bytes; };
+
+// The whole items of workgroup wg < FA_XCDS * n_bundle: first, first + n_bundle, ... (count of
+// them, maybe 0).  Workgroup wg runs on XCD wg % 8, and each XCD has a contiguous range of the
+// items, its workgroups side by side in it: the items of one head run at the same time and read
+// its K and V from that XCD's L2.  With consecutive items in a workgroup instead, a head's
+// second item came after its first had moved on (320 heads, 320 queries, 4,096 keys: 499 us a
+// call, now 438; 432 with one item a workgroup).
+struct FlashRun { int first, count; };
+constexpr FlashRun flash_whole_run(int wg, int n_whole, int n_bundle) {
+  const int per = (n_whole + FA_XCDS - 1) / FA_XCDS, x = wg % FA_XCDS;
+  const int first = x * per + wg / FA_XCDS;
+  const int end = (x + 1) * per < n_whole ? (x + 1) * per : n_whole;
+  return FlashRun{first, first < end ? (end - first + n_bundle - 1) / n_bundle : 0};
+}
 
 // One workgroup fills a CU's LDS, so the chip runs FA_CUS of them at a time, and a last round
 // of r < FA_CUS items takes as long as a full one.
@@ -39,6 +55,7 @@ inline FlashPlan flash_plan(int64_t n_work, int n_tiles, bool may_split) {
   f.n_whole = (int)n_work;
   f.n_chunk = 0;
   f.bundle = 1;
+  int64_t per_xcd = 0;
   if (n_tiles > 0) {                     // 0: a size query for a call without keys (refused later)
     if (may_split && rest > 0) {
       const int64_t g = std::min<int64_t>(FA_CUS, std::max<int64_t>(rest, rest * n_tiles / FA_MIN_CHUNK));
@@ -47,18 +64,19 @@ inline FlashPlan flash_plan(int64_t n_work, int n_tiles, bool may_split) {
         f.n_chunk = (int)g;
       }
     }
-    const int64_t per_cu = ((int64_t)f.n_whole + FA_CUS - 1) / FA_CUS;
+    per_xcd = ((int64_t)f.n_whole + FA_XCDS - 1) / FA_XCDS;
+    const int64_t cus = FA_CUS / FA_XCDS, per_cu = (per_xcd + cus - 1) / cus;
     int64_t best = INT64_MAX;
     for (int64_t m = 1; m <= std::max<int64_t>(1, std::min<int64_t>(per_cu, FA_BUNDLE_TILES / n_tiles)); ++m) {
-      const int64_t n = (f.n_whole + m - 1) / m;
-      const int64_t cost = (n + FA_CUS - 1) / FA_CUS * (m * n_tiles + FA_START_TILES);
+      const int64_t n = (per_xcd + m - 1) / m;
+      const int64_t cost = (n + cus - 1) / cus * (m * n_tiles + FA_START_TILES);
       if (cost < best) {
         best = cost;
         f.bundle = (int)m;
       }
     }
   }
-  f.n_bundle = (f.n_whole + f.bundle - 1) / f.bundle;
+  f.n_bundle = (int)((per_xcd + f.bundle - 1) / f.bundle);
   f.part_bytes = f.n_chunk ? (int64_t)(f.n_chunk + rest) * FA_PART_FLOATS * 4 : 0;
   return f;
 }

@@ -114,7 +114,7 @@ struct FlashParams {
   OutView out;
   float scale_log2;                // log2(e) / sqrt(D)
   float* part; int64_t part_bytes; // room for the partials of split items (part_bytes 0: none)
-  int n_whole, bundle, n_bundle, n_chunk;   // FlashPlan, set by launch_flash
+  int n_whole, n_bundle, n_chunk;  // FlashPlan, set by launch_flash
 };
 hipError_t launch_flash(FlashParams p, hipStream_t stream);
 

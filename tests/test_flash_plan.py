@@ -10,7 +10,7 @@ from icsa_hip import build
 
 pytestmark = pytest.mark.cpu
 
-CUS = 256
+CUS, XCDS = 256, 8
 START = 3                      # a workgroup's start, in tiles
 COMBINE = 8                    # the sums of split items: 9-13 us, a tile 1.7 us
 
@@ -21,8 +21,13 @@ int main() {
   long long n; int tiles, split;
   while (std::scanf("%lld %d %d", &n, &tiles, &split) == 3) {
     const FlashPlan f = flash_plan(n, tiles, split != 0);
-    std::printf("%d %d %d %d %lld %lld\\n", f.n_whole, f.bundle, f.n_bundle, f.n_chunk, (long long)f.part_bytes,
+    std::printf("%d %d %lld %lld", f.n_whole, f.n_chunk, (long long)f.part_bytes,
                 (long long)flash_part_bytes_max(tiles));
+    for (int wg = 0; wg < FA_XCDS * f.n_bundle; ++wg) {
+      const FlashRun r = flash_whole_run(wg, f.n_whole, f.n_bundle);
+      std::printf(" %d %d", r.first, r.count);
+    }
+    std::printf("\\n");
   }
 }
 """
@@ -40,7 +45,11 @@ def plans(tmp_path_factory):
                    check=True)
     out = subprocess.run([str(d / "main")], input="\n".join("%d %d %d" % g for g in GRID), capture_output=True,
                          text=True, check=True).stdout
-    return dict(zip(GRID, ([int(x) for x in line.split()] for line in out.splitlines())))
+    res = {}
+    for g, line in zip(GRID, out.splitlines()):
+        x = [int(y) for y in line.split()]
+        res[g] = x[:4] + [list(zip(x[4::2], x[5::2]))]
+    return res
 
 
 def _span(lengths):
@@ -52,8 +61,9 @@ def _span(lengths):
 
 
 def test_plan_covers_the_items(plans):
-    for (n, tiles, split), (whole, bundle, n_bundle, chunks, part, part_max) in plans.items():
-        assert bundle >= 1 and (n_bundle - 1) * bundle < max(whole, 1) <= max(n_bundle * bundle, 1)
+    for (n, tiles, split), (whole, chunks, part, part_max, runs) in plans.items():
+        step = len(runs) // XCDS
+        assert sorted(first + i * step for first, count in runs for i in range(count)) == list(range(whole))
         if chunks == 0:
             assert whole == n and part == 0
         else:                                   # a chunk holds tiles of at most two items
@@ -61,14 +71,25 @@ def test_plan_covers_the_items(plans):
             assert 0 < part <= part_max
 
 
+def test_neighbouring_items_run_side_by_side(plans):
+    """The i-th items of an XCD's workgroups are consecutive: the items of a head share its K and
+    V in that XCD's L2 (640 items of 64 tiles, two a head, one after the other in a workgroup:
+    499 us a call, side by side 438)."""
+    for whole, chunks, part, part_max, runs in plans.values():
+        step = len(runs) // XCDS
+        for x in range(XCDS):
+            for i in range(max([c for _, c in runs[x::XCDS]], default=0)):
+                at = [first + i * step for first, count in runs[x::XCDS] if count > i]
+                assert at == list(range(at[0], at[0] + len(at)))
+
+
 def test_plan_is_no_slower_than_an_item_a_workgroup(plans):
     """Several items a workgroup, or the last round's cut up, take no more time than one whole item
-    a workgroup (2 %): 768 items of 256 tiles took 1,590 us in pairs, 1,390 us one by one."""
+    a workgroup (2 %): 768 items of 256 tiles took 1,541 us in pairs, 1,350 one by one."""
     slow = []
-    for (n, tiles, split), (whole, bundle, n_bundle, chunks, part, part_max) in plans.items():
-        lengths = [min(bundle, whole - i * bundle) * tiles for i in range(n_bundle)]
-        lengths += [(n - whole) * tiles / max(chunks, 1)] * chunks
-        t = _span(lengths) + (COMBINE if chunks else 0)
+    for (n, tiles, split), (whole, chunks, part, part_max, runs) in plans.items():
+        t = _span([c * tiles for _, c in runs if c] + [(n - whole) * tiles / max(chunks, 1)] * chunks)
+        t += COMBINE if chunks else 0
         if t > 1.02 * _span([tiles] * n):
-            slow.append((n, tiles, split, bundle, round(t / _span([tiles] * n), 3)))
+            slow.append((n, tiles, split, round(t / _span([tiles] * n), 3)))
     assert not slow, slow
