@@ -527,6 +527,26 @@ icsa_flash_kernel(FlashParams p) {
   int tile = tile0;                        // tile of iteration k
   int seg_len = len0;
   int k = 0;
+  // A wave without rows in any of the workgroup's items only moves tiles: its products and
+  // exponentials would take issue slots from the others (calls of one head, 64 queries, 1,000
+  // keys 29.9 -> 25.6 us; 320 heads, 1 query, 512 keys 50.6 -> 45.2; 640 heads, 64 queries, 2,048
+  // keys 366 -> 359).  Decided once: the same test around every product and exponential
+  // costs 168 spilled vector registers and 2 to 3 times the time.
+  if (sg.q_valid == 0 && (n_it <= len0 || (ngrp == 1 && p.qblocks == nullptr))) {
+    for (;;) {
+      dma_setup();
+      issue_all();
+      if (!lag) wait_tile(false);
+      ATT_BARRIER();
+      if (k + 1 == n_it) break;
+      wait_k(k + 2, false);
+      ATT_BARRIER();
+      ++k;
+    }
+    if (!lag) ATT_BARRIER();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return;
+  }
   // Every segment goes through the general iteration below for its first and its last tile
   // and through the plain loop for those between.
   bool wrote = false;                      // the GEMM phase before this SOFT phase issued 8 stores or more
