@@ -269,6 +269,9 @@ int icsa_sparse_piecewise_attn_bwd(
  * blocks whose keys are split over several workgroups.  A workspace that holds the V^T alone
  * (B * H * D * 64 ceil(Sk / 64) bf16, rounded up to 256 bytes) is accepted as well. */
 int64_t icsa_flash_attn_workspace_size(int B, int Sk, int H, int D);
+/* The same for a call of Sq queries: as many partials as that call has (none in most), where the
+ * size for any Sq counts the most there can be, 69 MB from 13 key tiles on. */
+int64_t icsa_flash_attn_workspace_size_for(int B, int Sq, int Sk, int H, int D);
 
 /* Dense non-causal attention softmax(q k^T / sqrt(D)) v: q [B, Sq, H, D], k/v [B, Sk, H, D]
  * bf16, out [B, Sq, H, D] bf16 or f32.  Also this library's dense baseline. */

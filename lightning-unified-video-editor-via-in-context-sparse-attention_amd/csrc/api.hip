@@ -941,6 +941,12 @@ int64_t icsa_flash_attn_workspace_size(int B, int Sk, int H, int D) {
   return flash_vt_bytes(B, Sk, H) + flash_part_bytes_max(ceil_div(Sk, ICSA_BLOCK));
 }
 
+int64_t icsa_flash_attn_workspace_size_for(int B, int Sq, int Sk, int H, int D) {
+  if (B <= 0 || Sk <= 0 || H <= 0 || D != ICSA_D) return -1;
+  const int64_t items = flash_items(B * H, ceil_div(std::max(Sq, 0), ICSA_BLOCK));
+  return flash_vt_bytes(B, Sk, H) + flash_plan(items, ceil_div(Sk, ICSA_BLOCK), true).part_bytes;
+}
+
 int icsa_flash_attn(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
                     const void* k, int64_t k_sb, int64_t k_ss, int64_t k_sh,
                     const void* v, int64_t v_sb, int64_t v_ss, int64_t v_sh,

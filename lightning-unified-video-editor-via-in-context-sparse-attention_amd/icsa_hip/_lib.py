@@ -41,7 +41,8 @@ EXPORTS = [
     "icsa_editing_sparse_attention", "icsa_editing_sparse_attention_ev",
     "icsa_editing_sparse_attention_noalloc",
     "icsa_sparse_piecewise_workspace_size",
-    "icsa_sparse_piecewise_attn", "icsa_flash_attn_workspace_size", "icsa_flash_attn",
+    "icsa_sparse_piecewise_attn", "icsa_flash_attn_workspace_size",
+    "icsa_flash_attn_workspace_size_for", "icsa_flash_attn",
     "icsa_pool", "icsa_gather_kv", "icsa_wan_qk_workspace_size", "icsa_wan_qk_prologue",
     "icsa_editing_sparse_attention_presummed", "icsa_wan_ln_modulate", "icsa_last_error",
     "icsa_version", "icsa_sparse_piecewise_attn_fwd", "icsa_sparse_piecewise_attn_bwd_workspace_size",
@@ -124,6 +125,7 @@ _SIGNATURES = {
         _p, _i, _l, _l, _l,
         _p, _l, _p]),
     "icsa_flash_attn_workspace_size": (_l, [_i, _i, _i, _i]),
+    "icsa_flash_attn_workspace_size_for": (_l, [_i, _i, _i, _i, _i]),
     "icsa_flash_attn": (_i, [
         _p, _l, _l, _l,
         _p, _l, _l, _l,

@@ -356,9 +356,9 @@ def flash_attn_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, dropout_p
     out_dtype = out_dtype or torch.bfloat16
     out = torch.empty(B, Sq, H, D, dtype=out_dtype, device=q.device)
     L = _lib.lib()
-    ws_bytes = L.icsa_flash_attn_workspace_size(B, Sk, H, D)
+    ws_bytes = L.icsa_flash_attn_workspace_size_for(B, Sq, Sk, H, D)
     if ws_bytes < 0:
-        raise _lib.IcsaError("icsa_flash_attn_workspace_size", int(ws_bytes))
+        raise _lib.IcsaError("icsa_flash_attn_workspace_size_for", int(ws_bytes))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
     with on_device(q.device):
         rc = L.icsa_flash_attn(

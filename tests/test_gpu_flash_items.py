@@ -96,3 +96,16 @@ def test_layer_heads_as_alone(gpu, S, t):
     for h in range(0, H, 7):
         y, _ = _editing_sparse_attention_hip(*(a[:, :, h:h + 1] for a in (q, k, v)), t)
         assert torch.equal(x[:, :, h], y[:, :, 0]), h
+
+
+def test_small_call_allocates_little(gpu):
+    """64 queries, 1,000 keys, one head: V^T (256 KB), no partials; 64 queries, 1,500 keys: 6 chunks of
+    one item, 7 partials of 135 KB at most."""
+    for Sk, most in ((1000, 2 ** 19), (1500, 2 ** 21)):
+        q, k, v = _inputs(1, 1, 64, Sk, Sk, gpu)
+        flash_attn_func(q, k, v)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        flash_attn_func(q, k, v)
+        assert torch.cuda.max_memory_allocated() - before <= most
