@@ -723,7 +723,7 @@ static int sparse_piecewise_impl(
   ICSA_HIP_TRY(launch_pool(pp, stream), "pool");
 
   int32_t* idx = idx_out ? idx_out : reinterpret_cast<int32_t*>(ws + L.idx);
-  if (inject_idx) {
+  if (inject_idx && inject_idx != idx) {          // lists handed in and out in one buffer stay there
     ICSA_HIP_TRY(hipMemcpyAsync(idx, inject_idx, (size_t)BH * NQ * top_k * 4, hipMemcpyDeviceToDevice,
                                 stream), "inject idx");
   }
