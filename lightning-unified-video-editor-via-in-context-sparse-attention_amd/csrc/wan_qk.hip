@@ -22,6 +22,7 @@
 // rotated (pad_freqs pads with ones).  Pair j of a head uses the f axis for j < D/2 - 2*(D/2/3),
 // then the h axis and the w axis for D/2/3 pairs each (rope_apply's freqs.split).
 #include "icsa_kernels.h"
+#include "wan_qk_rule.h"
 
 // The alpha gate of token s: bf16 arithmetic of the reference, sigmoid, - 0.5 and * 0.5 each
 // round to bf16
@@ -213,13 +214,8 @@ __global__ void __launch_bounds__(256) icsa_wan_qk_kernel(WanQkParams p) {
 // thread group 4 round + w of icsa_wan_qk_kernel takes, so all sums run in the same order
 // and the results are the same bits.  A chunk's registers take the next round's load as soon
 // as it is stored.  The block sums go through LDS chunk by chunk (512 dims, two buffers, one
-// barrier each).  40 heads, 28,080 tokens: 352 -> 281 us.  Few blocks leave most CUs idle for four
-// rounds: this kernel takes over from WQ_MIN_BLOCKS 64-token blocks of one head (q and k both
-// counted).  Measured, two passes / one: 40 heads 93 / 109 us at 7,840 such blocks, 124 / 124 at
-// 10,240, 190 / 160 at 15,600, 339 / 281 at 31,200; 12 heads 59 / 71 at 6,144, 113 / 109 at 9,360,
-// 146 / 117 at 12,288.
-#define WQ_MIN_BLOCKS 12000
-#define WQ_MAX_CH 10
+// barrier each).  40 heads, 28,080 tokens: 352 -> 281 us.  The two kernels above stay for few blocks
+// and for rows that leave most of the lanes empty (wan_one_pass).
 
 template <int NCH>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
@@ -337,11 +333,13 @@ icsa_wan_qk_rows_kernel(WanRmsParams rp, WanQkParams p) {
 
 hipError_t launch_wan_qk(const WanRmsParams& rp, const WanQkParams& qp, hipStream_t stream) {
   const int nt = qp.y[1].p != nullptr ? 2 : 1;
-  if (qp.y[0].dtype != ICSA_DT_F32 && qp.H <= 4 * WQ_MAX_CH && (int64_t)qp.NB * nt * qp.B * qp.H >= WQ_MIN_BLOCKS) {
+  if (qp.y[0].dtype != ICSA_DT_F32 && wan_one_pass((int64_t)qp.NB * nt * qp.B, qp.H, qp.sums[0] != nullptr)) {
     const dim3 rows_grid(qp.NB, nt, qp.B);
-    if (qp.H <= 12) hipLaunchKernelGGL(icsa_wan_qk_rows_kernel<3>, rows_grid, dim3(256), 0, stream, rp, qp);
-    else if (qp.H <= 20) hipLaunchKernelGGL(icsa_wan_qk_rows_kernel<5>, rows_grid, dim3(256), 0, stream, rp, qp);
-    else hipLaunchKernelGGL(icsa_wan_qk_rows_kernel<WQ_MAX_CH>, rows_grid, dim3(256), 0, stream, rp, qp);
+    switch (wan_row_chunks(qp.H)) {
+      case 3: hipLaunchKernelGGL(icsa_wan_qk_rows_kernel<3>, rows_grid, dim3(256), 0, stream, rp, qp); break;
+      case 5: hipLaunchKernelGGL(icsa_wan_qk_rows_kernel<5>, rows_grid, dim3(256), 0, stream, rp, qp); break;
+      default: hipLaunchKernelGGL(icsa_wan_qk_rows_kernel<WQ_MAX_CH>, rows_grid, dim3(256), 0, stream, rp, qp);
+    }
     return hipGetLastError();
   }
   const int64_t ntok = (int64_t)rp.B * rp.S;

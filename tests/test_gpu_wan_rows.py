@@ -1,8 +1,9 @@
 """GPU test of the q / k producer's one-pass kernel against its two-pass kernels: a batch of eight
-takes the one-pass kernel, each of its sequences alone the two-pass kernels.  The sums run in the
-same order in both, so the comparison is exact.  Head counts at the edges of the row chunks (4
-heads each) and of the instantiations, whole and ragged last blocks, one input or two, with
-and without block sums and gate."""
+takes the one-pass kernel where the rule of csrc/wan_qk_rule.h gives it the call, each of its
+sequences alone the two-pass kernels.  The sums run in the same order in both, so the comparison
+is exact.  Head counts at the edges of the row chunks (4 heads each) and of the
+instantiations, whole and ragged last blocks, one input or two, with and without block sums and
+gate."""
 import pytest
 import torch
 
@@ -11,13 +12,22 @@ from icsa_hip.wan import wan_freqs, wan_qk_prologue
 pytestmark = pytest.mark.gpu
 
 
+# 64-token blocks of one head from which a batch of eight takes the one-pass kernel (below: 12,000)
+SERVED = {6: 12000, 13: 12000, 21: 19400, 24: 19400, 40: 14000}
+
+
+@pytest.mark.parametrize("H,extra,two,sums", [(6, 5, True, True), (13, 63, True, True), (21, 40, True, False),
+                                              (24, 1, False, True), (40, 17, True, True)])
+def test_one_pass_equals_two_passes_where_it_serves(gpu, H, extra, two, sums):
+    test_one_pass_equals_two_passes(gpu, H, extra, two, sums, SERVED[H])
+
+
 @pytest.mark.parametrize("H,extra,two,sums", [(1, 1, True, True), (3, 0, True, True), (12, 0, True, True),
                                               (13, 63, True, True), (20, 0, False, True), (21, 40, True, False),
                                               (40, 17, True, True)])
-def test_one_pass_equals_two_passes(gpu, H, extra, two, sums):
+def test_one_pass_equals_two_passes(gpu, H, extra, two, sums, blocks=12000):
     B, D = 8, 128
-    # the batch holds the 12,000 blocks (of one head, q and k) from which the one-pass kernel serves
-    S = 64 * -(-12000 // (B * H * (2 if two else 1))) + extra
+    S = 64 * -(-blocks // (B * H * (2 if two else 1))) + extra
     g = torch.Generator().manual_seed(S + H)
     yq = torch.randn(B, S, H * D, generator=g).to(torch.bfloat16).to(gpu)
     yk = (torch.randn(B, S, H * D, generator=g) * 3).to(torch.bfloat16).to(gpu) if two else None
