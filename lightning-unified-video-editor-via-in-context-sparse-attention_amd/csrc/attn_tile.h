@@ -80,66 +80,11 @@ __device__ __forceinline__ unsigned lds_u32(const void* p) {
 // barrier are complete when it is passed (lgkmcnt(0)).
 #define ATT_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 
-// Register staging of one K + V^T tile for a workgroup of NT threads (NT = 256 or 128).
-template <int NT>
-struct TileRegs {
-  static constexpr int N = (ATT_BN * ICSA_D / 8) / NT;   // 16-byte chunks per thread per tile
-  u32x4 k[N];
-  u32x4 v[N];
-};
-
 __device__ __forceinline__ int k_lds_off(int row, int chunk) {     // in bf16 elements
   return row * ICSA_D + ((chunk ^ (row & 15)) << 3);
 }
 __device__ __forceinline__ int v_lds_off(int d, int chunk) {
   return d * ATT_BN + ((chunk ^ ((d >> 1) & 7)) << 3);
-}
-
-// Global -> registers for one tile.  krow0: pointer to key row 0 of the tile, k_rs: key row
-// stride (elements), k_valid: rows < k_valid are real (others read as 0).  vcol0: pointer
-// to V^T row d = 0 at the tile's first slot, v_rs: V^T row stride; v_zero: zero V^T tile.
-template <int NT>
-__device__ __forceinline__ void tile_load_regs(TileRegs<NT>& r, const bf16* krow0, int64_t k_rs,
-                                               int k_valid, const bf16* vcol0, int64_t v_rs,
-                                               bool v_zero) {
-  constexpr int N = TileRegs<NT>::N;
-  constexpr int KR = NT / 16;          // key rows covered per pass
-  constexpr int VR = NT / 8;           // V^T rows covered per pass
-  const int t = threadIdx.x;
-  const int kr = t >> 4, kc = t & 15;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const int row = kr + KR * i;
-    if (row < k_valid)
-      r.k[i] = *reinterpret_cast<const u32x4*>(krow0 + (int64_t)row * k_rs + 8 * kc);
-    else
-      r.k[i] = u32x4{0u, 0u, 0u, 0u};
-  }
-  const int vd = t >> 3, vc = t & 7;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const int d = vd + VR * i;
-    if (!v_zero)
-      r.v[i] = *reinterpret_cast<const u32x4*>(vcol0 + (int64_t)d * v_rs + 8 * vc);
-    else
-      r.v[i] = u32x4{0u, 0u, 0u, 0u};
-  }
-}
-
-template <int NT>
-__device__ __forceinline__ void tile_store_lds(const TileRegs<NT>& r, bf16* ks, bf16* vs) {
-  constexpr int N = TileRegs<NT>::N;
-  constexpr int KR = NT / 16;
-  constexpr int VR = NT / 8;
-  const int t = threadIdx.x;
-  const int kr = t >> 4, kc = t & 15;
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-    *reinterpret_cast<u32x4*>(ks + k_lds_off(kr + KR * i, kc)) = r.k[i];
-  const int vd = t >> 3, vc = t & 7;
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-    *reinterpret_cast<u32x4*>(vs + v_lds_off(vd + VR * i, vc)) = r.v[i];
 }
 
 // Q^T operand of one wave: 32 queries (rows qrow0 + lane%32, rows >= q_valid are zero).
@@ -171,38 +116,6 @@ __device__ __forceinline__ void settle_frags(bf16x8 f[8]) {
   asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]));
 #pragma unroll
   for (int i = 0; i < 8; ++i) f[i] = __builtin_bit_cast(bf16x8, x[i]);
-}
-
-// S^T for the 64 keys of an LDS K tile: s[ks] covers keys 32*ks .. 32*ks + 31.
-__device__ __forceinline__ void qk_tile(floatx16 s[2], const bf16* ks, const bf16x8 qf[8]) {
-  const int lane = threadIdx.x & 63;
-  const int li = lane & 31, hl = lane >> 5;
-#pragma unroll
-  for (int sub = 0; sub < 2; ++sub) {
-    floatx16 acc = {};
-    const int row = 32 * sub + li;
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(ks + k_lds_off(row, 2 * kk + hl));
-      acc = mfma32x32x16(a, qf[kk], acc);
-    }
-    s[sub] = acc;
-  }
-}
-
-// O^T[4 d-subtiles] += V^T P^T for one tile; p[m] holds the bf16 probabilities of 16-key
-// step m (m = 0..3).
-__device__ __forceinline__ void pv_tile(floatx16 o[4], const bf16* vs, const bf16x8 p[4]) {
-  const int lane = threadIdx.x & 63;
-  const int li = lane & 31, hl = lane >> 5;
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-#pragma unroll
-    for (int ds = 0; ds < 4; ++ds) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(vs + v_lds_off(32 * ds + li, 2 * m + hl));
-      o[ds] = mfma32x32x16(a, p[m], o[ds]);
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -276,15 +189,6 @@ __device__ __forceinline__ void pv_tile_tr(floatx16 o[4], const unsigned char* t
     if (t + PF < 16) a[t + PF] = rt_tr_operand<RV>(tile, tro, t + PF);
     o[t & 3] = mfma32x32x16(a[t], p[t >> 2], o[t & 3]);
     __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
-// bf16 B operand of PV step m from the score registers (keys of sub-tile m/2, half m%2).
-__device__ __forceinline__ void pack_p(bf16x8 p[4], const floatx16 s[2]) {
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) p[m][e] = (bf16)s[m >> 1][8 * (m & 1) + e];
   }
 }
 

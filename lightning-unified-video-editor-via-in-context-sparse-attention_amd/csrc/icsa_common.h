@@ -84,11 +84,6 @@ __device__ __forceinline__ float wave_sum(float x) {
   for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o, 64);
   return x;
 }
-__device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) x = fmaxf(x, __shfl_xor(x, o, 64));
-  return x;
-}
 
 // Order-preserving map float -> uint32 (larger float -> larger key).  NaN-free inputs.
 __device__ __forceinline__ uint32_t f2key(float f) {
@@ -114,27 +109,14 @@ __host__ __device__ __forceinline__ int xcd_grid(int n_work) { return ((n_work +
 // MFMA wrappers (gfx950).  Operand/result layouts (checked on the device):
 //  32x32x16 bf16: A lane l holds A[l%32][8*(l/32)+i], B lane l holds B[8*(l/32)+i][l%32],
 //                 C lane l element i is C[(i/4)*8 + (l/32)*4 + i%4][l%32].
-//  32x32x2 f32:   A lane l holds A[l%32][l/32],       B lane l holds B[l/32][l%32],
-//                 C as above.
 __device__ __forceinline__ floatx16 mfma32x32x16(bf16x8 a, bf16x8 b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ floatx16 mfma32x32x2f32(float a, float b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
 // Row (within a 32-row MFMA tile) held by accumulator element i of lane l.
 __device__ __forceinline__ int acc_row(int i, int lane) {
   return (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
 }
-
-// Row 32 sub + acc_row(i, lane) of a 64-row tile held as two 32x32 accumulators is at or
-// past `limit` iff the lane-independent part 32 sub + 8 (i / 4) + i % 4 reaches the
-// threshold mask_threshold(limit, lane).  Testing against that threshold compares each
-// element with a compile-time constant: no per-element row values are kept in registers
-// (which the compiler would otherwise rematerialise on every tile, mask or not).
-__device__ __forceinline__ int mask_threshold(int limit, int lane) { return limit - (lane >> 5) * 4; }
-__device__ __forceinline__ constexpr int acc_row_const(int sub, int i) { return 32 * sub + 8 * (i >> 2) + (i & 3); }
 
 // ---------------------------------------------------------------------------------------
 // kernel parameter blocks (passed by value)

@@ -112,11 +112,11 @@ __device__ __forceinline__ void bw_transpose_bits(const SparseBwdParams& p, int 
 }
 
 // ------------------------------------------------------------------------------------------
-// Tile DMA.  A 16 KB row tile (64 rows x 128 dims, swizzled by rt_swz) is 16
-// LDS-DMA instructions, 8 per wave; each lands 1 KB at consecutive LDS addresses (lane l
-// at +16 l), so the XOR swizzle is applied on the global side.  A step's tiles are the only
+// Tile DMA.  A 16 KB row tile (64 rows x 128 dims, swizzled by rt_swz) is 16 LDS-DMA
+// instructions, 4 for each of the four waves; each lands 1 KB at consecutive LDS addresses (lane
+// l at +16 l), so the XOR swizzle is applied on the global side.  A step's tiles are the only
 // loads in flight when a kernel waits for them (vmcnt(0)): the next step's tiles are issued
-// after the workgroup barrier that follows, which also tells that both waves are done with
+// after the workgroup barrier that follows, which also tells that all four waves are done with
 // the buffer they overwrite (two buffers, one barrier per step).
 // ------------------------------------------------------------------------------------------
 #define BW_WAIT(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
