@@ -31,15 +31,19 @@ def _inputs(B, H, Sq, Sk, seed, dev):
 
 
 @pytest.mark.parametrize("B,H,Sq,Sk", [
-    (1, 1, 64, 1024),       # one item, 16 tiles in 4 chunks
+    (1, 1, 64, 1024),       # one item, 16 tiles: run whole
     (1, 1, 65, 833),        # 14 tiles, a partial last one; a second block of one row
-    (2, 1, 300, 2000),      # 4 items, 2 of them of one block
-    (1, 3, 1000, 1500),     # chunks that end one item and start the next
-    (1, 40, 1800, 1000),    # one full round of items and 64 split ones
-    (1, 1, 64, 832),        # 13 tiles: the shortest that are split
-    (1, 1, 64, 768),        # 12 tiles: run whole
-    (1, 257, 64, 77),       # one item past a round, 2 tiles each: bundles of 2
-    (1, 130, 700, 64),      # one-tile items in bundles of 2, queries ending inside a block
+    (2, 1, 300, 2000),      # split: 4 items, 2 of them of one block, 8 chunks each
+    (1, 3, 1000, 1500),     # split: 12 items, 6 chunks each
+    (1, 40, 1800, 1000),    # one full round of items and 64 more, 16 tiles: run whole
+    (1, 1, 64, 832),        # 13 tiles
+    (1, 1, 64, 768),        # 12 tiles: no size of call is split
+    (1, 257, 64, 77),       # one item past a round, 2 tiles each: two items a workgroup
+    (1, 130, 700, 64),      # one-tile items, two a workgroup, queries ending inside a block
+    (1, 1, 64, 1088),       # 17 tiles: run whole
+    (1, 1, 64, 1152),       # 18 tiles: the shortest item that is split, 4 chunks
+    (1, 2, 500, 2900),      # 4 items of 46 tiles in 46 chunks: one in four ends an item and starts the next
+    (1, 40, 1800, 1200),    # one full round of items and 64 split ones, 256 chunks of 4 or 5 tiles
 ])
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
 def test_flash_work_split(gpu, B, H, Sq, Sk, out):
