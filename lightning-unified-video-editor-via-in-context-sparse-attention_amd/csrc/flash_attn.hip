@@ -16,13 +16,13 @@
 // are cut into, whose partial O, max and sum icsa_flash_combine_kernel adds up.  The tile
 // stream runs across segment boundaries, so the next item's tiles arrive while an item
 // ends.  Measured against one workgroup per item, with an epilogue of its own: 32 items of
-// 72 tiles (2 heads, 8,192 tokens) 101 -> 27 us plus 9 us for the sums; 640 items of 576
-// tiles (5 heads, 65,536 tokens; 2.5 rounds) 2,825 -> 2,511 + 10 us; 10,240 items of 8
-// tiles (512 keys, 40 heads, 65,520 queries) 853 -> 775 us; 5,120 items of 576 tiles (40
-// heads) unchanged at 20.0 ms.  The rate is then about 1.23 PFLOP/s at every size that
+// 72 tiles (2 heads, 8,192 tokens) 101 -> 30 us plus 9 us for the sums; 640 items of 576
+// tiles (5 heads, 65,536 tokens; 2.5 rounds) 2,825 -> 2,536 + 11 us; 10,240 items of 8
+// tiles (512 keys, 40 heads, 65,520 queries) 853 -> 768-790 us; 5,120 items of 576 tiles (40
+// heads) unchanged at 19.9 ms.  The rate is then about 1.2 PFLOP/s at every size that
 // fills the chip, the engine clock under this load being 1.7-1.9 GHz; with 8 tiles an item,
-// timing copies without the output stores and without the Q loads take 693 and 755 us (both:
-// 641 us).
+// timing copies without the output stores and without the Q loads took 693 and 755 us (both:
+// 641 us) when the kernel took 775.
 //
 // Workgroup = 8 waves = an item's query blocks (wave w: block w/2, rows 32*(w%2)..+31),
 // all sharing each K / V^T tile.  The waves form two groups, G0 = waves 0-3 and G1 = waves

@@ -39,7 +39,7 @@ constexpr FlashRun flash_whole_run(int wg, int n_whole, int n_bundle) {
 //  * Whole items go several to a workgroup, up to FA_BUNDLE_TILES tiles: beyond that a
 //    workgroup's start no longer counts and many workgroups even out the CUs (220 tiles an
 //    item, 8.6 rounds: 4,710 us with bundles of 1 or 2 items, 4,870 us with 8; 8 tiles an item,
-//    40 rounds: 783, 775 and 773 us with 14, 20 and 40 items).  Of these counts the one whose
+//    40 rounds: 1 % between 14, 20 and 40 items).  Of these counts the one whose
 //    rounds are shortest, a start costing FA_START_TILES tiles: bundles that do not fill the
 //    last round cost more than the starts they save (768 items of 256 tiles: in pairs 1,541 us,
 //    one by one 1,350; 1,792 of 147: in threes 2,093, one by one 1,804).
